@@ -3,10 +3,29 @@
 #include <atomic>
 #include <algorithm>
 
-#include "vh_gemm.hpp"
+#include "vh_gemm_epi.hpp"
 #include "vh_launch.hpp"
 
 namespace vh {
+
+// Merge of the kAttnMaxSplits attention partials of m rows into ao [m][heads * hd] (the PRO_ATTN prologue of the
+// GEMV, as its own pass before a GEMM). grid (heads, m), block hd.
+__global__ __launch_bounds__(128) void k_attn_merge(AttnPartials P, float *ao) {
+    const int h = blockIdx.x, i = blockIdx.y, e = threadIdx.x;
+    const int64_t base = (int64_t(i) * P.heads + h) * kAttnMaxSplits;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int q = 0; q < kAttnMaxSplits; ++q) mx = fmaxf(mx, P.pm[base + q]);
+    float L = 0.f, O = 0.f;
+#pragma unroll
+    for (int q = 0; q < kAttnMaxSplits; ++q) {
+        const float pmq = P.pm[base + q];
+        const float wq = pmq == -INFINITY ? 0.f : expf(pmq - mx);
+        L = fmaf(wq, P.pl[base + q], L);
+        O = fmaf(wq, P.po[(base + q) * P.hd + e], O);
+    }
+    ao[int64_t(i) * P.heads * P.hd + h * P.hd + e] = O * (1.0f / L);
+}
 
 template <int WT, int EPI, int ASRC, int T>
 static hipError_t gemm_run(const uint8_t *w, const float *scale, const float *A, const GemmArgs &g, int groups, hipStream_t s) {
@@ -74,9 +93,8 @@ static int split_plan(const GemmArgs &g, int *kchunk) {
 }
 template <int EPI>
 static hipError_t splitk_reduce(const GemmArgs &g, int splits, hipStream_t s) {
-    const int nout = EPI == EPI_SWIGLU ? g.n / 2 : g.n;
-    const int64_t total = int64_t(g.m) * nout;
-    return launch(k_gemm_splitk_reduce<EPI>, dim3(unsigned((total + 255) / 256)), dim3(256), 0, s, g, int32_t(splits));
+    const int64_t threads = int64_t(g.m) * ((g.n + 3) / 4);
+    return launch(k_gemm_splitk_reduce<EPI>, dim3(unsigned((threads + 255) / 256)), dim3(256), 0, s, g, int32_t(splits));
 }
 template <int WT, int EPI>
 static hipError_t gemm_splitk(const uint8_t *w, const float *scale, const float *A, const GemmArgs &g, hipStream_t s, bool *done) {
@@ -127,6 +145,15 @@ static bool rope_h16_ok(const GemmArgs &g) {
            g.n == g.rope_cols + g.rope_cols / 2 && g.ldvt >= g.seq && g.ldvt % 8 == 0 && g.lo_off % 8 == 0;
 }
 
+// The operands an epilogue needs beyond y.
+static bool gemm_args_ok(int epi, const GemmArgs &g) {
+    switch (epi) {
+        case EPI_GATED_ACC: return g.gate != nullptr;
+        case EPI_ACC_SNAKE: return g.snake_a && g.snake_ib && g.snake_y;
+        case EPI_ROPE_H16: return rope_h16_ok(g);
+        default: return true;
+    }
+}
 template <int WT>
 static hipError_t gemm_epi(int epi, const uint8_t *w, const float *scale, const float *A, const GemmArgs &g, hipStream_t s) {
     switch (epi) {
@@ -153,6 +180,11 @@ hipError_t launch_gemm(int wt, int epi, const uint8_t *w, const float *scale, co
     if (g.m <= 0) return hipSuccess;
     if (g.K % 8 || g.n <= 0 || g.lda % 4) return hipErrorInvalidValue;
     if ((epi == EPI_SWIGLU || epi == EPI_ROPE) && g.n % 2) return hipErrorInvalidValue;
+    if (wt == WT_F32 && g.wx && gemm_args_ok(epi, g)) {
+        bool done = false;
+        const hipError_t e = launch_gemm_x3p(ASRC_ROWS, epi, A, g, 1, s, &done);
+        if (e != hipSuccess || done) return e;
+    }
     switch (wt) {
         case WT_F32: return gemm_epi<WT_F32>(epi, w, scale, A, g, s);
         case WT_F16: return gemm_epi<WT_F16>(epi, w, scale, A, g, s);
@@ -275,6 +307,11 @@ hipError_t launch_conv_gemm(int epi, const float *w, const float *A, const GemmA
         g.K % 8 || g.seq <= 0 || g.lda % 4 || groups <= 0 || g.n <= 0)
         return hipErrorInvalidValue;
     const uint8_t *wb = reinterpret_cast<const uint8_t *>(w);
+    if (g.wx) {
+        bool done = false;
+        const hipError_t e = launch_gemm_x3p(ASRC_CONV, epi, A, g, groups, s, &done);
+        if (e != hipSuccess || done) return e;
+    }
     if (groups == 1 && (epi == EPI_STORE || epi == EPI_ACC)) {  // one group: K slices in place of groups when idle
         GemmArgs gs = g;
         const int splits = split_plan(g, &gs.kchunk);
@@ -322,10 +359,15 @@ hipError_t launch_stream_conv(int wt, int epi, const uint8_t *w, const float *sc
     if (g.m <= 0) return hipSuccess;
     if (g.cig <= 0 || g.cig % 4 || g.ksize <= 0 || g.dil <= 0 || g.K != g.ksize * g.cig || g.K % 8 || g.lda % 4 || g.n <= 0 ||
         g.ctx != (g.ksize - 1) * g.dil || (g.ctx && !g.hist) || !g.y ||
-        (g.hist_next && (!g.ctx || g.hist_next == g.hist)))
+        (g.hist_next && (!g.ctx || g.hist_next == g.hist)) || (epi == EPI_SNAKE && (!g.snake_a || !g.snake_ib)))
         return hipErrorInvalidValue;
+    if (wt == WT_F32 && g.wx) {
+        bool done = false;
+        const hipError_t e = launch_gemm_x3p(ASRC_STREAM, epi, x, g, 1, s, &done);
+        if (e != hipSuccess || done) return e;
+    }
     if (epi == EPI_STORE) return stream_conv_wt<EPI_STORE>(wt, w, scale, x, g, s);
-    if (epi == EPI_SNAKE) return g.snake_a && g.snake_ib ? stream_conv_wt<EPI_SNAKE>(wt, w, scale, x, g, s) : hipErrorInvalidValue;
+    if (epi == EPI_SNAKE) return stream_conv_wt<EPI_SNAKE>(wt, w, scale, x, g, s);
     return hipErrorInvalidValue;
 }
 

@@ -830,45 +830,6 @@ __global__ __launch_bounds__(128 * WN) __attribute__((amdgpu_waves_per_eu(Q8 ? 4
     gemm_epilogue<EPI, TM, TN>(acc, g, m0, n0, wm, wn, lane);
 }
 
-// The split-K partial slices ws[z][m][n], added in z order, then bias and the epilogue (STORE, ACC, GATED_ACC, SWIGLU,
-// SNAKE, GELU_ERF, ACC_SNAKE: one thread per output element; SWIGLU outputs pair columns 2u, 2u + 1). grid
-// ceil(m n' / 256).
-template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm_splitk_reduce(GemmArgs g, int32_t splits) {
-    const int nout = EPI == EPI_SWIGLU ? g.n / 2 : g.n;
-    const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (t >= int64_t(g.m) * nout) return;
-    const int row = int(t / nout), c = int(t % nout);
-    const int64_t slice = int64_t(g.m) * g.n;
-    auto sum = [&](int col) {  // 8 slices' loads in flight at once (past `splits`, slice 0, left out), added in order
-        float v = 0.f;
-        for (int z0 = 0; z0 < splits; z0 += 8) {
-            float t[8];
-#pragma unroll
-            for (int z = 0; z < 8; ++z) t[z] = g.ws[(z0 + z < splits ? z0 + z : 0) * slice + int64_t(row) * g.n + col];
-#pragma unroll
-            for (int z = 0; z < 8; ++z)
-                if (z0 + z < splits) v += t[z];
-        }
-        return v + (g.bias ? g.bias[col] : 0.f);
-    };
-    float *dst = g.y + int64_t(row) * g.ldy + c;
-    if (EPI == EPI_SWIGLU) *dst = silu(sum(2 * c)) * sum(2 * c + 1);
-    else if (EPI == EPI_STORE) *dst = sum(c);
-    else if (EPI == EPI_ACC) *dst += sum(c);
-    else if (EPI == EPI_GATED_ACC) *dst += g.gate[c] * sum(c);
-    else if (EPI == EPI_SNAKE) {
-        const float v = sum(c), sn = sinf(v * g.snake_a[c]);
-        *dst = v + g.snake_ib[c] * sn * sn;
-    }
-    else if (EPI == EPI_GELU_ERF) *dst = gelu_erf_f(sum(c));
-    else if (EPI == EPI_ACC_SNAKE) {
-        const float v = *dst + sum(c), sn = sinf(v * g.snake_a[c]);
-        *dst = v;
-        g.snake_y[int64_t(row) * g.ldy + c] = v + g.snake_ib[c] * sn * sn;
-    }
-}
-
 // The split-K slices of an EPI_ACC product added into its rows, y[row][c] += (sum_z ws[z][row][c]) + bias[c], as
 // k_gemm_splitk_reduce<EPI_ACC> does, then the RMSNorm (gamma, eps) of each updated row written as f16 halves (hi at
 // out16, lo at out16 + lo_off, rows of ldo halves) with k_rmsnorm_rows_h16's arithmetic: the residual add and the
@@ -922,25 +883,6 @@ __global__ __launch_bounds__(256) void k_splitk_acc_rms_h16(GemmArgs g, int32_t 
         }
     }
     raise_status(g.status, bad, kStatusF16Range);
-}
-
-// Merge of the kAttnMaxSplits attention partials of m rows into ao [m][heads * hd] (the PRO_ATTN prologue of the
-// GEMV, as its own pass before a GEMM). grid (heads, m), block hd.
-__global__ __launch_bounds__(128) void k_attn_merge(AttnPartials P, float *ao) {
-    const int h = blockIdx.x, i = blockIdx.y, e = threadIdx.x;
-    const int64_t base = (int64_t(i) * P.heads + h) * kAttnMaxSplits;
-    float mx = -INFINITY;
-#pragma unroll
-    for (int q = 0; q < kAttnMaxSplits; ++q) mx = fmaxf(mx, P.pm[base + q]);
-    float L = 0.f, O = 0.f;
-#pragma unroll
-    for (int q = 0; q < kAttnMaxSplits; ++q) {
-        const float pmq = P.pm[base + q];
-        const float wq = pmq == -INFINITY ? 0.f : expf(pmq - mx);
-        L = fmaf(wq, P.pl[base + q], L);
-        O = fmaf(wq, P.po[(base + q) * P.hd + e], O);
-    }
-    ao[int64_t(i) * P.heads * P.hd + h * P.hd + e] = O * (1.0f / L);
 }
 
 }  // namespace vh

@@ -70,6 +70,12 @@ void set_gemm_hh_tile(int tile);
 // it did (otherwise the caller runs the norm).
 hipError_t launch_gemm_hh_acc_rms(const _Float16 *w, const float *q8_scale, const GemmArgs &g, const float *gamma, float eps,
                                   _Float16 *out16, int64_t ldo, int64_t lo_off, hipStream_t s, bool *normed);
+// F32 weights [n][K] as k_gemm_x3p reads them, pack_x3_bytes(n, K) bytes at out (weights of |w| < 64).
+int64_t pack_x3_bytes(int64_t n, int64_t K);
+hipError_t launch_pack_x3(const float *w, int64_t n, int64_t K, void *out, hipStream_t s);
+// The product of launch_gemm / launch_conv_gemm / launch_stream_conv (A source asrc) on packed F32 weights g.wx; *done
+// tells whether it ran (else the caller's own kernel takes it).
+hipError_t launch_gemm_x3p(int asrc, int epi, const float *A, const GemmArgs &g, int groups, hipStream_t s, bool *done);
 hipError_t launch_conv_gemm(int epi, const float *w, const float *A, const GemmArgs &g, int groups, hipStream_t s);
 // Merge of the split attention partials of m rows into ao [m][heads * hd].
 hipError_t launch_attn_merge(const AttnPartials &P, float *ao, int m, hipStream_t s);

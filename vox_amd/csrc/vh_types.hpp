@@ -225,6 +225,10 @@ struct GemmArgs {
     // F32 weights with max |w| >= 63 (or NaN): the split kernel's 2^10-scaled f16 halves cannot hold them, so they
     // take k_gemm_f32
     int32_t f32_wide;
+    // F32 weights laid out by launch_pack_x3 (per group of a grouped convolution, one after the other), or null: with
+    // them the product takes k_gemm_x3p. cig_magic: ceil(2^32 / cig), set by its launcher
+    const void *wx;
+    uint32_t cig_magic;
 };
 
 // CosyVoice2 LM sampling (lm_logp + ras_sample + lm_generate's trial loop, cosyvoice.cpp:598-690).

@@ -72,6 +72,7 @@ struct GpuMat {
     uint64_t bytes = 0;  // weights + scales + bias bytes (the GEMV's algorithmic stream)
     _Float16 *w16 = nullptr;  // Q8: the int8 values widened to f16 for the split-f16 GEMM, made on first use
     float wmax = 0.f;  // F32: max |w| (NaN when a weight is NaN), which picks the GEMM kernel (f32_wide)
+    void *wx = nullptr;  // F32: the weights laid out for k_gemm_x3p, made by the first user that multiplies rows with them
 };
 
 struct LayerDev {
@@ -375,6 +376,30 @@ float host_absmax(const float *w, size_t n) {
     return mx;
 }
 
+// The layout of F32 weights that k_gemm_x3p reads (rows of K weights per group, one group after the other), or null when
+// it cannot be allocated: the products then keep k_gemm_x3. Not during a capture.
+void *pack_x3(const float *w, int64_t rows, int64_t K, int groups, hipStream_t s) {
+    const int64_t one = vh::pack_x3_bytes(rows, K);
+    uint8_t *p = nullptr;
+    try {
+        p = static_cast<uint8_t *>(dalloc(size_t(one * groups)));
+    } catch (const Fail &) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    for (int i = 0; i < groups; ++i) {
+        const hipError_t e = vh::launch_pack_x3(w + int64_t(i) * rows * K, rows, K, p + one * i, s);
+        if (e != hipSuccess) {
+            dfree(p);
+            HIPCHECK(e);
+        }
+    }
+    return p;
+}
+void prepare_x3(GpuMat &m, hipStream_t s) {
+    if (m.type == VOXHIP_F32 && !m.wx && !f32_wide(m)) m.wx = pack_x3(reinterpret_cast<const float *>(m.w), m.rows, m.cols, 1, s);
+}
+
 // f32 -> f16 bits when the value is exactly representable as a normal or zero f16 (the scales a device Q4 matrix
 // may store in 2 bytes without changing its arithmetic).
 bool f16_exact(float f, uint16_t *out) {
@@ -408,7 +433,7 @@ int new_mat(int32_t type, int64_t rows, int64_t cols, bool bias, bool s16 = fals
 void free_mat(int id) {
     if (id < 0 || size_t(id) >= g.mats.size()) return;
     GpuMat &m = g.mats[size_t(id)];
-    dfree(m.w); dfree(m.s); dfree(m.b); dfree(m.w16);
+    dfree(m.w); dfree(m.s); dfree(m.b); dfree(m.w16); dfree(m.wx);
     m = GpuMat();
 }
 
@@ -594,6 +619,7 @@ void gemv(const GpuMat &m, int64_t m_total, int pro, int epi, const float *x, in
         ga.ws = sc.ws; ga.ws_cap = sc.ws_cap;
         ga.gate = yscale;  // a row scale of the GEMV is the GEMM's gated residual (y += gate[col] (c + bias))
         ga.f32_wide = f32_wide(m);
+        ga.wx = m.wx;
         HIPCHECK(launch_gemm(gemv_type(m), yscale ? EPI_GATED_ACC : epi, m.w, m.s, A, ga, s));
         return;
     }
@@ -1042,6 +1068,9 @@ int forward_rows(Xfmr &X, int64_t m, RowsOf rows_of, const float *x, int in_proj
         for (int i = 0; i < mc && fused; ++i)
             for (int j = 0; j < i; ++j)
                 if (rr[size_t(i)].k == rr[size_t(j)].k) { fused = false; break; }
+        for (int li = first_layer; li < first_layer + n_layers; ++li)
+            for (int id : {X.L[size_t(li)].qkv, X.L[size_t(li)].o, X.L[size_t(li)].gu, X.L[size_t(li)].down})
+                if (gemm_path(g.mats[size_t(id)], m_total, mc)) prepare_x3(g.mats[size_t(id)], g.stream);
         if (pass_attn_of(X, mc, fused)) prepare_planes(X, first_layer, n_layers, m_total, mc, g.stream);
         run_layers(X, mc, m_total, first_layer, n_layers, fused);
         if (hidden_out) {
@@ -1410,9 +1439,10 @@ int voxhip_matmul(int mat, const float *x, int64_t m, float *y) {
     return guard_int([&] {
         require_ok();
         vh::prof_stage("matmul");
-        const GpuMat &M = mat_at(mat);
+        GpuMat &M = mat_at(mat);
         if (m <= 0) return 1;
         const int chunk = rows_per_pass(M, m);
+        if (gemm_path(M, m, int(std::min<int64_t>(chunk, m)))) prepare_x3(M, g.stream);
         const size_t xb = size_t(chunk) * size_t(M.cols) * 4, yb = size_t(chunk) * size_t(M.rows) * 4;
         float *pin = pinned(std::max(xb, yb) + 64);
         float *dx = dev_scratch(g.dbuf_x, g.dbuf_x_bytes, xb), *dy = dev_scratch(g.dbuf_y, g.dbuf_y_bytes, yb);
@@ -1488,7 +1518,7 @@ int voxhip_convt(int mat, int32_t K, int32_t stride, int32_t pad, int32_t out_pa
     return guard_int([&] {
         require_ok();
         vh::prof_stage("convt");
-        const GpuMat &M = mat_at(mat);
+        GpuMat &M = mat_at(mat);
         if (K < 1 || stride < 1 || pad < 0 || out_pad < 0 || T < 1 || !x || !y)
             throw Fail("convt: K, stride and T must be positive, pad and out_pad not negative, x and y given");
         if (M.rows % K) throw Fail("convt: the matrix rows are not K cout");
@@ -1509,6 +1539,7 @@ int voxhip_convt(int mat, int32_t K, int32_t stride, int32_t pad, int32_t out_pa
         HIPCHECK(copy_h2d(dx, pin, xb + bb, g.stream));
         // z = x W^T, frames in passes of the matrix's pass height, then the padded overlap-add + bias
         const int chunk = rows_per_pass(M, T);
+        if (gemm_path(M, T, int(std::min<int64_t>(chunk, T)))) prepare_x3(M, g.stream);
         for (int64_t c0 = 0; c0 < T; c0 += chunk) {
             const int mc = int(std::min<int64_t>(chunk, T - c0));
             gemv(M, T, PRO_X, EPI_STORE, dx + c0 * cin, cin, mc, dz + c0 * KO, KO, nullptr, 0.f, nullptr, g.stream);
@@ -2210,6 +2241,7 @@ struct F5Block {
 struct F5Conv {
     float *w = nullptr, *b = nullptr;  // w [groups][cout/groups][kpad] (K * cin/groups, zero-padded to a multiple of 8)
     int cin = 0, cout = 0, K = 0, groups = 0, kpad = 0;
+    void *wx = nullptr;  // w laid out for k_gemm_x3p (not the wide ones)
     bool wide = false;  // max |w| >= 63 or NaN: the conv GEMM on f32 matrix cores (GemmArgs::f32_wide)
 };
 struct F5VBlock {  // a Vocos ConvNeXt block (f5.cpp:235-240)
@@ -2385,6 +2417,7 @@ F5Conv upload_conv_gemm(const voxhip_f5_conv &c, const char *what) {
     d.wide = f32_wide(host_absmax(w.data(), w.size()));
     d.w = dalloc_t<float>(w.size());
     h2d(d.w, w.data(), w.size() * 4);
+    if (!d.wide) d.wx = pack_x3(d.w, cog, d.kpad, c.groups, g.stream);
     if (c.b) {
         d.b = dalloc_t<float>(size_t(c.cout));
         h2d(d.b, c.b, size_t(c.cout) * 4);
@@ -2430,6 +2463,7 @@ GemmArgs gemm_args(const GpuMat &m, const float *bias, float *y, int64_t lda, in
     ga.bias = bias; ga.y = y; ga.lda = lda; ga.ldy = ldy; ga.m = int32_t(rows); ga.n = int32_t(m.rows); ga.K = int32_t(m.cols);
     ga.ws = g.gemm_ws; ga.ws_cap = kGemmWsFloats;
     ga.f32_wide = f32_wide(m);
+    ga.wx = m.wx;
     return ga;
 }
 void f5_gemm(const GpuMat &m, int epi, const float *A, GemmArgs ga, hipStream_t s) {
@@ -2474,6 +2508,7 @@ void f5_enqueue(F5 &F, hipStream_t s) {
         ga.bias = cv.b; ga.y = c == 0 ? F.a : F.h; ga.lda = D; ga.ldy = D; ga.m = int32_t(R);
         ga.n = cv.cout / cv.groups; ga.cig = cv.cin / cv.groups; ga.ksize = cv.K; ga.K = cv.kpad; ga.seq = F.N;
         ga.f32_wide = cv.wide;
+        ga.wx = cv.wx;
         HIPCHECK(launch_conv_gemm(c == 0 ? EPI_MISH : EPI_MISH_ACC, cv.w, c == 0 ? F.h : F.a, ga, cv.groups, s));
     }
     const float scale = 1.0f / std::sqrt(float(F.hd));
@@ -2579,6 +2614,11 @@ int voxhip_f5_create(const voxhip_f5_desc *d) {
             }
             F->vdim = VD; F->vinter = VI; F->vout = VO; F->v_head = d->v_head;
         }
+        std::vector<int> ids{F->in_proj, F->proj_out};  // the linears that multiply rows, where they are F32
+        for (const F5Block &fb : F->blocks) ids.insert(ids.end(), {fb.qkv, fb.o, fb.ff1, fb.ff2});
+        for (const F5VBlock &vb : F->vblocks) ids.insert(ids.end(), {vb.pw1, vb.pw2});
+        if (F->vdim) ids.push_back(F->v_head);
+        for (int id : ids) prepare_x3(mat_at(id), g.stream);
         g.f5.push_back(F.release());
         return int(g.f5.size()) - 1;
     }, -1);
@@ -2657,6 +2697,7 @@ int voxhip_f5_vocos(int id, const float *mel, int T, float *head) {
         ge.bias = ce.b; ge.y = F.vx; ge.lda = ce.cin; ge.ldy = VD; ge.m = T; ge.n = ce.cout / ce.groups;
         ge.cig = ce.cin / ce.groups; ge.ksize = ce.K; ge.K = ce.kpad; ge.seq = T;
         ge.f32_wide = ce.wide;
+        ge.wx = ce.wx;
         HIPCHECK(launch_conv_gemm(EPI_STORE, ce.w, F.vm, ge, ce.groups, s));
         HIPCHECK(launch_layernorm_rows(F.vx, T, VD, F.v_ln_w, F.v_ln_b, F.vx, s));
         for (const F5VBlock &b : F.vblocks) {
@@ -2782,6 +2823,7 @@ CosyX cosy_x_up(const voxhip_cosy_x &x, int C, int heads, int hd) {
     o.qkv = stack_rows_heads({x.q, x.k, x.v}, heads, hd, kF5HeadDim);
     o.o = pad_head_cols(x.o, heads, hd, kF5HeadDim);
     o.ff1 = x.ff1; o.ff2 = x.ff2; o.ff = x.ff_dim;
+    for (int id : {o.qkv, o.o, o.ff1, o.ff2}) prepare_x3(mat_at(id), g.stream);  // where they are F32
     return o;
 }
 
@@ -2792,6 +2834,7 @@ void cosy_conv(const Cosy &E, const F5Conv &cv, int epi, const float *X, int64_t
     ga.cig = cv.cin; ga.ksize = cv.K; ga.K = cv.kpad; ga.seq = E.T; ga.causal = 1;
     ga.ws = g.gemm_ws; ga.ws_cap = kGemmWsFloats;  // split K when the 64 x 64 tiles leave the CUs idle
     ga.f32_wide = cv.wide;
+    ga.wx = cv.wx;
     HIPCHECK(launch_conv_gemm(epi, cv.w, X, ga, 1, s));
 }
 
@@ -3124,6 +3167,7 @@ void codec_conv(const CodecConv &c, Hist2 *h, int par, const float *X, int64_t l
     if (ga.ctx && !h) throw Fail("codec convolution without its history");
     if (ga.ctx) ga.hist_next = h->b[1 - par];
     ga.f32_wide = f32_wide(M);
+    ga.wx = M.wx;
     HIPCHECK(launch_stream_conv(gemv_type(M), snake ? EPI_SNAKE : EPI_STORE, M.w, M.s, X, ga, s));
 }
 // y (=, +=, gelu, gamma-gated +=) W x + bias over rows of the f32-activation GEMM (the f32 tile semantics of matmul
@@ -3351,6 +3395,15 @@ int voxhip_codec_create(const voxhip_codec_desc *d) {
         E->pre = dalloc_t<float>(F * size_t(std::max(E->H, E->I)));
         E->rope = dalloc_t<float>(F * size_t(E->hd));
         E->z = dalloc_t<float>(F * size_t(E->cdim));
+        // every product of a call takes the packed weights (its launches are captured: nothing is laid out later)
+        std::vector<int> ids{E->pre_conv.mat, E->pt_in, E->pt_out, E->conv0.mat, E->fin.mat};
+        for (const LayerDev &d : xf_at(E->xf).L) ids.insert(ids.end(), {d.qkv, d.o, d.gu, d.down});
+        for (const CodecUp &u : E->ups) ids.insert(ids.end(), {u.tr, u.pw1, u.pw2});
+        for (const CodecBlk &b : E->blocks) {
+            ids.push_back(b.tr);
+            for (int u = 0; u < 3; ++u) ids.insert(ids.end(), {b.c1[u].mat, b.c2[u].mat});
+        }
+        for (int id : ids) prepare_x3(mat_at(id), g.stream);
         g.codecs.push_back(E.release());
         return int(g.codecs.size()) - 1;
     }, -1);
