@@ -35,6 +35,13 @@ __device__ __forceinline__ bool split_f16(float x, _Float16 &hi, _Float16 &lo) {
     lo = _Float16(x - float(hi));
     return __builtin_isinf(float(hi)) && !__builtin_isinf(x);
 }
+// Where element (row, k) of an activation matrix of K columns (a multiple of 32) kept as f16 halves lies: 16-row by
+// 32-column tiles in MFMA fragment order, [row / 16][k / 32][hi, lo][(k % 32) / 8 x 16 + row % 16][8]; the lo half kPlaneLo
+// halves after the hi one. A fragment is 1 KiB of consecutive bytes. The buffer of m rows has planes_halves(m, K) halves.
+constexpr int kPlaneLo = 512;
+VH_DEV int64_t plane_off(int64_t row, int k, int K) {
+    return ((row >> 4) * (K >> 5) + (k >> 5)) * 1024 + ((((k >> 3) & 3) << 4) + (row & 15)) * 8 + (k & 7);
+}
 // Sets `bit` in the status word when `bad` (a vector atomic; the common path is one predicated branch).
 __device__ __forceinline__ void raise_status(int32_t *status, bool bad, int32_t bit) {
     if (__builtin_expect(bad, 0) && status) __hip_atomic_fetch_or(status, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -8,17 +8,17 @@ hipError_t launch_norm_rows(const NormArgs &a0, hipStream_t s) {
     NormArgs a = a0;
     a.status = status_word();
     if (a.R <= 0) return hipSuccess;
-    if (a.D <= 0 || a.D % 4 || !a.x || (!a.y && !a.y16) || a.lo_off % 4 || !a.sc || (!a.affine && !a.sh) || !(a.eps > 0.0))
+    if (a.D <= 0 || a.D % 4 || !a.x || (!a.y && !a.y16) || (a.y16 && a.D % 32) || !a.sc || (!a.affine && !a.sh) || !(a.eps > 0.0))
         return hipErrorInvalidValue;
     if (a.D <= 4 * 256) return launch(k_f5_modulate<4, true>, dim3(unsigned((a.R + 3) / 4)), dim3(256), 0, s, a);
     return launch(k_f5_modulate<kNormRegChunks, false>, dim3(unsigned((a.R + 3) / 4)), dim3(256), 0, s, a);
 }
 
 hipError_t launch_f5_modulate(const float *x, int64_t R, int D, const float *sc, const float *sh, float *y, _Float16 *y16,
-                              int64_t lo_off, hipStream_t s) {
+                              hipStream_t s) {
     if (R > INT32_MAX) return hipErrorInvalidValue;
     NormArgs a{};
-    a.x = x; a.y = y; a.y16 = y16; a.lo_off = lo_off; a.sc = sc; a.sh = sh;
+    a.x = x; a.y = y; a.y16 = y16; a.sc = sc; a.sh = sh;
     a.eps = 1e-6;  // the modulation adds the double 1e-6 (f5.cpp:608-625)
     a.R = int32_t(R); a.D = D;
     return launch_norm_rows(a, s);
@@ -47,12 +47,12 @@ hipError_t launch_f5_fill_x(const float *x, int N, int mel, float *cat, int W, i
                   int32_t(B));
 }
 
-hipError_t launch_f5_attn(const _Float16 *qkv16, int64_t lo_off, float *out, _Float16 *out16, int64_t out_lo, int B, int N,
+hipError_t launch_f5_attn(const _Float16 *qkv16, int64_t lo_off, float *out, _Float16 *out16, int B, int N,
                           int heads, int hd, int ldvt, int ldo, float scale, hipStream_t s) {
     if (B <= 0 || N <= 0) return hipSuccess;
-    if (hd != kF5Hd || heads <= 0 || ldvt < N || ldvt % 64 || lo_off % 8 || ldo % 4 || (!out && !out16)) return hipErrorInvalidValue;
+    if (hd != kF5Hd || heads <= 0 || ldvt < N || ldvt % 64 || lo_off % 8 || ldo % 4 || (out16 && ldo % 32) || (!out && !out16)) return hipErrorInvalidValue;
     if ((int64_t(N) + 64) * 2 * heads * hd * 2 > INT32_MAX) return hipErrorInvalidValue;  // the q / k buffer offsets
-    F5AttnArgs a{qkv16, lo_off, out, int32_t(N), int32_t(ldo), int32_t(heads * hd), int32_t(ldvt), scale, out16, out_lo};
+    F5AttnArgs a{qkv16, lo_off, out, int32_t(N), int32_t(ldo), int32_t(heads * hd), int32_t(ldvt), scale, out16};
     // 4 query waves (64 rows) per block; when that leaves fewer blocks than CUs, 2 query waves (32 rows) times 2 key
     // halves
     if (int64_t((N + 63) / 64) * heads * B >= 256)

@@ -112,9 +112,9 @@ __global__ __launch_bounds__(256) void k_f5_modulate(NormArgs a) {
                 lo[e] = l;
             }
             raise_status(a.status, bad, kStatusF16Range);
-            _Float16 *hr = a.y16 + int64_t(row) * D + i;
+            _Float16 *hr = a.y16 + plane_off(row, i, D);
             *reinterpret_cast<f16x4a *>(hr) = hi;
-            *reinterpret_cast<f16x4a *>(hr + a.lo_off) = lo;
+            *reinterpret_cast<f16x4a *>(hr + kPlaneLo) = lo;
         } else {
             *reinterpret_cast<f32x4a *>(a.y + int64_t(row) * D + i) = r;
         }
@@ -181,8 +181,7 @@ struct F5AttnArgs {
     float *out;           // [B N][ldo], head h at column h * 64
     int32_t N, ldo, inner, ldvt;
     float scale;
-    _Float16 *out16;      // when set: the output as f16 halves, hi at out16, lo at out16 + out_lo (rows of ldo)
-    int64_t out_lo;
+    _Float16 *out16;      // when set: the output as f16 planes of ldo columns (plane_off's layout)
 };
 constexpr int kF5Hd = kF5HeadDim;
 typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
@@ -358,7 +357,8 @@ __global__ __launch_bounds__(64 * W * KS) void k_f5_attn(F5AttnArgs a) {
     const int qr = q0 + 16 * qw + lr;
     if (qr >= a.N) return;
     const float inv = 1.0f / lrow;
-    const int64_t off = (int64_t(b) * a.N + qr) * a.ldo + int64_t(h) * kF5Hd + 4 * lg;
+    const int64_t orow = int64_t(b) * a.N + qr;
+    const int ocol = h * kF5Hd + 4 * lg;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
         const f32x4a y = o[dt] * inv;
@@ -369,10 +369,11 @@ __global__ __launch_bounds__(64 * W * KS) void k_f5_attn(F5AttnArgs a) {
                 hi[i] = _Float16(y[i]);
                 lo[i] = _Float16(y[i] - float(hi[i]));
             }
-            *reinterpret_cast<h16x4 *>(a.out16 + off + 16 * dt) = hi;
-            *reinterpret_cast<h16x4 *>(a.out16 + a.out_lo + off + 16 * dt) = lo;
+            _Float16 *o16 = a.out16 + plane_off(orow, ocol + 16 * dt, a.ldo);
+            *reinterpret_cast<h16x4 *>(o16) = hi;
+            *reinterpret_cast<h16x4 *>(o16 + kPlaneLo) = lo;
         } else {
-            *reinterpret_cast<f32x4a *>(a.out + off + 16 * dt) = y;
+            *reinterpret_cast<f32x4a *>(a.out + orow * a.ldo + ocol + 16 * dt) = y;
         }
     }
 }

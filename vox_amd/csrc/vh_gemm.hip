@@ -140,7 +140,7 @@ static hipError_t gemm_tile(const uint8_t *w, const float *scale, const float *A
 }
 
 
-static bool rope_h16_ok(const GemmArgs &g) {
+bool rope_h16_ok(const GemmArgs &g) {
     return g.h16 && g.hd > 0 && g.hd % 2 == 0 && g.seq > 0 && g.rope_cols % (2 * g.hd) == 0 && g.m % g.seq == 0 &&
            g.n == g.rope_cols + g.rope_cols / 2 && g.ldvt >= g.seq && g.ldvt % 8 == 0 && g.lo_off % 8 == 0;
 }
@@ -190,110 +190,6 @@ hipError_t launch_gemm(int wt, int epi, const uint8_t *w, const float *scale, co
         case WT_F16: return gemm_epi<WT_F16>(epi, w, scale, A, g, s);
         case WT_BF16: return gemm_epi<WT_BF16>(epi, w, scale, A, g, s);
         case WT_Q8: return g.K % 32 ? hipErrorInvalidValue : gemm_epi<WT_Q8>(epi, w, scale, A, g, s);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-// 64 x 64 tiles, K steps of 64: measured faster on the DiT shapes than 64 x 128 tiles or K steps of 128.
-// Tiles by how many 64 x 64 tiles the product has (measured on the flow estimator's and the DiT's shapes): below 256
-// the 32 x 32 tiles (the 1024 x 256 projections: 4.4 against 8.0 us, and faster than splitting K), below 512 with
-// K <= 512 the 32 x 64 ones (1024 x 1536, K 256: 7.0 against 8.4 us), else 64 x 64 (2000 x 1024, K 1024: 19.0
-// against 21-25 us for the smaller tiles). Below 256 tiles with K >= 2048 (the 512-row prefill's down projection,
-// K 4864) the 64 x 64 tiles split K instead, as the f32-activation GEMM does. Q8: the int8 values as f16 in w, the
-// block scales in q8_scale.
-template <int EPI, int TM, int TN, bool Q8, int WN = 2>
-static hipError_t gemm_hh_tiles(const _Float16 *w, const float *q8_scale, const GemmArgs &g, hipStream_t s) {
-    const dim3 grid(unsigned((g.n + 16 * TN * WN - 1) / (16 * TN * WN)), unsigned((g.m + 32 * TM - 1) / (32 * TM)),
-                    unsigned(g.kchunk ? (g.K + g.kchunk - 1) / g.kchunk : 1));
-    return launch(k_gemm_hh<EPI, TM, TN, 64, Q8, WN>, grid, dim3(128 * WN), 0, s, w, q8_scale, g);
-}
-// A tile forced by voxhip_bench_gemm_hh (0: the policy below): 1 32 x 32, 2 32 x 64, 3 64 x 64, 4 64 x 128 (8
-// waves), as rows of A x rows of W.
-static std::atomic<int> g_hh_tile{0};
-void set_gemm_hh_tile(int tile) { g_hh_tile.store(tile); }
-template <int EPI, bool Q8>
-static hipError_t gemm_hh_forced(int tile, const _Float16 *w, const float *q8_scale, const GemmArgs &g, hipStream_t s) {
-    switch (tile) {
-        case 1: return gemm_hh_tiles<EPI, 1, 1, Q8>(w, q8_scale, g, s);
-        case 2: return gemm_hh_tiles<EPI, 1, 2, Q8>(w, q8_scale, g, s);
-        case 3: return gemm_hh_tiles<EPI, 2, 2, Q8>(w, q8_scale, g, s);
-        case 4: return gemm_hh_tiles<EPI, 2, 2, Q8, 4>(w, q8_scale, g, s);
-        default: return hipErrorInvalidValue;
-    }
-}
-template <int EPI, bool Q8>
-static hipError_t gemm_hh_run(const _Float16 *w, const float *q8_scale, const GemmArgs &g, hipStream_t s) {
-    if (const int tile = g_hh_tile.load()) return gemm_hh_forced<EPI, Q8>(tile, w, q8_scale, g, s);
-    const int64_t blocks = int64_t((g.n + 63) / 64) * ((g.m + 63) / 64);
-    if constexpr (EPI == EPI_STORE || EPI == EPI_ACC || EPI == EPI_GATED_ACC || EPI == EPI_SWIGLU) {
-        GemmArgs gs = g;
-        const int splits = blocks < 256 && g.K >= 2048 ? split_plan(g, &gs.kchunk) : 0;
-        if (splits) {
-            hipError_t e = gemm_hh_tiles<EPI_STORE, 2, 2, Q8>(w, q8_scale, gs, s);
-            return e != hipSuccess ? e : splitk_reduce<EPI>(g, splits, s);
-        }
-    }
-    if (blocks < 256) return gemm_hh_tiles<EPI, 1, 1, Q8>(w, q8_scale, g, s);
-    if (blocks < 512 && g.K <= 512) return gemm_hh_tiles<EPI, 1, 2, Q8>(w, q8_scale, g, s);
-    // f16 weights: 64 x 128 tiles of 8 waves while they still make 256 blocks (the DiT's 2000 x 3072 x 1024 q|k|v
-    // 36.5 against 42.2 us, 2000 x 1024 x 2048 27.9 against 31.2 us, 1000 x 2048 x 1024 16.7 against 19.0 us; at 128
-    // blocks they lose, 1000 x 1024 x 2048 24.9 against 21.6 us; the q8 prefill shapes measured slower, 37.2 against
-    // 36.1 us for 512 x 9728 x 896)
-    if constexpr (!Q8)
-        if (int64_t((g.n + 127) / 128) * ((g.m + 63) / 64) >= 256) return gemm_hh_tiles<EPI, 2, 2, Q8, 4>(w, q8_scale, g, s);
-    return gemm_hh_tiles<EPI, 2, 2, Q8>(w, q8_scale, g, s);
-}
-template <int EPI>
-static hipError_t gemm_hh_wt(const _Float16 *w, const float *q8_scale, const GemmArgs &g, hipStream_t s) {
-    return q8_scale ? gemm_hh_run<EPI, true>(w, q8_scale, g, s) : gemm_hh_run<EPI, false>(w, nullptr, g, s);
-}
-
-static bool hh_args_ok(const _Float16 *w, const float *q8_scale, const GemmArgs &g) {
-    return w && g.a16 && g.n > 0 && g.K > 0 && g.K % 64 == 0 && g.lda >= g.K && g.lda % 8 == 0 && g.a_lo % 8 == 0 &&
-           int64_t(64) * g.lda * 2 <= INT32_MAX && int64_t(64) * g.K * 2 <= INT32_MAX &&
-           (!q8_scale || int64_t(64) * (g.K / 32) * 4 <= INT32_MAX);
-}
-
-hipError_t launch_gemm_hh_acc_rms(const _Float16 *w, const float *q8_scale, const GemmArgs &g0, const float *gamma, float eps,
-                                  _Float16 *out16, int64_t ldo, int64_t lo_off, hipStream_t s, bool *normed) {
-    GemmArgs g = g0;
-    g.status = status_word();
-    *normed = false;
-    if (g.m <= 0) return hipSuccess;
-    if (!hh_args_ok(w, q8_scale, g) || !g.y) return hipErrorInvalidValue;
-    const int64_t blocks = int64_t((g.n + 63) / 64) * ((g.m + 63) / 64);
-    GemmArgs gs = g;
-    const int splits = blocks < 256 && g.K >= 2048 ? split_plan(g, &gs.kchunk) : 0;
-    // the row pass holds 8 columns per thread; without a split the ACC epilogue already wrote y
-    if (!splits || splits > 8 || g.n > 8 * 256 || !gamma || !out16 || ldo < g.n || lo_off % 8)
-        return launch_gemm_hh(EPI_ACC, w, q8_scale, g, s);
-    hipError_t e = q8_scale ? gemm_hh_tiles<EPI_STORE, 2, 2, true>(w, q8_scale, gs, s)
-                            : gemm_hh_tiles<EPI_STORE, 2, 2, false>(w, nullptr, gs, s);
-    if (e != hipSuccess) return e;
-    const dim3 grid(unsigned(g.m));
-    if (g.n <= 4 * 256) e = launch(k_splitk_acc_rms_h16<4>, grid, dim3(256), 0, s, g, int32_t(splits), gamma, eps, out16, ldo, lo_off);
-    else e = launch(k_splitk_acc_rms_h16<8>, grid, dim3(256), 0, s, g, int32_t(splits), gamma, eps, out16, ldo, lo_off);
-    if (e == hipSuccess) *normed = true;
-    return e;
-}
-
-hipError_t launch_gemm_hh(int epi, const _Float16 *w, const float *q8_scale, const GemmArgs &g0, hipStream_t s) {
-    GemmArgs g = g0;
-    g.status = status_word();
-    if (g.m <= 0) return hipSuccess;
-    if (!hh_args_ok(w, q8_scale, g)) return hipErrorInvalidValue;
-    if ((epi == EPI_SWIGLU || epi == EPI_SWIGLU_H16) && g.n % 2) return hipErrorInvalidValue;
-    const bool y_ok = g.y != nullptr;
-    switch (epi) {
-        case EPI_STORE: return y_ok ? gemm_hh_wt<EPI_STORE>(w, q8_scale, g, s) : hipErrorInvalidValue;
-        case EPI_ACC: return y_ok ? gemm_hh_wt<EPI_ACC>(w, q8_scale, g, s) : hipErrorInvalidValue;
-        case EPI_GATED_ACC: return y_ok && g.gate ? gemm_hh_wt<EPI_GATED_ACC>(w, q8_scale, g, s) : hipErrorInvalidValue;
-        case EPI_GELU: return y_ok ? gemm_hh_wt<EPI_GELU>(w, q8_scale, g, s) : hipErrorInvalidValue;
-        case EPI_SWIGLU: return y_ok && g.ldy >= g.n / 2 ? gemm_hh_wt<EPI_SWIGLU>(w, q8_scale, g, s) : hipErrorInvalidValue;
-        case EPI_GELU_H16: return g.h16 && g.ldy >= g.n ? gemm_hh_wt<EPI_GELU_H16>(w, q8_scale, g, s) : hipErrorInvalidValue;
-        case EPI_SWIGLU_H16:
-            return g.h16 && g.ldy >= g.n / 2 ? gemm_hh_wt<EPI_SWIGLU_H16>(w, q8_scale, g, s) : hipErrorInvalidValue;
-        case EPI_ROPE_H16: return rope_h16_ok(g) ? gemm_hh_wt<EPI_ROPE_H16>(w, q8_scale, g, s) : hipErrorInvalidValue;
         default: return hipErrorInvalidValue;
     }
 }

@@ -136,20 +136,9 @@ VH_DEV void gemm_epilogue(const f32x4v (&acc)[TM][TN], const GemmArgs &g, int m0
                 const float c = acc[i][j][v] + bz;
                 const bool in = row < g.m && col < g.n;
                 float *dst = g.y + int64_t(row) * g.ldy + col;
-                if (EPI == EPI_SWIGLU || EPI == EPI_SWIGLU_H16) {
+                if (EPI == EPI_SWIGLU) {
                     const float up = __shfl_xor(c, 1, kWave);  // column col ^ 1 of the same row
-                    if (in && (col & 1) == 0) {
-                        const float r = silu(c) * up;
-                        if (EPI == EPI_SWIGLU) {
-                            g.y[int64_t(row) * g.ldy + col / 2] = r;
-                        } else {
-                            _Float16 hi, lo;
-                            bad |= split_f16(r, hi, lo);
-                            const int64_t idx = int64_t(row) * g.ldy + col / 2;
-                            g.h16[idx] = hi;
-                            g.h16[g.lo_off + idx] = lo;
-                        }
-                    }
+                    if (in && (col & 1) == 0) g.y[int64_t(row) * g.ldy + col / 2] = silu(c) * up;
                 } else if (EPI == EPI_ROPE || EPI == EPI_ROPE_H16) {
                     const float o = __shfl_xor(c, 1, kWave);  // the pair partner (2j <-> 2j + 1)
                     float r = c;
@@ -184,14 +173,6 @@ VH_DEV void gemm_epilogue(const f32x4v (&acc)[TM][TN], const GemmArgs &g, int m0
                     else if (EPI == EPI_GATED_ACC) *dst += gt * c;
                     else if (EPI == EPI_GELU) *dst = gelu_tanh_f(c);
                     else if (EPI == EPI_GELU_ERF) *dst = gelu_erf_f(c);
-                    else if (EPI == EPI_GELU_H16) {
-                        const float r = g.gelu_erf ? gelu_erf_f(c) : gelu_tanh_f(c);
-                        _Float16 hi, lo;
-                        bad |= split_f16(r, hi, lo);
-                        const int64_t idx = int64_t(row) * g.ldy + col;
-                        g.h16[idx] = hi;
-                        g.h16[g.lo_off + idx] = lo;
-                    }
                     else if (EPI == EPI_SNAKE) {
                         const float sn = sinf(c * g.snake_a[col]);
                         *dst = c + g.snake_ib[col] * sn * sn;
@@ -231,7 +212,7 @@ VH_DEV void gemm_store_partial(const f32x4v (&acc)[TM][TN], const GemmArgs &g, i
 // silu(gate) * up; EPI_GATED_ACC y += gate[col] * (c + bias); EPI_GELU y = gelu_tanh(c + bias); EPI_MISH
 // y = mish(c + bias); EPI_MISH_ACC y += mish(c + bias); EPI_GELU_ERF y = gelu_erf(c + bias); EPI_ROPE y = c + bias
 // with the pairs of q | k rotated;
-// EPI_ROPE_H16 and EPI_GELU_H16 write their results as f16 halves (hi, lo) for a following split-f16 product.
+// EPI_ROPE_H16 writes its results as f16 halves (hi, lo) for the attention's split-f16 products.
 // ASRC_CONV: W (F32) and y columns are those of group blockIdx.z.
 template <int WT, int EPI, int ASRC, int TM, int TN>
 __global__ __launch_bounds__(256) void k_gemm_f32(const uint8_t *__restrict__ w, const float *__restrict__ scale,
@@ -550,7 +531,7 @@ __global__ __launch_bounds__(256) void k_gemm_h16(const uint8_t *__restrict__ w,
     gemm_epilogue<EPI, TM, TN>(acc, g, m0, n0, wm, wn, lane);
 }
 
-// k_gemm_h16 for K (and the split-K chunk) a multiple of 64, with k_gemm_hh's load pipeline: buffer loads cut at
+// k_gemm_h16 for K (and the split-K chunk) a multiple of 64, with buffer loads cut at
 // the tile's last row of A and of W (rows past m or n read as zeros, no per-load bounds check, the K offset in the
 // scalar operand), two K steps in flight in alternating register sets, unconditional fetches (steps past the end
 // re-read the last one) so the wait counts are exact. A arrives as f32 and is split into hi / lo at staging; Q8
@@ -694,195 +675,6 @@ __global__ __launch_bounds__(256) void k_gemm_h16b(const uint8_t *__restrict__ w
     raise_status(g.status, bad, kStatusF16Range);
     if (g.kchunk) return gemm_store_partial<2, 2>(acc, g, m0, n0, wm, wn, lane);
     gemm_epilogue<EPI, 2, 2>(acc, g, m0, n0, wm, wn, lane);
-}
-
-// The split-f16 GEMM of k_gemm_h16 when the producer has already split A: hi plane g.a16, lo plane g.a16 + g.a_lo
-// (rows of g.lda halves), K a multiple of BK. Weights: F16, or (Q8) the int8 values of Q8 weights widened once to f16
-// (exact) with their block scales `scale` [n][K / 32], applied per 32-deep block as k_gemm_h16 does (the block's
-// two MFMAs start from zero, s (q . a) goes into the accumulator). Block tile 32 TM rows of A x 32 TN rows of W (4
-// waves of 16 TM x 16 TN), K steps of BK through LDS as 16-byte copies (rows padded by 16 halves: fewer LDS bank
-// conflicts than 8 on the DiT shapes), no conversion. The loads go through buffer resources cut at the block's last
-// row of A and of W, so rows past m or n read as zeros without a per-load bounds check, and the K offset of a step
-// is the scalar offset. Two K steps are in flight (two register sets alternate), so a load has two steps' MFMAs to
-// arrive. g.kchunk: slice blockIdx.z of K (a multiple of BK) as partial sums into g.ws (k_gemm_splitk_reduce).
-template <int EPI, int TM, int TN, int BK, bool Q8 = false, int WN = 2>
-// The q8 instances hold the accumulators in VGPRs for the scale FMA; asking for 4 waves per SIMD (128 VGPRs, a
-// register or two spilled) measured faster on the prefill shapes than the 3 their unconstrained 165 registers allow.
-__global__ __launch_bounds__(128 * WN) __attribute__((amdgpu_waves_per_eu(Q8 ? 4 : 1))) void k_gemm_hh(const _Float16 *__restrict__ w, const float *__restrict__ scale, GemmArgs g) {
-    // 2 x WN waves of 16 TM x 16 TN outputs each (WN = 2: 64 x 64 tiles for TM = TN = 2, 256 threads; WN = 4: 64 x 128,
-    // 512 threads, so each block's A tile serves twice the columns)
-    constexpr int NT = 128 * WN, LD = BK + 16, BM = 32 * TM, BN = 16 * TN * WN, CPR = BK / 8, RS = NT / CPR, AQ = BM / RS,
-                  WQ = BN / RS;
-    constexpr int SB = BK / 32;  // scale blocks per K step
-    static_assert(AQ >= 1 && WQ >= 1 && BM % RS == 0 && BN % RS == 0, "tile rows per load pass");
-    static_assert(!Q8 || BN * SB <= NT, "one scale per thread per K step");
-    __shared__ __align__(16) _Float16 Ah[BM][LD], Al[BM][LD], Bs[BN][LD];
-    __shared__ float Ss[Q8 ? BN : 1][SB];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave / WN, wn = wave % WN;
-    int tm, tn;  // A as two f16 planes (4 bytes an element) against W f16 (2)
-    gemm_tile(gridDim.x, gridDim.y, g.n > 2 * g.m, tm, tn);
-    const int m0 = tm * BM, n0 = tn * BN, K = g.K, nb = K / 32;
-    const int kbeg = g.kchunk ? int(blockIdx.z) * g.kchunk : 0, kend = g.kchunk ? min(K, kbeg + g.kchunk) : K;
-    const int mr = min(BM, g.m - m0), nr = min(BN, g.n - n0);
-    const _Float16 *a0 = g.a16 + int64_t(m0) * g.lda;
-    const __amdgpu_buffer_rsrc_t rah = buf_rsrc(a0, int32_t(mr * g.lda * 2));
-    const __amdgpu_buffer_rsrc_t ral = buf_rsrc(a0 + g.a_lo, int32_t(mr * g.lda * 2));
-    const __amdgpu_buffer_rsrc_t rw = buf_rsrc(w + int64_t(n0) * K, nr * K * 2);
-    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(Q8 ? scale + int64_t(n0) * nb : scale, Q8 ? nr * nb * 4 : 0);
-    // this thread's 8-half chunks of a tile: rows r + RS q, columns c8 .. c8 + 7
-    const int r = tid / CPR, c8 = (tid % CPR) * 8;
-    int va[AQ], vw[WQ];
-#pragma unroll
-    for (int q = 0; q < AQ; ++q) va[q] = int32_t(((r + RS * q) * g.lda + c8) * 2);
-#pragma unroll
-    for (int q = 0; q < WQ; ++q) vw[q] = ((r + RS * q) * K + c8) * 2;
-    const int vs = ((tid / SB) * nb + tid % SB) * 4;  // Q8: threads < BN SB take row tid / SB, block tid % SB
-    f32x4v acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    u32x4 xa0[2 * AQ], xw0[WQ], xa1[2 * AQ], xw1[WQ];
-    float xs0 = 0.f, xs1 = 0.f;
-    auto fetch = [&](u32x4(&a)[2 * AQ], u32x4(&b)[WQ], float &sc, int k0) {
-        const int so = k0 * 2;
-#pragma unroll
-        for (int q = 0; q < AQ; ++q) {
-            a[q] = buf_ld16(rah, va[q], so);
-            a[AQ + q] = buf_ld16(ral, va[q], so);
-        }
-#pragma unroll
-        for (int q = 0; q < WQ; ++q) b[q] = buf_ld16(rw, vw[q], so);
-        if (Q8) sc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, vs, k0 / 32 * 4, 0));
-    };
-    auto stage = [&](const u32x4(&a)[2 * AQ], const u32x4(&b)[WQ], float sc) {
-#pragma unroll
-        for (int q = 0; q < AQ; ++q) {
-            *reinterpret_cast<u32x4 *>(&Ah[r + RS * q][c8]) = a[q];
-            *reinterpret_cast<u32x4 *>(&Al[r + RS * q][c8]) = a[AQ + q];
-        }
-#pragma unroll
-        for (int q = 0; q < WQ; ++q) *reinterpret_cast<u32x4 *>(&Bs[r + RS * q][c8]) = b[q];
-        if (Q8 && tid < BN * SB) Ss[tid / SB][tid % SB] = sc;
-    };
-    auto mma = [&]() {
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 32) {
-            f16x8v ah[TM], al[TM], b[TN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const int rr = wm * 16 * TM + i * 16 + (lane & 15);
-                ah[i] = *reinterpret_cast<const f16x8v *>(&Ah[rr][kk + 8 * (lane >> 4)]);
-                al[i] = *reinterpret_cast<const f16x8v *>(&Al[rr][kk + 8 * (lane >> 4)]);
-            }
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                b[j] = *reinterpret_cast<const f16x8v *>(&Bs[wn * 16 * TN + j * 16 + (lane & 15)][kk + 8 * (lane >> 4)]);
-            if (Q8) {
-                float sc[TN];  // the block scale of this lane's W row (its C column)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) sc[j] = Ss[wn * 16 * TN + j * 16 + (lane & 15)][kk / 32];
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        f32x4v tt = {0.f, 0.f, 0.f, 0.f};
-                        tt = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], b[j], tt, 0, 0, 0);
-                        tt = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], b[j], tt, 0, 0, 0);
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) acc[i][j][v] = fmaf(tt[v], sc[j], acc[i][j][v]);
-                    }
-            } else {
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], b[j], acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], b[j], acc[i][j], 0, 0, 0);
-                    }
-            }
-        }
-    };
-    // Every fetch is unconditional (steps past the end re-read the last one), so the compiler's count of loads in
-    // flight is exact: staging one set waits only for that set, the other stays in flight.
-    const int ns = (kend - kbeg) / BK, klast = kend - BK;
-    fetch(xa0, xw0, xs0, kbeg);
-    __builtin_amdgcn_sched_barrier(0);  // keep the first set's loads ahead of the second's
-    fetch(xa1, xw1, xs1, min(kbeg + BK, klast));
-    for (int s = 0; s + 1 < ns; s += 2) {  // one back edge: the first set is always the older in flight
-        stage(xa0, xw0, xs0);
-        __syncthreads();
-        fetch(xa0, xw0, xs0, min(kbeg + (s + 2) * BK, klast));
-        mma();
-        __syncthreads();
-        stage(xa1, xw1, xs1);
-        __syncthreads();
-        fetch(xa1, xw1, xs1, min(kbeg + (s + 3) * BK, klast));
-        mma();
-        __syncthreads();
-    }
-    if (ns & 1) {  // the last step, in the first set
-        stage(xa0, xw0, xs0);
-        __syncthreads();
-        mma();
-    }
-    if (g.kchunk) return gemm_store_partial<TM, TN>(acc, g, m0, n0, wm, wn, lane);
-    gemm_epilogue<EPI, TM, TN>(acc, g, m0, n0, wm, wn, lane);
-}
-
-// The split-K slices of an EPI_ACC product added into its rows, y[row][c] += (sum_z ws[z][row][c]) + bias[c], as
-// k_gemm_splitk_reduce<EPI_ACC> does, then the RMSNorm (gamma, eps) of each updated row written as f16 halves (hi at
-// out16, lo at out16 + lo_off, rows of ldo halves) with k_rmsnorm_rows_h16's arithmetic: the residual add and the
-// next norm in one pass over the row. grid m, block 256, n <= 256 NV, splits <= 8.
-template <int NV>
-__global__ __launch_bounds__(256) void k_splitk_acc_rms_h16(GemmArgs g, int32_t splits, const float *gamma, float eps,
-                                                           _Float16 *out16, int64_t ldo, int64_t lo_off) {
-    __shared__ float red[4];
-    const int row = int(blockIdx.x);
-    const int64_t slice = int64_t(g.m) * g.n;
-    float *yr = g.y + int64_t(row) * g.ldy;
-    // every slice's value and the row's own first, so the loads are in flight together (slices past `splits`, at
-    // most kMaxSplits, read slice 0 and are left out), then the sums in split order as the reduce kernel adds them
-    constexpr int kMaxSplits = 8;
-    float t[NV][kMaxSplits], hv[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        const int c = min(int(threadIdx.x) + 256 * k, g.n - 1);
-        hv[k] = yr[c];
-#pragma unroll
-        for (int z = 0; z < kMaxSplits; ++z) t[k][z] = g.ws[(z < splits ? z : 0) * slice + int64_t(row) * g.n + c];
-    }
-    float ss = 0.f;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        const int c = int(threadIdx.x) + 256 * k;
-        if (c < g.n) {
-            float v = 0.f;
-#pragma unroll
-            for (int z = 0; z < kMaxSplits; ++z)
-                if (z < splits) v += t[k][z];
-            v = v + (g.bias ? g.bias[c] : 0.f);
-            hv[k] = hv[k] + v;
-            yr[c] = hv[k];
-            ss = fmaf(hv[k], hv[k], ss);
-        } else {
-            hv[k] = 0.f;
-        }
-    }
-    ss = block_sum<256>(ss, red);
-    const float inv = 1.0f / sqrtf(ss / float(g.n) + eps);
-    bool bad = false;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        const int c = int(threadIdx.x) + 256 * k;
-        if (c < g.n) {
-            _Float16 hi, lo;
-            bad |= split_f16(gamma[c] * (hv[k] * inv), hi, lo);
-            out16[int64_t(row) * ldo + c] = hi;
-            out16[lo_off + int64_t(row) * ldo + c] = lo;
-        }
-    }
-    raise_status(g.status, bad, kStatusF16Range);
 }
 
 }  // namespace vh

@@ -4,20 +4,6 @@
 
 namespace vh {
 
-// Four f32 values as f16 halves (split_f16x2).
-VH_DEV void split4(const f32x4v &x, uint2 &hi, uint2 &lo) {
-    split_f16x2(x[0], x[1], hi.x, lo.x);
-    split_f16x2(x[2], x[3], hi.y, lo.y);
-}
-// The range check of the split, two instructions a value: |x| is finite and >= 65520 exactly when twice its magnitude
-// bits less those of 65520, unsigned, is below the distance to infinity. ovf4 keeps the smallest such difference seen.
-constexpr uint32_t kOvfBase = 0x477FF000u << 1, kOvfSpan = (0x7F800000u << 1) - (0x477FF000u << 1);
-VH_DEV uint32_t ovf4(const f32x4v &x, uint32_t mn) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) mn = min(mn, (__float_as_uint(x[e]) << 1) - kOvfBase);
-    return mn;
-}
-
 // F32 weights and f32 activations on the f16 matrix cores, as k_gemm_x3 takes them (both as f16 halves, three products
 // per pair, the weights scaled by 2^10), for weights laid
 // out once by k_pack_x3 in the order the MFMA reads them: [n / 16][k / 32][hi, lo][lane][8]. A wave then loads its W
@@ -143,6 +129,7 @@ VH_DEV void x3p_body(const uint8_t *__restrict__ w, const float *__restrict__ A,
         }
     };
     const int ns = (kend - kbeg + BK - 1) / BK;
+    const int rbase = m0 + 16 * wm * TM + lr, cbase = n0 + 16 * wn * TN + 4 * lg;
     fetch_a(ra[0], kbeg);
     fetch_w(0, kbeg);
     __builtin_amdgcn_sched_barrier(0);
@@ -167,32 +154,19 @@ VH_DEV void x3p_body(const uint8_t *__restrict__ w, const float *__restrict__ A,
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = (acc[i][j] + acx[i][j]) * kWsInv;
-    const int rbase = m0 + 16 * wm * TM + lr, cbase = n0 + 16 * wn * TN + 4 * lg;
     if (g.kchunk) {
         float *ws = g.ws + int64_t(blockIdx.z) * g.m * g.n;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int r = rbase + 16 * i, c = cbase + 16 * j;
-                if (r >= g.m) continue;
-                const f32x4v v = acc[i][j];
-                if (g.n % 4 == 0) {
-                    if (c < g.n) *reinterpret_cast<f32x4v *>(ws + int64_t(r) * g.n + c) = v;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (c + e < g.n) ws[int64_t(r) * g.n + c + e] = v[e];
-                }
-            }
+            for (int j = 0; j < TN; ++j)
+                store_partial(acc[i][j], ws, g, rbase + 16 * i, cbase + 16 * j);
         return;
     }
-    const bool vec = epi_vec<EPI>(g);
     bool bad = false;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) epi_tile<EPI>(acc[i][j], g, rbase + 16 * i, cbase + 16 * j, vec, lane, bad);
+    EpiOps<EPI, TM, TN> ops;  // here, not before the loop: its registers are the loop's own
+    ops.load(g, rbase, cbase);
+    ops.finish(acc, g, rbase, cbase, lane, bad);
     raise_status(g.status, bad, kStatusF16Range);
 }
 

@@ -155,7 +155,7 @@ const char *prof_report(const char *device) {
                   "avg us", "share");
     g_report += line;
     for (const auto &p : v) {
-        std::snprintf(line, sizeof line, "  %-28s %8llu %10.2f %9.1f %5.1f%%\n", p.first.c_str(),
+        std::snprintf(line, sizeof line, "  %-28s %8llu %10.3f %9.1f %5.1f%%\n", p.first.c_str(),
                       (unsigned long long)p.second.calls, p.second.ns / 1e6,
                       p.second.ns / 1e3 / double(std::max<uint64_t>(1, p.second.calls)), 100.0 * p.second.ns / std::max(1.0, total));
         g_report += line;
@@ -339,16 +339,11 @@ hipError_t launch_rmsnorm_rows(const float *x, int64_t ldx, const float *w, int 
     if (m <= 0) return hipSuccess;
     return launch(k_rmsnorm_rows, dim3(m), dim3(256), 0, s, x, ldx, w, K, eps, out, ldo);
 }
-hipError_t launch_rmsnorm_rows_h16(const float *x, int64_t ldx, const float *w, int K, float eps, _Float16 *out16,
-                                   int64_t ldo, int64_t lo_off, int m, hipStream_t s) {
+hipError_t launch_rmsnorm_rows_h16(const float *x, int64_t ldx, const float *w, int K, float eps, _Float16 *out16, int m,
+                                   hipStream_t s) {
     if (m <= 0) return hipSuccess;
-    if (!out16 || ldo < K || lo_off < int64_t(m) * ldo) return hipErrorInvalidValue;
-    return launch(k_rmsnorm_rows_h16, dim3(m), dim3(256), 0, s, x, ldx, w, K, eps, out16, ldo, lo_off, status_word());
-}
-hipError_t launch_q8_to_f16(const int8_t *q, _Float16 *out, int64_t n, hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    if (n % 8) return hipErrorInvalidValue;
-    return launch(k_q8_to_f16, grid1(n / 8, 256), dim3(256), 0, s, q, out, n);
+    if (!out16 || K <= 0 || K % 32) return hipErrorInvalidValue;
+    return launch(k_rmsnorm_rows_h16, dim3(m), dim3(256), 0, s, x, ldx, w, K, eps, out16, status_word());
 }
 hipError_t launch_fill_normal(float *out, int64_t n, uint64_t seed, uint32_t stream, float mean, float std,
                               hipStream_t s) {

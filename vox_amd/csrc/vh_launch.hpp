@@ -59,17 +59,27 @@ hipError_t launch_qk_post(const QkArgs &a, int m, hipStream_t s);
 // Multi-row f32 GEMM on the matrix cores (F32 / F16 / BF16 / Q8 weights).
 hipError_t launch_gemm(int wt, int epi, const uint8_t *w, const float *scale, const float *A, const GemmArgs &g, hipStream_t s);
 // Grouped "same" Conv1d as an implicit-im2col GEMM (f32 weights [groups][cout/groups][K][cin/groups]).
-// Split-f16 GEMM with A already split by its producer (g.a16 hi, g.a16 + g.a_lo lo), K % 64 == 0: F16 weights
-// (q8_scale null), or Q8 weights as their int8 values widened to f16 with the block scales [n][K / 32] in q8_scale;
-// epilogues STORE, ACC, GATED_ACC, GELU, SWIGLU, GELU_H16, SWIGLU_H16, ROPE_H16 (split K uses g.ws).
-hipError_t launch_gemm_hh(int epi, const _Float16 *w, const float *q8_scale, const GemmArgs &g, hipStream_t s);
+// The h16 buffers of EPI_ROPE_H16 fit the product.
+bool rope_h16_ok(const GemmArgs &g);
+// Split-f16 GEMM with A already in f16 planes by its producer (g.a16, plane_off's layout), K % 64 == 0: F16 weights in
+// fragment order (launch_pack_f16; scale_t null), or Q8 weights as their int8 values in that order with the block scales
+// transposed (launch_scale_t); epilogues STORE, ACC, SWIGLU_H16, and for F16 weights GATED_ACC, GELU_H16, ROPE_H16 (split K
+// uses g.ws).
+hipError_t launch_gemm_hh(int epi, const _Float16 *w, const float *scale_t, const GemmArgs &g, hipStream_t s);
+// F16 weights (q8: int8 values) [n][K], K % 32 == 0, in fragment order: pack_f16_halves(n, K) halves at out. Block scales
+// [n][K / 32] transposed: scale_t_floats(n, K) floats. hi / lo rows [m][K] into planes (planes_halves(m, K) halves).
+int64_t pack_f16_halves(int64_t n, int64_t K);
+hipError_t launch_pack_f16(const uint8_t *w, bool q8, int64_t n, int64_t K, _Float16 *out, hipStream_t s);
+int64_t scale_t_floats(int64_t n, int64_t K);
+hipError_t launch_scale_t(const float *sc, int64_t n, int64_t K, float *out, hipStream_t s);
+hipError_t launch_pack_planes(const _Float16 *hi, const _Float16 *lo, int64_t m, int64_t K, _Float16 *out, hipStream_t s);
 // Forces launch_gemm_hh's block tile (0: its shape policy); voxhip_bench_gemm_hh only.
 void set_gemm_hh_tile(int tile);
-// The same with EPI_ACC, and when the product splits K, the next RMSNorm (gamma, eps) of the updated rows of y written
-// as f16 halves (out16, ldo, lo_off as launch_rmsnorm_rows_h16) by the split-K reduce itself: *normed tells whether
-// it did (otherwise the caller runs the norm).
-hipError_t launch_gemm_hh_acc_rms(const _Float16 *w, const float *q8_scale, const GemmArgs &g, const float *gamma, float eps,
-                                  _Float16 *out16, int64_t ldo, int64_t lo_off, hipStream_t s, bool *normed);
+// The same with EPI_ACC, and when the product splits K, the next RMSNorm (gamma, eps) of the updated rows of y into planes
+// out16 (as launch_rmsnorm_rows_h16) by the split-K reduce itself: *normed tells whether it did (otherwise the caller runs
+// the norm).
+hipError_t launch_gemm_hh_acc_rms(const _Float16 *w, const float *scale_t, const GemmArgs &g, const float *gamma, float eps,
+                                  _Float16 *out16, hipStream_t s, bool *normed);
 // F32 weights [n][K] as k_gemm_x3p reads them, pack_x3_bytes(n, K) bytes at out (weights of |w| < 64).
 int64_t pack_x3_bytes(int64_t n, int64_t K);
 hipError_t launch_pack_x3(const float *w, int64_t n, int64_t K, void *out, hipStream_t s);
@@ -97,11 +107,9 @@ hipError_t launch_to_f16(const float *x, int64_t n, void *y, hipStream_t s);
 hipError_t launch_to_bf16(const float *x, int64_t n, void *y, hipStream_t s);
 hipError_t launch_rmsnorm_rows(const float *x, int64_t ldx, const float *w, int K, float eps, float *out, int64_t ldo,
                                int m, hipStream_t s);
-// The same RMSNorm written as f16 halves (hi rows of ldo halves at out16, lo rows at out16 + lo_off).
-hipError_t launch_rmsnorm_rows_h16(const float *x, int64_t ldx, const float *w, int K, float eps, _Float16 *out16,
-                                   int64_t ldo, int64_t lo_off, int m, hipStream_t s);
-// int8 values widened to f16 (n a multiple of 8).
-hipError_t launch_q8_to_f16(const int8_t *q, _Float16 *out, int64_t n, hipStream_t s);
+// The same RMSNorm into f16 planes (plane_off's layout of K columns; K % 32 == 0).
+hipError_t launch_rmsnorm_rows_h16(const float *x, int64_t ldx, const float *w, int K, float eps, _Float16 *out16, int m,
+                                   hipStream_t s);
 hipError_t launch_fill_normal(float *out, int64_t n, uint64_t seed, uint32_t stream, float mean, float std,
                               hipStream_t s);
 hipError_t launch_fill_cache(void *c, int64_t planes, int64_t cap, int64_t len, int hd, uint64_t seed, uint32_t stream,
@@ -120,7 +128,7 @@ hipError_t launch_attn_rows(const AttnRowsArgs &a, int m, hipStream_t s);
 hipError_t launch_prefill_attn(const PrefillAttnArgs &a, int hd, hipStream_t s);
 // F5-TTS DiT step: AdaLN modulation of R rows of D, the step input's x columns, attention (head_dim 64).
 hipError_t launch_f5_modulate(const float *x, int64_t R, int D, const float *sc, const float *sh, float *y, _Float16 *y16,
-                              int64_t lo_off, hipStream_t s);
+                              hipStream_t s);
 hipError_t launch_f5_fill_x(const float *x, int N, int mel, float *cat, int W, int B, hipStream_t s);
 // Vocos: LayerNorm with weight and bias (double statistics, eps 1e-6) of R rows of D; depthwise "same" conv over
 // batches of seq rows (w [C][K], bias or null).
@@ -128,7 +136,7 @@ hipError_t launch_layernorm_rows(const float *x, int64_t R, int D, const float *
 // Any row norm of NormArgs (LayerNorm / modulation, optional mish and channel bias; the CosyVoice2 estimator's blocks).
 hipError_t launch_norm_rows(const NormArgs &a, hipStream_t s);
 hipError_t launch_dwconv(const float *x, const float *w, const float *b, float *y, int64_t R, int C, int K, int seq, hipStream_t s);
-hipError_t launch_f5_attn(const _Float16 *qkv16, int64_t lo_off, float *out, _Float16 *out16, int64_t out_lo, int B, int N,
+hipError_t launch_f5_attn(const _Float16 *qkv16, int64_t lo_off, float *out, _Float16 *out16, int B, int N,
                           int heads, int hd, int ldvt, int ldo, float scale, hipStream_t s);
 // Qwen3-TTS codec decoder: streaming histories (dst != old), the causal depthwise conv, the transposed conv's
 // overlap-add (tail_old -> tail_new, K <= 2 stride, with an optional Snake output), the pre-transformer's RoPE + ring

@@ -185,8 +185,9 @@ __global__ __launch_bounds__(256) void k_prefill_attn(PrefillAttnArgs a) {
             for (int dt = 0; dt < ND; ++dt) {
                 const float x = o[dt][i] * inv;
                 const _Float16 hi = _Float16(x);
-                a.out16[off + 16 * dt + lr] = hi;
-                a.out16[a.lo_off + off + 16 * dt + lr] = _Float16(x - float(hi));
+                _Float16 *o16 = a.out16 + plane_off(row, h * HD + 16 * dt + lr, int(qd));
+                o16[0] = hi;
+                o16[kPlaneLo] = _Float16(x - float(hi));
             }
         } else {
 #pragma unroll
@@ -196,8 +197,7 @@ __global__ __launch_bounds__(256) void k_prefill_attn(PrefillAttnArgs a) {
 }
 
 // The runs of a key-split prefill attention merged per (row, head): M = the runs' largest max, the sums and
-// outputs scaled by exp(max - M) and added in run order, then out = O (1 / L) as f32 or as f16 halves (hi at out16,
-// lo at out16 + lo_off). grid (ceil(heads HD / 256), m), block 256: thread t of a block takes element t % HD of
+// outputs scaled by exp(max - M) and added in run order, then out = O (1 / L) as f32 or as f16 planes. grid (ceil(heads HD / 256), m), block 256: thread t of a block takes element t % HD of
 // head (256 blockIdx.x + t) / HD; every run's values are loaded before any is used.
 template <int HD>
 __global__ __launch_bounds__(256) void k_pattn_merge(PrefillAttnArgs a) {
@@ -229,8 +229,9 @@ __global__ __launch_bounds__(256) void k_pattn_merge(PrefillAttnArgs a) {
     const int64_t off = int64_t(i) * a.heads * HD + int64_t(h) * HD + e;
     if (a.out16) {
         const _Float16 hi = _Float16(x);
-        a.out16[off] = hi;
-        a.out16[a.lo_off + off] = _Float16(x - float(hi));
+        _Float16 *o16 = a.out16 + plane_off(i, h * HD + e, a.heads * HD);
+        o16[0] = hi;
+        o16[kPlaneLo] = _Float16(x - float(hi));
     } else {
         a.out[off] = x;
     }

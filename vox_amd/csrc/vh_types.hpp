@@ -136,8 +136,7 @@ struct PrefillAttnArgs {
     const float *q;        // [m][heads hd] normed + rotated queries
     const _Float16 *k, *v; // the sequence's cache bases ([layer][kv_head][cap][hd])
     float *out;            // [m][heads hd]
-    _Float16 *out16;       // or, when set, the output as f16 halves: hi [m][heads hd] at out16, lo at out16 + lo_off
-    int64_t lo_off;
+    _Float16 *out16;       // or, when set, the output as f16 planes of heads hd columns (plane_off's layout)
     const RowRef *rows;    // the pass's row table: the kernel takes pos0 from rows[0].pos, so a captured pass
                            // replays at whatever position the host last wrote there
     int64_t cap, pos0;     // pos0: the host's copy of rows[0].pos at launch, checked against cap
@@ -189,14 +188,12 @@ struct GemmArgs {
     // h16 instead of y: plane hi then plane lo (lo_off halves apart), each = q | k rows [m][rope_cols] followed by
     // v transposed per batch and head, [m / seq][heads][hd][ldvt] (ldvt >= seq, a multiple of 8); rope null: the
     // same layout without the rotation
-    // EPI_GELU_H16: gelu(c + bias) as f16 halves into h16 (hi) and h16 + lo_off (lo), rows of ldy halves; the tanh
+    // EPI_GELU_H16: gelu(c + bias) into f16 planes h16 of ldy columns (plane_off's layout); the tanh
     // form, or the erf form when gelu_erf is set. EPI_SWIGLU_H16: EPI_SWIGLU's silu(gate) up written the same way.
     _Float16 *h16;
     int64_t lo_off;
     int32_t ldvt;
-    // k_gemm_hh: A already split into f16 halves, hi plane a16 and lo plane a16 + a_lo, rows of lda halves
-    const _Float16 *a16;
-    int64_t a_lo;
+    const _Float16 *a16;  // k_gemm_hh: A as f16 planes of K columns (plane_off's layout)
     // ASRC_CONV: x [m][lda] rows of `seq`-row batches; group g = blockIdx.z reads channels [g cig, (g + 1) cig) at
     // rows t + k - ksize / 2 of the same batch (causal: t + k - (ksize - 1)) (zeros outside) for A column k cig + i;
     // W and y are offset per group
@@ -262,12 +259,11 @@ struct LmEmbedArgs {
 // Row LayerNorm of R rows of D (k_f5_modulate), one wave per row, double statistics:
 // n = (x - float(mean)) * float(1 / sqrt(var + eps)); modulate (affine 0): y = n * (1 + sc) + sh; affine:
 // y = n * sc + sh (sh null: 0); then mish (the nn.hpp form) when set, then + tb (null: none). y as f32 rows, or as
-// f16 halves (hi at y16, lo at y16 + lo_off) when y16 is set. x and y may be the same rows.
+// f16 planes of D columns (plane_off's layout) when y16 is set. x and y may be the same rows.
 struct NormArgs {
     const float *x;
     float *y;
     _Float16 *y16;
-    int64_t lo_off;
     const float *sc, *sh, *tb;
     double eps;
     int32_t R, D, affine, mish;
@@ -292,6 +288,8 @@ struct PredEmbedArgs {
     RowRef base;           // cache view of the sequence; pos = pos0
     int32_t *err;          // set to 1 when a code falls outside the embedding
 };
+// Halves of the f16 planes (plane_off's layout) of m rows of K columns.
+inline int64_t planes_halves(int64_t m, int64_t K) { return (m + 15) / 16 * 16 * K * 2; }
 constexpr int kF5HeadDim = 64;   // head_dim of the F5 attention kernel
 constexpr int kLmMaxK = 1024;  // top_k limit of the device RAS sampler (sorted in LDS above 64)
 constexpr int kLmMaxN = 8192;  // vocabulary limit of the device RAS sampler (8 entries per thread)

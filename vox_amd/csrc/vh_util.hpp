@@ -91,12 +91,12 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float *x, int64_t ld
     for (int i = threadIdx.x; i < K; i += 256) out[int64_t(blockIdx.x) * ldo + i] = w[i] * (xr[i] * inv);
 }
 
-// k_rmsnorm_rows with the normed rows written as f16 halves for a split-f16 product: x = hi + lo, hi = f16(x),
-// lo = f16(x - hi); hi rows of ldo halves at out16, lo rows at out16 + lo_off.
+// k_rmsnorm_rows with the normed rows written into f16 planes for a split-f16 product: x = hi + lo, hi = f16(x),
+// lo = f16(x - hi), in plane_off's layout of K columns (K % 32 == 0).
 // Rows of up to 8 x 256 values keep the row and the weights in registers, both loaded before the sum, so the
 // weights' round trip overlaps the row's; the sums and products are those of the loop below.
 __global__ __launch_bounds__(256) void k_rmsnorm_rows_h16(const float *x, int64_t ldx, const float *w, int K, float eps,
-                                                         _Float16 *out16, int64_t ldo, int64_t lo_off, int32_t *status) {
+                                                         _Float16 *out16, int32_t *status) {
     __shared__ float red[4];
     const float *xr = x + int64_t(blockIdx.x) * ldx;
     float ss = 0.f;
@@ -121,8 +121,9 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows_h16(const float *x, int64_
             if (i >= K) continue;
             _Float16 hi, lo;
             bad |= split_f16(wv[c] * (xv[c] * inv), hi, lo);
-            out16[int64_t(blockIdx.x) * ldo + i] = hi;
-            out16[lo_off + int64_t(blockIdx.x) * ldo + i] = lo;
+            _Float16 *o = out16 + plane_off(int64_t(blockIdx.x), i, K);
+            o[0] = hi;
+            o[kPlaneLo] = lo;
         }
         raise_status(status, bad, kStatusF16Range);
         return;
@@ -133,21 +134,11 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows_h16(const float *x, int64_
     for (int i = threadIdx.x; i < K; i += 256) {
         _Float16 hi, lo;
         bad |= split_f16(w[i] * (xr[i] * inv), hi, lo);
-        out16[int64_t(blockIdx.x) * ldo + i] = hi;
-        out16[lo_off + int64_t(blockIdx.x) * ldo + i] = lo;
+        _Float16 *o = out16 + plane_off(int64_t(blockIdx.x), i, K);
+        o[0] = hi;
+        o[kPlaneLo] = lo;
     }
     raise_status(status, bad, kStatusF16Range);
-}
-
-// int8 weight values widened to f16 (exact: |q| <= 127), 8 per thread; n a multiple of 8.
-__global__ __launch_bounds__(256) void k_q8_to_f16(const int8_t *q, _Float16 *out, int64_t n) {
-    const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 8;
-    if (i >= n) return;
-    const uint2 u = *reinterpret_cast<const uint2 *>(q + i);
-    _Float16 h[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) h[e] = _Float16(int8_t((e < 4 ? u.x : u.y) >> (8 * (e & 3))));
-    *reinterpret_cast<uint4 *>(out + i) = *reinterpret_cast<const uint4 *>(h);
 }
 
 // Synthetic N(mean, std) data: Philox4x32-10 counter (pair p, stream, draw 0/1) under key (seed), Box-Muller.

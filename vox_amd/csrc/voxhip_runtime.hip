@@ -70,7 +70,10 @@ struct GpuMat {
     bool s16 = false;
     float *b = nullptr;
     uint64_t bytes = 0;  // weights + scales + bias bytes (the GEMV's algorithmic stream)
-    _Float16 *w16 = nullptr;  // Q8: the int8 values widened to f16 for the split-f16 GEMM, made on first use
+    // F16 and Q8: the weights (the int8 values as f16) in the order k_gemm_hh reads them, and Q8's block scales
+    // transposed; made before a planes pass first uses them
+    _Float16 *w16 = nullptr;
+    float *st = nullptr;
     float wmax = 0.f;  // F32: max |w| (NaN when a weight is NaN), which picks the GEMM kernel (f32_wide)
     void *wx = nullptr;  // F32: the weights laid out for k_gemm_x3p, made by the first user that multiplies rows with them
 };
@@ -123,8 +126,8 @@ struct Xfmr {
     // scratch for cap_rows rows (grown by ensure_rows); pre: the GEMM path's prologue output (normed or merged rows)
     int cap_rows = 0;
     float *h = nullptr, *xin = nullptr, *qkv = nullptr, *q = nullptr, *g = nullptr, *xnorm = nullptr, *pre = nullptr;
-    // f16 halves (hi plane, then lo plane) of the GEMM inputs of a planes pass: pa16 the normed rows and the attention
-    // output (planes of cap_rows x max(H, qd)), pb16 the SwiGLU output (planes of cap_rows x I)
+    // f16 planes (plane_off's layout) of the GEMM inputs of a planes pass: pa16 the normed rows and the attention
+    // output (cap_rows x max(H, qd)), pb16 the SwiGLU output (cap_rows x I)
     _Float16 *pa16 = nullptr, *pb16 = nullptr;
     float *pm = nullptr, *pl = nullptr, *po = nullptr, *logits = nullptr;
     int64_t xin_elems = 0, logits_elems = 0;
@@ -433,7 +436,7 @@ int new_mat(int32_t type, int64_t rows, int64_t cols, bool bias, bool s16 = fals
 void free_mat(int id) {
     if (id < 0 || size_t(id) >= g.mats.size()) return;
     GpuMat &m = g.mats[size_t(id)];
-    dfree(m.w); dfree(m.s); dfree(m.b); dfree(m.w16); dfree(m.wx);
+    dfree(m.w); dfree(m.s); dfree(m.b); dfree(m.w16); dfree(m.st); dfree(m.wx);
     m = GpuMat();
 }
 
@@ -704,8 +707,8 @@ void ensure_rows(Xfmr &X, int rows) {
     X.g = dalloc_t<float>(M * X.I);
     X.xnorm = dalloc_t<float>(M * X.H);
     X.pre = dalloc_t<float>(M * std::max<size_t>(size_t(X.H), qd));
-    X.pa16 = dalloc_t<_Float16>(2 * M * std::max<size_t>(size_t(X.H), qd));
-    X.pb16 = dalloc_t<_Float16>(2 * M * size_t(X.I));
+    X.pa16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(M), std::max<int64_t>(X.H, int64_t(qd)))));
+    X.pb16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(M), X.I)));
     X.pm = dalloc_t<float>(M * X.heads * kAttnMaxSplits);
     X.pl = dalloc_t<float>(M * X.heads * kAttnMaxSplits);
     X.po = dalloc_t<float>(M * X.heads * kAttnMaxSplits * X.hd);
@@ -811,34 +814,41 @@ bool planes_layer(const Xfmr &X, int li, int64_t m_total, int mc, bool need_read
     const LayerDev &L = X.L[size_t(li)];
     for (int id : {L.qkv, L.o, L.gu, L.down}) {
         const GpuMat &m = g.mats[size_t(id)];
-        if (!planes_mat(m, m_total, mc) || (need_ready && m.type == VOXHIP_Q8 && !m.w16)) return false;
+        if (!planes_mat(m, m_total, mc) || (need_ready && !m.w16)) return false;
     }
     return true;
 }
-// The f16 weights of a planes GEMM: F16 as stored; Q8's int8 values widened into m.w16 on first use (outside any
-// graph capture: forward_rows prepares them before its passes).
-const _Float16 *planes_weights(GpuMat &m, hipStream_t s) {
-    if (m.type == VOXHIP_F16) return reinterpret_cast<const _Float16 *>(m.w);
-    if (!m.w16) {
-        _Float16 *w16 = dalloc_t<_Float16>(size_t(m.rows) * size_t(m.cols));
-        HIPCHECK(launch_q8_to_f16(reinterpret_cast<const int8_t *>(m.w), w16, m.rows * m.cols, s));
-        m.w16 = w16;
+// The weights of a planes GEMM (F16, Q8) laid out for k_gemm_hh, on first use (outside any graph capture: forward_rows
+// and the F5 / estimator creates prepare them). They are an optimisation: when they cannot be allocated (VRAM limit or
+// device memory), m.w16 stays null and the passes over this matrix take the f32-activation GEMM.
+void prepare_w16(GpuMat &m, hipStream_t s) {
+    if (m.w16) return;
+    const bool q8 = m.type == VOXHIP_Q8;
+    _Float16 *w16 = nullptr;
+    float *st = nullptr;
+    try {
+        w16 = dalloc_t<_Float16>(size_t(pack_f16_halves(m.rows, m.cols)));
+        if (q8) st = dalloc_t<float>(size_t(scale_t_floats(m.rows, m.cols)));
+    } catch (const Fail &) {
+        (void)hipGetLastError();  // a failed hipMalloc leaves its error for the next query
+        dfree(w16);
+        return;
     }
-    return m.w16;
+    hipError_t e = launch_pack_f16(m.w, q8, m.rows, m.cols, w16, s);
+    if (e == hipSuccess && q8) e = launch_scale_t(m.s, m.rows, m.cols, st, s);
+    if (e != hipSuccess) {
+        dfree(w16);
+        dfree(st);
+        HIPCHECK(e);
+    }
+    m.w16 = w16;
+    m.st = st;
 }
-// The widened copies are an optimisation: when one cannot be allocated (VRAM limit or device memory), its matrix keeps
-// m.w16 null, planes_layer(need_ready) then sends that layer to the f32-activation GEMM, and the pass still runs.
 void prepare_planes(Xfmr &X, int first, int count, int64_t m_total, int mc, hipStream_t s) {
     for (int li = first; li < first + count; ++li)
         if (planes_layer(X, li, m_total, mc, false)) {
             const LayerDev &L = X.L[size_t(li)];
-            for (int id : {L.qkv, L.o, L.gu, L.down}) {
-                try {
-                    (void)planes_weights(g.mats[size_t(id)], s);
-                } catch (const Fail &) {
-                    (void)hipGetLastError();  // a failed hipMalloc leaves its error for the next query
-                }
-            }
+            for (int id : {L.qkv, L.o, L.gu, L.down}) prepare_w16(g.mats[size_t(id)], s);
         }
 }
 
@@ -861,28 +871,24 @@ void enqueue_layers(Xfmr &X, int mc, int64_t m_total, int first, int count, hipS
         const GpuMat &Mqkv = g.mats[size_t(L.qkv)], &Mo = g.mats[size_t(L.o)], &Mgu = g.mats[size_t(L.gu)],
                      &Md = g.mats[size_t(L.down)];
         const float *qn = L.qk ? X.norms + L.qn : nullptr, *kn = L.qk ? X.norms + L.kn : nullptr;
-        // planes pass: GEMM inputs as f16 halves, hi plane then lo plane PA (PB) halves on
+        // planes pass: GEMM inputs as f16 planes
         const bool planes = pass_attn && !rows_attn && planes_layer(X, li, m_total, mc, true);
-        const int64_t PA = int64_t(X.cap_rows) * std::max<int64_t>(X.H, qd), PB = int64_t(X.cap_rows) * X.I;
-        auto hh_args = [&](const GpuMat &M, const _Float16 *a16, int64_t a_lo, float *y, int64_t ldy) {
+        auto hh_args = [&](const GpuMat &M, const _Float16 *a16, float *y, int64_t ldy) {
             const PassScratch sc = lib_scratch();
             GemmArgs ga{};
             ga.bias = M.b; ga.y = y; ga.ldy = ldy; ga.m = mc; ga.n = int32_t(M.rows); ga.K = int32_t(M.cols);
-            ga.a16 = a16; ga.a_lo = a_lo; ga.lda = M.cols; ga.ws = sc.ws; ga.ws_cap = sc.ws_cap;
+            ga.a16 = a16; ga.ws = sc.ws; ga.ws_cap = sc.ws_cap;
             return ga;
         };
-        auto w16_of = [](const GpuMat &M) {
-            return M.type == VOXHIP_F16 ? reinterpret_cast<const _Float16 *>(M.w) : static_cast<const _Float16 *>(M.w16);
-        };
-        auto hh = [&](const GpuMat &M, int epi, const _Float16 *a16, int64_t a_lo, float *y, int64_t ldy) {
-            GemmArgs ga = hh_args(M, a16, a_lo, y, ldy);
-            if (epi == EPI_SWIGLU_H16) { ga.y = nullptr; ga.h16 = X.pb16; ga.lo_off = PB; }
-            HIPCHECK(launch_gemm_hh(epi, w16_of(M), M.type == VOXHIP_Q8 ? M.s : nullptr, ga, s));
+        auto hh = [&](const GpuMat &M, int epi, const _Float16 *a16, float *y, int64_t ldy) {
+            GemmArgs ga = hh_args(M, a16, y, ldy);
+            if (epi == EPI_SWIGLU_H16) ga.h16 = X.pb16;
+            HIPCHECK(launch_gemm_hh(epi, M.w16, M.st, ga, s));
         };
         probed(pr, VOXHIP_K_QKV, [&] {
             if (planes) {
-                if (!pa_normed) HIPCHECK(launch_rmsnorm_rows_h16(X.h, X.H, X.norms + L.ln1, int(X.H), X.eps, X.pa16, X.H, PA, mc, s));
-                hh(Mqkv, EPI_STORE, X.pa16, PA, X.qkv, ldqkv);
+                if (!pa_normed) HIPCHECK(launch_rmsnorm_rows_h16(X.h, X.H, X.norms + L.ln1, int(X.H), X.eps, X.pa16, mc, s));
+                hh(Mqkv, EPI_STORE, X.pa16, X.qkv, ldqkv);
             } else {
                 gemv(Mqkv, m_total, PRO_RMS, EPI_STORE, direct && li == first ? x0 : X.h, X.H, mc, X.qkv, ldqkv, X.norms + L.ln1, X.eps,
                      nullptr, s, nullptr, X.pre, nullptr, acc_live ? X.acc : nullptr);
@@ -906,11 +912,11 @@ void enqueue_layers(Xfmr &X, int mc, int64_t m_total, int first, int count, hipS
             pa.q = X.q; pa.k = r0.k; pa.v = r0.v; pa.out = X.pre; pa.rows = X.rows_dev; pa.cap = r0.cap; pa.pos0 = r0.pos;
             pa.m = mc;
             pa.heads = X.heads; pa.kv_heads = X.kvh; pa.layer = li; pa.scale = 1.0f / std::sqrt(float(X.hd));
-            if (planes) { pa.out16 = X.pa16; pa.lo_off = PA; }
+            if (planes) pa.out16 = X.pa16;
             pa.part = part;  // key-split runs (the partial buffers hold cap_rows rows)
             probed(pr, VOXHIP_K_ATTN, [&] { HIPCHECK(launch_prefill_attn(pa, X.hd, s)); });
             probed(pr, VOXHIP_K_O, [&] {
-                if (planes) hh(Mo, EPI_ACC, X.pa16, PA, X.h, X.H);
+                if (planes) hh(Mo, EPI_ACC, X.pa16, X.h, X.H);
                 else gemv(Mo, m_total, PRO_X, EPI_ACC, X.pre, qd, mc, X.h, X.H, nullptr, 0.f, nullptr, s);
             });
         } else {
@@ -941,8 +947,8 @@ void enqueue_layers(Xfmr &X, int mc, int64_t m_total, int first, int count, hipS
         const bool gq_on = !planes && ffn_quant_epilogue(Mgu, Md, m_total, mc, lib_scratch(), &gq);
         probed(pr, VOXHIP_K_GATEUP, [&] {
             if (planes) {
-                HIPCHECK(launch_rmsnorm_rows_h16(X.h, X.H, X.norms + L.ln2, int(X.H), X.eps, X.pa16, X.H, PA, mc, s));
-                hh(Mgu, EPI_SWIGLU_H16, X.pa16, PA, nullptr, X.I);
+                HIPCHECK(launch_rmsnorm_rows_h16(X.h, X.H, X.norms + L.ln2, int(X.H), X.eps, X.pa16, mc, s));
+                hh(Mgu, EPI_SWIGLU_H16, X.pa16, nullptr, X.I);
             } else {
                 gemv(Mgu, m_total, PRO_RMS, EPI_SWIGLU, X.h, X.H, mc, X.g, X.I, X.norms + L.ln2, X.eps, nullptr, s, nullptr, X.pre,
                      nullptr, nullptr, nullptr, nullptr, gq_on ? &gq : nullptr);
@@ -952,11 +958,10 @@ void enqueue_layers(Xfmr &X, int mc, int64_t m_total, int first, int count, hipS
         probed(pr, VOXHIP_K_DOWN, [&] {
             // the next layer's first RMSNorm rides on this split-K reduce when that layer is a planes pass too
             if (planes && li + 1 < first + count && planes_layer(X, li + 1, m_total, mc, true)) {
-                const GemmArgs ga = hh_args(Md, X.pb16, PB, X.h, X.H);
-                HIPCHECK(launch_gemm_hh_acc_rms(w16_of(Md), Md.type == VOXHIP_Q8 ? Md.s : nullptr, ga,
-                                                X.norms + X.L[size_t(li + 1)].ln1, X.eps, X.pa16, X.H, PA, s, &pa_normed));
+                const GemmArgs ga = hh_args(Md, X.pb16, X.h, X.H);
+                HIPCHECK(launch_gemm_hh_acc_rms(Md.w16, Md.st, ga, X.norms + X.L[size_t(li + 1)].ln1, X.eps, X.pa16, s, &pa_normed));
             } else if (planes) {
-                hh(Md, EPI_ACC, X.pb16, PB, X.h, X.H);
+                hh(Md, EPI_ACC, X.pb16, X.h, X.H);
             } else {
                 gemv(Md, m_total, PRO_X, EPI_ACC, X.g, X.I, mc, X.h, X.H, nullptr, 0.f, nullptr, s, nullptr, nullptr, nullptr,
                      nullptr, nullptr, nullptr, nullptr, gq_on ? &gq : nullptr);
@@ -2277,7 +2282,7 @@ struct F5 {
     _Float16 *qkv16 = nullptr;
     int64_t lo_off = 0;
     int ldvt = 0;
-    // split: the modulated rows, the attention output and the GELU output as hi / lo planes ([R][width] each)
+    // split: the modulated rows, the attention output and the GELU output as f16 planes (R rows each)
     _Float16 *nrm16 = nullptr, *at16 = nullptr, *ffb16 = nullptr;
 };
 
@@ -2471,14 +2476,11 @@ void f5_gemm(const GpuMat &m, int epi, const float *A, GemmArgs ga, hipStream_t 
     if (int_path(m, ga.m)) throw Fail("DiT / flow estimator linears need f32 / f16 / bf16 weights, or q8 with more than 8 rows");
     HIPCHECK(launch_gemm(gemv_type(m), epi, m.w, m.s, A, ga, s));
 }
-// A block linear: from the f16 planes of A (width ga.K, lo plane R ga.K halves on) when the model is split,
-// else from the f32 rows A.
+// A block linear: from the f16 planes of A (width ga.K) when the model is split, else from the f32 rows A.
 void split_lin(bool split, const GpuMat &m, int epi, const float *A, const _Float16 *A16, GemmArgs ga, hipStream_t s) {
     if (!split) return f5_gemm(m, epi, A, ga, s);
     ga.a16 = A16;
-    ga.a_lo = int64_t(ga.m) * ga.K;
-    ga.lda = ga.K;
-    HIPCHECK(launch_gemm_hh(epi, reinterpret_cast<const _Float16 *>(m.w), nullptr, ga, s));
+    HIPCHECK(launch_gemm_hh(epi, m.w16, nullptr, ga, s));
 }
 void f5_lin(const F5 &F, const GpuMat &m, int epi, const float *A, const _Float16 *A16, GemmArgs ga, hipStream_t s) {
     split_lin(F.split, m, epi, A, A16, ga, s);
@@ -2516,28 +2518,29 @@ void f5_enqueue(F5 &F, hipStream_t s) {
         const F5Block &L = F.blocks[size_t(i)];
         const float *ada = F.ada + size_t(i) * 6 * D;  // shift, scale, gate (msa), shift, scale, gate (mlp)
         float *nrm = F.split ? nullptr : F.nrm;
-        HIPCHECK(launch_f5_modulate(F.h, R, D, ada + D, ada, nrm, F.nrm16, R * D, s));
+        HIPCHECK(launch_f5_modulate(F.h, R, D, ada + D, ada, nrm, F.nrm16, s));
         const GpuMat &Mq = mat_at(L.qkv);
         GemmArgs gq = gemm_args(Mq, Mq.b, nullptr, D, 3 * INNER, R);
         gq.rope = F.rope; gq.seq = F.N; gq.hd = F.hp; gq.rope_hd = F.hd; gq.rope_cols = 2 * INNER; gq.rope_heads = F.pe;
         gq.h16 = F.qkv16; gq.lo_off = F.lo_off; gq.ldvt = F.ldvt;
         f5_lin(F, Mq, EPI_ROPE_H16, F.nrm, F.nrm16, gq, s);
-        HIPCHECK(launch_f5_attn(F.qkv16, F.lo_off, F.split ? nullptr : F.at, F.at16, R * INNER, F.B, F.N, F.heads, F.hp,
+        HIPCHECK(launch_f5_attn(F.qkv16, F.lo_off, F.split ? nullptr : F.at, F.at16, F.B, F.N, F.heads, F.hp,
                                 F.ldvt, INNER, scale, s));
         const GpuMat &Mo = mat_at(L.o);
         GemmArgs go = gemm_args(Mo, Mo.b, F.h, INNER, D, R);
         go.gate = ada + 2 * D;
         f5_lin(F, Mo, EPI_GATED_ACC, F.at, F.at16, go, s);
-        HIPCHECK(launch_f5_modulate(F.h, R, D, ada + 4 * D, ada + 3 * D, nrm, F.nrm16, R * D, s));
+        HIPCHECK(launch_f5_modulate(F.h, R, D, ada + 4 * D, ada + 3 * D, nrm, F.nrm16, s));
         const GpuMat &M1 = mat_at(L.ff1), &M2 = mat_at(L.ff2);
         GemmArgs g1 = gemm_args(M1, M1.b, F.split ? nullptr : F.ffb, D, F.ff, R);
-        g1.h16 = F.ffb16; g1.lo_off = R * F.ff;
+        g1.h16 = F.ffb16;
+        if (F.split) g1.ldy = F.ff;
         f5_lin(F, M1, F.split ? EPI_GELU_H16 : EPI_GELU, F.nrm, F.nrm16, g1, s);
         GemmArgs g2 = gemm_args(M2, M2.b, F.h, F.ff, D, R);
         g2.gate = ada + 5 * D;
         f5_lin(F, M2, EPI_GATED_ACC, F.ffb, F.ffb16, g2, s);
     }
-    HIPCHECK(launch_f5_modulate(F.h, R, D, F.fin, F.fin + D, F.nrm, nullptr, 0, s));  // final modulation: (scale, shift)
+    HIPCHECK(launch_f5_modulate(F.h, R, D, F.fin, F.fin + D, F.nrm, nullptr, s));  // final modulation: (scale, shift)
     const GpuMat &Mp = mat_at(F.proj_out);
     f5_gemm(Mp, EPI_STORE, F.nrm, gemm_args(Mp, Mp.b, F.out, D, F.mel, R), s);
 }
@@ -2587,6 +2590,12 @@ int voxhip_f5_create(const voxhip_f5_desc *d) {
         F->split = D % 64 == 0 && FF % 64 == 0;  // the attention width (heads x 64) always is
         for (const F5Block &fb : F->blocks)
             for (int id : {fb.qkv, fb.o, fb.ff1, fb.ff2}) F->split = F->split && mat_at(id).type == VOXHIP_F16;
+        if (F->split)
+            for (const F5Block &fb : F->blocks)
+                for (int id : {fb.qkv, fb.o, fb.ff1, fb.ff2}) {
+                    prepare_w16(mat_at(id), g.stream);
+                    F->split = F->split && mat_at(id).w16;
+                }
         F->pos1 = upload_conv(d->pos1, D);
         F->pos2 = upload_conv(d->pos2, D);
         if (d->vocos_dim > 0) {  // Vocos (f5.cpp:333-346): the linears are matrix handles, the rest host arrays
@@ -2635,9 +2644,9 @@ int voxhip_f5_begin(int id, int B, int N, const float *cat0, const float *rope) 
         F.cat = dalloc_t<float>(R * W); F.h = dalloc_t<float>(R * D); F.a = dalloc_t<float>(R * D);
         F.nrm = dalloc_t<float>(R * D);
         if (F.split) {
-            F.nrm16 = dalloc_t<_Float16>(2 * R * D);
-            F.at16 = dalloc_t<_Float16>(2 * R * INNER);
-            F.ffb16 = dalloc_t<_Float16>(2 * R * size_t(F.ff));
+            F.nrm16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(D))));
+            F.at16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(INNER))));
+            F.ffb16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), F.ff)));
         } else {
             F.at = dalloc_t<float>(R * INNER);
             F.ffb = dalloc_t<float>(R * size_t(F.ff));
@@ -2843,7 +2852,7 @@ void cosy_conv(const Cosy &E, const F5Conv &cv, int epi, const float *X, int64_t
 void cosy_norm(const Cosy &E, const float *x, const float *w, const float *b, bool mish, const float *tb, float *y,
                _Float16 *y16, hipStream_t s) {
     NormArgs a{};
-    a.x = x; a.y = y; a.y16 = y16; a.lo_off = int64_t(2) * E.T * E.C; a.sc = w; a.sh = b; a.tb = tb;
+    a.x = x; a.y = y; a.y16 = y16; a.sc = w; a.sh = b; a.tb = tb;
     a.eps = double(1e-5f); a.R = 2 * E.T; a.D = E.C; a.affine = 1; a.mish = mish;
     HIPCHECK(launch_norm_rows(a, s));
 }
@@ -2871,14 +2880,14 @@ void cosy_xblock(const Cosy &E, const CosyX &L, float *A, hipStream_t s) {
     gq.rope = nullptr; gq.seq = E.T; gq.hd = kF5HeadDim; gq.rope_cols = 2 * INNER;
     gq.h16 = E.qkv16; gq.lo_off = E.lo_off; gq.ldvt = E.ldvt;
     split_lin(E.split, Mq, EPI_ROPE_H16, E.xn, E.xn16, gq, s);
-    HIPCHECK(launch_f5_attn(E.qkv16, E.lo_off, E.split ? nullptr : E.at, E.at16, R * INNER, 2, E.T, E.heads, kF5HeadDim,
+    HIPCHECK(launch_f5_attn(E.qkv16, E.lo_off, E.split ? nullptr : E.at, E.at16, 2, E.T, E.heads, kF5HeadDim,
                             E.ldvt, INNER, 1.0f / std::sqrt(float(E.hd)), s));
     const GpuMat &Mo = mat_at(L.o);
     split_lin(E.split, Mo, EPI_ACC, E.at, E.at16, gemm_args(Mo, Mo.b, A, INNER, C, R), s);
     cosy_norm(E, A, L.n3w, L.n3b, false, nullptr, xn, E.xn16, s);
     const GpuMat &M1 = mat_at(L.ff1), &M2 = mat_at(L.ff2);
     GemmArgs g1 = gemm_args(M1, M1.b, E.split ? nullptr : E.ff, C, L.ff, R);
-    g1.h16 = E.ff16; g1.lo_off = R * L.ff; g1.gelu_erf = 1;
+    g1.h16 = E.ff16; g1.gelu_erf = 1;
     split_lin(E.split, M1, E.split ? EPI_GELU_H16 : EPI_GELU_ERF, E.xn, E.xn16, g1, s);
     split_lin(E.split, M2, EPI_ACC, E.ff, E.ff16, gemm_args(M2, M2.b, A, L.ff, C, R), s);
 }
@@ -2963,6 +2972,17 @@ int voxhip_cosy_create(const voxhip_cosy_desc *d) {
         };
         split = split && all_f16(E->down_x) && all_f16(E->up_x);
         for (const auto &v : E->mid_x) split = split && all_f16(v);
+        auto prepare = [&](const std::vector<CosyX> &v) {
+            for (const CosyX &x : v)
+                for (int id : {x.qkv, x.o, x.ff1, x.ff2})
+                    if (split) {
+                        prepare_w16(mat_at(id), g.stream);
+                        split = split && mat_at(id).w16;
+                    }
+        };
+        prepare(E->down_x);
+        prepare(E->up_x);
+        for (const auto &v : E->mid_x) prepare(v);
         E->split = split;
         g.cosy.push_back(E.release());
         return int(g.cosy.size()) - 1;
@@ -2982,9 +3002,9 @@ int voxhip_cosy_begin(int id, int T, const float *in0) {
         E.a = dalloc_t<float>(R * C); E.b = dalloc_t<float>(R * C); E.h = dalloc_t<float>(R * C);
         E.cat = dalloc_t<float>(R * 2 * C);
         if (E.split) {
-            E.xn16 = dalloc_t<_Float16>(2 * R * C);
-            E.at16 = dalloc_t<_Float16>(2 * R * INNER);
-            E.ff16 = dalloc_t<_Float16>(2 * R * FF);
+            E.xn16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(C))));
+            E.at16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(INNER))));
+            E.ff16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(FF))));
         } else {
             E.xn = dalloc_t<float>(R * C);
             E.at = dalloc_t<float>(R * INNER);
@@ -4067,52 +4087,56 @@ int voxhip_bench_gemm_hh(int64_t m, int64_t n, int64_t K, int q8, int tile, int 
             throw Fail("bad bench arguments");
         if (m > (int64_t(1) << 20) || n > (int64_t(1) << 20) || m * K > (int64_t(1) << 28) || n * K > (int64_t(1) << 28))
             throw Fail("bench_gemm_hh: shape too large");
-        _Float16 *a16 = nullptr, *w16 = nullptr;
-        float *tmp = nullptr, *sc = nullptr, *y = nullptr;
+        _Float16 *a16 = nullptr, *planes = nullptr, *w16 = nullptr, *pack = nullptr;
+        float *tmp = nullptr, *sc = nullptr, *st = nullptr, *y = nullptr;
         int8_t *q = nullptr;
         hipEvent_t e0 = nullptr, e1 = nullptr;
         auto cleanup = [&] {
             (void)hipStreamSynchronize(g.stream);
             vh::set_gemm_hh_tile(0);
-            dfree(a16); dfree(w16); dfree(tmp); dfree(sc); dfree(y); dfree(q);
+            dfree(a16); dfree(planes); dfree(w16); dfree(pack); dfree(tmp); dfree(sc); dfree(st); dfree(y); dfree(q);
             if (e0) (void)hipEventDestroy(e0);
             if (e1) (void)hipEventDestroy(e1);
         };
         try {
             // A: hi plane ~N(0, 1) as f16, lo plane ~N(0, 1e-3) as f16; W: ~N(0, 0.02) as f16, or its q8 form (int8
-            // values as f16 and the block scales)
+            // values and the block scales), both laid out as the kernel reads them
             a16 = dalloc_t<_Float16>(size_t(2 * m * K));
-            w16 = dalloc_t<_Float16>(size_t(n * K));
+            planes = dalloc_t<_Float16>(size_t(planes_halves(m, K)));
+            pack = dalloc_t<_Float16>(size_t(pack_f16_halves(n, K)));
             tmp = dalloc_t<float>(size_t(std::max(m, n) * K));
             y = dalloc_t<float>(size_t(m * n));
             HIPCHECK(launch_fill_normal(tmp, m * K, 11, 0x90u, 0.f, 1.f, g.stream));
             HIPCHECK(launch_to_f16(tmp, m * K, a16, g.stream));
             HIPCHECK(launch_fill_normal(tmp, m * K, 12, 0x91u, 0.f, 1e-3f, g.stream));
             HIPCHECK(launch_to_f16(tmp, m * K, a16 + m * K, g.stream));
+            HIPCHECK(launch_pack_planes(a16, a16 + m * K, m, K, planes, g.stream));
             HIPCHECK(launch_fill_normal(tmp, n * K, 13, 0x92u, 0.f, 0.02f, g.stream));
             if (q8) {
                 q = dalloc_t<int8_t>(size_t(n * K));
                 sc = dalloc_t<float>(size_t(n * K / 32));
+                st = dalloc_t<float>(size_t(scale_t_floats(n, K)));
                 HIPCHECK(launch_quant_q8(tmp, n * K / 32, q, sc, g.stream));
-                HIPCHECK(launch_q8_to_f16(q, w16, n * K, g.stream));
+                HIPCHECK(launch_pack_f16(reinterpret_cast<const uint8_t *>(q), true, n, K, pack, g.stream));
+                HIPCHECK(launch_scale_t(sc, n, K, st, g.stream));
             } else {
+                w16 = dalloc_t<_Float16>(size_t(n * K));
                 HIPCHECK(launch_to_f16(tmp, n * K, w16, g.stream));
+                HIPCHECK(launch_pack_f16(reinterpret_cast<const uint8_t *>(w16), false, n, K, pack, g.stream));
             }
             GemmArgs ga{};
             ga.m = int32_t(m);
             ga.n = int32_t(n);
             ga.K = int32_t(K);
-            ga.a16 = a16;
-            ga.a_lo = m * K;
-            ga.lda = int32_t(K);
+            ga.a16 = planes;
             ga.y = y;
             ga.ldy = int32_t(n);
             vh::set_gemm_hh_tile(tile);
-            for (int i = 0; i < warmup; ++i) HIPCHECK(launch_gemm_hh(EPI_STORE, w16, sc, ga, g.stream));
+            for (int i = 0; i < warmup; ++i) HIPCHECK(launch_gemm_hh(EPI_STORE, pack, st, ga, g.stream));
             HIPCHECK(hipEventCreate(&e0));
             HIPCHECK(hipEventCreate(&e1));
             HIPCHECK(hipEventRecord(e0, g.stream));
-            for (int i = 0; i < iters; ++i) HIPCHECK(launch_gemm_hh(EPI_STORE, w16, sc, ga, g.stream));
+            for (int i = 0; i < iters; ++i) HIPCHECK(launch_gemm_hh(EPI_STORE, pack, st, ga, g.stream));
             HIPCHECK(hipEventRecord(e1, g.stream));
             HIPCHECK(hipEventSynchronize(e1));
             float ms = 0.f;
