@@ -10,6 +10,17 @@ hipError_t launch_norm_rows(const NormArgs &a0, hipStream_t s) {
     if (a.R <= 0) return hipSuccess;
     if (a.D <= 0 || a.D % 4 || !a.x || (!a.y && !a.y16) || (a.y16 && a.D % 32) || !a.sc || (!a.affine && !a.sh) || !(a.eps > 0.0))
         return hipErrorInvalidValue;
+    // Rows of 256, 512, 768 and 1024 take k_norm_rows, a row per wave where its width allows (1000 x 1024 planes 3.7 us, two
+    // rows per wave 4.2), except many planes rows, where half-waves' runs of 32 bytes per plane matter more (2000 x 1024:
+    // 4.9 against 5.5).
+    auto rows = [&](auto kernel, int lanes) { return launch(kernel, dim3(unsigned((a.R + 256 / lanes - 1) / (256 / lanes))), dim3(256), 0, s, a); };
+    switch (a.D) {
+        case 256: return rows(k_norm_rows<32, 1>, 32);
+        case 512: return rows(k_norm_rows<64, 1>, 64);
+        case 768: return rows(k_norm_rows<32, 3>, 32);
+        case 1024: return a.y16 && a.R >= 1536 ? rows(k_norm_rows<32, 4>, 32) : rows(k_norm_rows<64, 2>, 64);
+        default: break;
+    }
     if (a.D <= 4 * 256) return launch(k_f5_modulate<4, true>, dim3(unsigned((a.R + 3) / 4)), dim3(256), 0, s, a);
     return launch(k_f5_modulate<kNormRegChunks, false>, dim3(unsigned((a.R + 3) / 4)), dim3(256), 0, s, a);
 }

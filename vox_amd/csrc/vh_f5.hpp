@@ -17,7 +17,7 @@ VH_DEV float mish_nn_f(float x) {
     return x * (n / (n + 2.0f));
 }
 
-// Row LayerNorm (NormArgs), one wave per row (4 rows per 256-thread block): mean and variance in double (two passes
+// Row LayerNorm (NormArgs) of any D, one wave per row (4 rows per 256-thread block): mean and variance in double (two passes
 // over the row, which stays in L1), inv = float(1 / sqrt(var + eps)). The forms: AdaLN modulation without
 // parameters (f5.cpp:608-625, eps 1e-6), y = (x - float(mean)) * inv * (1 + scale) + shift; LayerNorm with weight
 // and bias (kernels.cpp:714-723 and nn.cpp:248-265, which compute alike), y = (x - float(mean)) * inv * w + b; then
@@ -132,6 +132,112 @@ __global__ __launch_bounds__(256) void k_f5_modulate(NormArgs a) {
         else emit_load(4 * lane + 256 * c, reg[c]);
     }
     for (int i = tail0 + 4 * lane; i < D; i += 256) emit_load(i, *reinterpret_cast<const f32x4a *>(xr + i));
+}
+
+// k_f5_modulate for rows of 8 L C values: L lanes per row (64 / L rows per wave), 8 neighbouring columns of a lane at a
+// time (a lane's 8 halves of a plane are one store), the parameters loaded with the row. Both moments are summed in one
+// pass over x minus the row's first value (a difference of floats: rounded at 2^-53, and a row far from zero or constant
+// cancels nothing), their sums by DPP and row swaps. Bound by the round trip to rows another XCD wrote, and the launch; the
+// two reductions of k_f5_modulate through LDS were a second round trip. Launches back to back, k_f5_modulate -> here (us):
+// f32 rows 1024 x 256 2.9 -> 2.1, 938 x 512 3.0 -> 2.4, 2000 x 1024 4.8 -> 4.3; planes 1024 x 256 3.0 -> 2.4, 333 x 1024
+// 3.7 -> 2.9, 2000 x 1024 6.1 -> 4.9. The outputs are the same bits there.
+template <int CTRL>
+VH_DEV double dpp_add(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = uint32_t(dpp<CTRL>(int(uint32_t(u)))), hi = uint32_t(dpp<CTRL>(int(uint32_t(u >> 32))));
+    return v + __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+}
+// v summed over groups of L lanes (16, 32, 64), the same bits in every lane of a group.
+template <int L>
+VH_DEV double lanes_sum(double v) {
+    v = dpp_add<kDppXor1>(v);
+    v = dpp_add<kDppXor2>(v);
+    v = dpp_add<kDppRowHalfMirror>(v);
+    v = dpp_add<kDppRowMirror>(v);
+    auto swap_add = [&](auto sw) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const auto l = sw(uint32_t(u)), h = sw(uint32_t(u >> 32));
+        v = __builtin_bit_cast(double, uint64_t(h[0]) << 32 | l[0]) + __builtin_bit_cast(double, uint64_t(h[1]) << 32 | l[1]);
+    };
+    if (L >= 32) swap_add([](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
+    if (L >= 64) swap_add([](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
+    return v;
+}
+template <int L, int C>
+__global__ __launch_bounds__(256) void k_norm_rows(NormArgs a) {
+    constexpr int D = 8 * L * C, RB = 256 / L;
+    const int l = threadIdx.x % L, row = blockIdx.x * RB + threadIdx.x / L;
+    const float *xr = a.x + int64_t(min(row, a.R - 1)) * D;
+    f32x4a v[C][2], cs[C][2], sh[C][2], tb[C][2];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) v[c][h] = *reinterpret_cast<const f32x4a *>(xr + 8 * L * c + 8 * l + 4 * h);
+    const float x0 = xr[0];
+    const float *shp = a.sh ? a.sh : a.sc, *tbp = a.tb ? a.tb : a.sc;  // never used when absent
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int i = 8 * L * c + 8 * l + 4 * h;
+            cs[c][h] = *reinterpret_cast<const f32x4a *>(a.sc + i);
+            sh[c][h] = *reinterpret_cast<const f32x4a *>(shp + i);
+            tb[c][h] = *reinterpret_cast<const f32x4a *>(tbp + i);
+        }
+    double s = 0.0, q = 0.0;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const double d = double(v[c][h][e]) - double(x0);
+                s += d;
+                q = __builtin_fma(d, d, q);
+            }
+    s = lanes_sum<L>(s) / D;
+    q = lanes_sum<L>(q) / D;
+    double var = q - s * s;
+    var = var < 0.0 ? 0.0 : var;  // rounding only; a NaN stays
+    const float inv = float(1.0 / sqrt(var + a.eps)), fm = float(double(x0) + s);
+    if (row >= a.R) return;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        float r[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float p = cs[c][e / 4][e % 4];
+            r[e] = (v[c][e / 4][e % 4] - fm) * inv * (a.affine ? p : 1.0f + p) + (a.sh ? sh[c][e / 4][e % 4] : 0.f);
+        }
+        if (a.mish) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) r[e] = mish_nn_f(r[e]);
+        }
+        if (a.tb) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) r[e] += tb[c][e / 4][e % 4];
+        }
+        const int i = 8 * L * c + 8 * l;
+        if (a.y16) {
+            f16x4a hi[2], lo[2];
+            bool bad = false;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                _Float16 h, w;
+                bad |= split_f16(r[e], h, w);
+                hi[e / 4][e % 4] = h;
+                lo[e / 4][e % 4] = w;
+            }
+            raise_status(a.status, bad, kStatusF16Range);
+            _Float16 *o = a.y16 + plane_off(row, i, D);
+            *reinterpret_cast<u32x4 *>(o) = __builtin_bit_cast(u32x4, hi);
+            *reinterpret_cast<u32x4 *>(o + kPlaneLo) = __builtin_bit_cast(u32x4, lo);
+        } else {
+            float *o = a.y + int64_t(row) * D + i;
+            *reinterpret_cast<f32x4a *>(o) = f32x4a{r[0], r[1], r[2], r[3]};
+            *reinterpret_cast<f32x4a *>(o + 4) = f32x4a{r[4], r[5], r[6], r[7]};
+        }
+    }
 }
 
 // Depthwise "same" Conv1d (f5_ops.cpp:106-147 with groups = channels: the Vocos blocks' dwconv, f5.cpp:341) over

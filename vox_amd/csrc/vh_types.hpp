@@ -256,7 +256,7 @@ struct LmEmbedArgs {
     int32_t hd;
     int64_t spare_pos;
 };
-// Row LayerNorm of R rows of D (k_f5_modulate), one wave per row, double statistics:
+// Row LayerNorm of R rows of D (k_norm_rows, k_f5_modulate), double statistics:
 // n = (x - float(mean)) * float(1 / sqrt(var + eps)); modulate (affine 0): y = n * (1 + sc) + sh; affine:
 // y = n * sc + sh (sh null: 0); then mish (the nn.hpp form) when set, then + tb (null: none). y as f32 rows, or as
 // f16 planes of D columns (plane_off's layout) when y16 is set. x and y may be the same rows.
