@@ -73,6 +73,10 @@ hipError_t launch_pack_f16(const uint8_t *w, bool q8, int64_t n, int64_t K, _Flo
 int64_t scale_t_floats(int64_t n, int64_t K);
 hipError_t launch_scale_t(const float *sc, int64_t n, int64_t K, float *out, hipStream_t s);
 hipError_t launch_pack_planes(const _Float16 *hi, const _Float16 *lo, int64_t m, int64_t K, _Float16 *out, hipStream_t s);
+// The row-local part of a transformer block as one launch, where block_tail_ok (256 channels, inner and ff multiples of
+// 256 that fit LDS).
+bool block_tail_ok(int64_t R, int C, int inner, int ff);
+hipError_t launch_block_tail(const BlockTailArgs &a, hipStream_t s);
 // Forces launch_gemm_hh's block tile (0: its shape policy); voxhip_bench_gemm_hh only.
 void set_gemm_hh_tile(int tile);
 // The same with EPI_ACC, and when the product splits K, the next RMSNorm (gamma, eps) of the updated rows of y into planes

@@ -270,6 +270,18 @@ struct NormArgs {
     int32_t *status;  // the range-status word (y16 values beyond the f16 range); set by the launcher
 };
 
+// The row-local part of a 256-channel transformer block (k_block_tail).
+struct BlockTailArgs {
+    const _Float16 *a16, *wo, *w1, *w2;          // a16: planes of `inner` columns; weights [256][inner], [ff][256], [256][ff]
+    const float *bo, *b1, *b2;                   // may be null
+    const float *lw, *lb, *nw, *nb;              // the norm before the FFN; the next block's first (nw null: none)
+    float *x;                                    // [R][256]
+    _Float16 *out16;
+    double eps;
+    int32_t R, inner, ff;                        // inner and ff multiples of 256
+    int32_t *status;
+};
+
 // One pass of the code-predictor frame loop (gpu_pred_frame): the pass's m rows of the sequence at positions
 // pos0 .. pos0 + m - 1 (row table + RoPE rows), and for a pass after the first the embedding row of the code the
 // previous pass sampled (codes[code_idx]) into x.

@@ -2869,12 +2869,15 @@ void cosy_resnet(const Cosy &E, const CosyRes &r, int j, const float *X, int64_t
 }
 
 // BasicTransformerBlock (cosyvoice.cpp:182-221) on the rows A in place: LayerNorm -> q | k | v (no bias) -> full
-// attention per sequence -> to_out + residual -> LayerNorm -> ff.0 + GELU (erf) -> ff.2 + residual.
-void cosy_xblock(const Cosy &E, const CosyX &L, float *A, hipStream_t s) {
+// attention per sequence -> to_out + residual -> LayerNorm -> ff.0 + GELU (erf) -> ff.2 + residual. From to_out on, one
+// launch where the widths allow, which also does the first LayerNorm of the next block (`next`, may be null); normed: the
+// block before did this one's.
+void cosy_xblock(const Cosy &E, const CosyX &L, const CosyX *next, bool *normed, float *A, hipStream_t s) {
     const int C = E.C, INNER = E.inner;
     const int64_t R = int64_t(2) * E.T;
     float *xn = E.split ? nullptr : E.xn;
-    cosy_norm(E, A, L.n1w, L.n1b, false, nullptr, xn, E.xn16, s);
+    if (!*normed) cosy_norm(E, A, L.n1w, L.n1b, false, nullptr, xn, E.xn16, s);
+    *normed = false;
     const GpuMat &Mq = mat_at(L.qkv);
     GemmArgs gq = gemm_args(Mq, Mq.b, nullptr, C, 3 * INNER, R);
     gq.rope = nullptr; gq.seq = E.T; gq.hd = kF5HeadDim; gq.rope_cols = 2 * INNER;
@@ -2882,14 +2885,28 @@ void cosy_xblock(const Cosy &E, const CosyX &L, float *A, hipStream_t s) {
     split_lin(E.split, Mq, EPI_ROPE_H16, E.xn, E.xn16, gq, s);
     HIPCHECK(launch_f5_attn(E.qkv16, E.lo_off, E.split ? nullptr : E.at, E.at16, 2, E.T, E.heads, kF5HeadDim,
                             E.ldvt, INNER, 1.0f / std::sqrt(float(E.hd)), s));
-    const GpuMat &Mo = mat_at(L.o);
+    const GpuMat &Mo = mat_at(L.o), &M1 = mat_at(L.ff1), &M2 = mat_at(L.ff2);
+    if (E.split && block_tail_ok(R, C, INNER, L.ff)) {
+        BlockTailArgs t{};
+        t.a16 = E.at16; t.wo = Mo.w16; t.w1 = M1.w16; t.w2 = M2.w16;
+        t.bo = Mo.b; t.b1 = M1.b; t.b2 = M2.b; t.lw = L.n3w; t.lb = L.n3b;
+        if (next) { t.nw = next->n1w; t.nb = next->n1b; }
+        t.x = A; t.out16 = E.xn16; t.eps = double(1e-5f); t.R = int32_t(R); t.inner = INNER; t.ff = L.ff;
+        HIPCHECK(launch_block_tail(t, s));
+        *normed = next != nullptr;
+        return;
+    }
     split_lin(E.split, Mo, EPI_ACC, E.at, E.at16, gemm_args(Mo, Mo.b, A, INNER, C, R), s);
     cosy_norm(E, A, L.n3w, L.n3b, false, nullptr, xn, E.xn16, s);
-    const GpuMat &M1 = mat_at(L.ff1), &M2 = mat_at(L.ff2);
     GemmArgs g1 = gemm_args(M1, M1.b, E.split ? nullptr : E.ff, C, L.ff, R);
     g1.h16 = E.ff16; g1.gelu_erf = 1;
     split_lin(E.split, M1, E.split ? EPI_GELU_H16 : EPI_GELU_ERF, E.xn, E.xn16, g1, s);
     split_lin(E.split, M2, EPI_ACC, E.ff, E.ff16, gemm_args(M2, M2.b, A, L.ff, C, R), s);
+}
+
+void cosy_xblocks(const Cosy &E, const std::vector<CosyX> &v, float *A, hipStream_t s) {
+    bool normed = false;
+    for (size_t i = 0; i < v.size(); ++i) cosy_xblock(E, v[i], i + 1 < v.size() ? &v[i + 1] : nullptr, &normed, A, s);
 }
 
 // The estimator of one Euler step (cosyvoice.cpp:839-863; gpu_f5.cpp:490-547): x and the time biases already on
@@ -2899,19 +2916,19 @@ void cosy_enqueue(Cosy &E, hipStream_t s) {
     const int64_t R = int64_t(2) * E.T;
     HIPCHECK(launch_f5_fill_x(E.x, E.T, M, E.in, 4 * M, 2, s));
     cosy_resnet(E, E.down_res, 0, E.in, 4 * M, E.a, s);
-    for (const CosyX &L : E.down_x) cosy_xblock(E, L, E.a, s);
+    cosy_xblocks(E, E.down_x, E.a, s);
     // the skip half of the up block's input [x | skip]
     HIPCHECK(hipMemcpy2DAsync(E.cat + C, size_t(2 * C) * 4, E.a, size_t(C) * 4, size_t(C) * 4, size_t(R), hipMemcpyDeviceToDevice, s));
     cosy_conv(E, E.down_conv, EPI_STORE, E.a, C, E.b, C, s);
     float *cur = E.b, *oth = E.a;
     for (size_t i = 0; i < E.mid_res.size(); ++i) {
         cosy_resnet(E, E.mid_res[i], int(1 + i), cur, C, oth, s);
-        for (const CosyX &L : E.mid_x[i]) cosy_xblock(E, L, oth, s);
+        cosy_xblocks(E, E.mid_x[i], oth, s);
         std::swap(cur, oth);
     }
     HIPCHECK(hipMemcpy2DAsync(E.cat, size_t(2 * C) * 4, cur, size_t(C) * 4, size_t(C) * 4, size_t(R), hipMemcpyDeviceToDevice, s));
     cosy_resnet(E, E.up_res, int(1 + E.mid_res.size()), E.cat, 2 * C, oth, s);
-    for (const CosyX &L : E.up_x) cosy_xblock(E, L, oth, s);
+    cosy_xblocks(E, E.up_x, oth, s);
     cosy_conv(E, E.up_out, EPI_STORE, oth, C, cur, C, s);
     cosy_conv(E, E.final_conv, EPI_STORE, cur, C, oth, C, s);
     cosy_norm(E, oth, E.fn_w, E.fn_b, true, nullptr, oth, nullptr, s);
