@@ -42,6 +42,17 @@ constexpr int kPlaneLo = 512;
 VH_DEV int64_t plane_off(int64_t row, int k, int K) {
     return ((row >> 4) * (K >> 5) + (k >> 5)) * 1024 + ((((k >> 3) & 3) << 4) + (row & 15)) * 8 + (k & 7);
 }
+// q, k and v of an attention with heads of 64 dimensions as f16 halves in the order its MFMA operands are read, the lo half
+// kPlaneLo halves after the hi one: per section (q, k, v), batch and head, np rows (the sequence padded to 64). q, k:
+// [row / 16][d / 32][hi, lo][(d % 32) / 8 x 16 + row % 16][8]; v: [key / 32][d / 16][hi, lo][(key / 4) % 4 x 16 + d % 16][8]
+// where the 8 are keys 4 g .. 4 g + 3 and 16 + 4 g .. (the keys of P that lane group g holds). 64 keys of k, or of v, are
+// 16 KiB of consecutive bytes.
+constexpr int kQkvHead = 64;
+VH_DEV int64_t qkv_off(int sec, int b, int h, int n, int d, int B, int heads, int np) {
+    const int64_t base = ((int64_t(sec) * B + b) * heads + h) * np * (2 * kQkvHead);
+    if (sec < 2) return base + int64_t((n >> 4) * 2 + (d >> 5)) * 1024 + (((d >> 3) & 3) * 16 + (n & 15)) * 8 + (d & 7);
+    return base + int64_t((n >> 5) * 4 + (d >> 4)) * 1024 + (((n >> 2) & 3) * 16 + (d & 15)) * 8 + ((n >> 4) & 1) * 4 + (n & 3);
+}
 // Sets `bit` in the status word when `bad` (a vector atomic; the common path is one predicated branch).
 __device__ __forceinline__ void raise_status(int32_t *status, bool bad, int32_t bit) {
     if (__builtin_expect(bad, 0) && status) __hip_atomic_fetch_or(status, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -70,6 +81,29 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *base, int
 }
 __device__ __forceinline__ u32x4 buf_ld16(__amdgpu_buffer_rsrc_t r, int32_t voff, int32_t soff) {
     return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+}
+
+// LDS filled by DMA.
+typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void;
+
+VH_DEV u32x4s dma_rsrc(const void *p) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    return u32x4s{uint32_t(a), uint32_t(a >> 32) & 0xFFFFu, 0x7FFFFFFFu, uint32_t(kBufFlags)};
+}
+// 16 (4) bytes per lane from the buffer to LDS address lds + 16 lane (4 lane). Asm, because the compiler would wait for
+// every DMA in flight before each LDS read it cannot tell apart from them; no register is loaded, and the waits are
+// wait_step's.
+VH_DEV void dma_b128(u32x4s r, uint32_t lds, int voff, int soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+}
+VH_DEV void dma_b32(u32x4s r, uint32_t lds, int voff, int soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+}
+// All but the newest N of this wave's DMAs have landed, and its LDS reads have returned.
+template <int N>
+VH_DEV void wait_step() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
 
 // Cross-lane steps on the DPP path (no LDS round trip): quad permutations and row mirrors within 16-lane rows.

@@ -58,17 +58,26 @@ hipError_t launch_f5_fill_x(const float *x, int N, int mel, float *cat, int W, i
                   int32_t(B));
 }
 
-hipError_t launch_f5_attn(const _Float16 *qkv16, int64_t lo_off, float *out, _Float16 *out16, int B, int N,
-                          int heads, int hd, int ldvt, int ldo, float scale, hipStream_t s) {
+template <int W, int QT, int KS>
+static hipError_t f5_attn(const F5AttnArgs &a, int heads, int B, hipStream_t s) {
+    const hipError_t e = ensure_smem(reinterpret_cast<const void *>(&k_f5_attn<W, QT, KS>), f5_attn_smem(KS));
+    if (e != hipSuccess) return e;
+    return launch(k_f5_attn<W, QT, KS>, dim3(unsigned((a.N + 16 * QT * W - 1) / (16 * QT * W)), unsigned(heads), unsigned(B)),
+                  dim3(64 * W * KS), f5_attn_smem(KS), s, a);
+}
+hipError_t launch_f5_attn(const _Float16 *qkv16, float *out, _Float16 *out16, int B, int N, int heads, int hd, int np, int ldo,
+                          float scale, hipStream_t s) {
     if (B <= 0 || N <= 0) return hipSuccess;
-    if (hd != kF5Hd || heads <= 0 || ldvt < N || ldvt % 64 || lo_off % 8 || ldo % 4 || (out16 && ldo % 32) || (!out && !out16)) return hipErrorInvalidValue;
-    if ((int64_t(N) + 64) * 2 * heads * hd * 2 > INT32_MAX) return hipErrorInvalidValue;  // the q / k buffer offsets
-    F5AttnArgs a{qkv16, lo_off, out, int32_t(N), int32_t(ldo), int32_t(heads * hd), int32_t(ldvt), scale, out16};
-    // 4 query waves (64 rows) per block; when that leaves fewer blocks than CUs, 2 query waves (32 rows) times 2 key
-    // halves
-    if (int64_t((N + 63) / 64) * heads * B >= 256)
-        return launch(k_f5_attn<4, 1>, dim3(unsigned((N + 63) / 64), unsigned(heads), unsigned(B)), dim3(256), 0, s, a);
-    return launch(k_f5_attn<2, 2>, dim3(unsigned((N + 31) / 32), unsigned(heads), unsigned(B)), dim3(256), 0, s, a);
+    if (hd != kF5Hd || heads <= 0 || np < N || np % 64 || ldo % 4 || (out16 && ldo % 32) || (!out && !out16)) return hipErrorInvalidValue;
+    if ((int64_t(N) + 64) * 2 * heads * hd * 2 > INT32_MAX) return hipErrorInvalidValue;
+    const F5AttnArgs a{qkv16, out, out16, int32_t(N), int32_t(np), int32_t(ldo), scale};
+    // One block per CU (128 KiB of LDS): the fewest query rows per block that still fit the CUs at once. flow estimator,
+    // 2 x 8 heads of 512: 32-row blocks 9.6 us, 64-row 10.2, 128-row 14.8; DiT, 16 heads of 333: 7.8, 8.5, 12.6; 2 x 16 heads of
+    // 1000, more than fit with any: 60, 38 and 32, where a key tile read for 32 rows per wave costs half the LDS reads.
+    auto blocks = [&](int rows) { return int64_t((N + rows - 1) / rows) * heads * B; };
+    if (blocks(64) > 256) return f5_attn<4, 2, 2>(a, heads, B, s);
+    if (blocks(32) > 256) return f5_attn<4, 1, 2>(a, heads, B, s);
+    return f5_attn<2, 1, 2>(a, heads, B, s);
 }
 
 }  // namespace vh

@@ -141,8 +141,8 @@ static hipError_t gemm_tile(const uint8_t *w, const float *scale, const float *A
 
 
 bool rope_h16_ok(const GemmArgs &g) {
-    return g.h16 && g.hd > 0 && g.hd % 2 == 0 && g.seq > 0 && g.rope_cols % (2 * g.hd) == 0 && g.m % g.seq == 0 &&
-           g.n == g.rope_cols + g.rope_cols / 2 && g.ldvt >= g.seq && g.ldvt % 8 == 0 && g.lo_off % 8 == 0;
+    return g.h16 && g.hd == kQkvHead && g.seq > 0 && g.rope_cols % (2 * g.hd) == 0 && g.m % g.seq == 0 &&
+           g.n == g.rope_cols + g.rope_cols / 2 && g.seq_pad >= g.seq && g.seq_pad % 64 == 0;
 }
 
 // The operands an epilogue needs beyond y.

@@ -111,12 +111,11 @@ VH_DEV void gemm_epilogue(const f32x4v (&acc)[TM][TN], const GemmArgs &g, int m0
             const float gt = (EPI == EPI_GATED_ACC && col < g.n) ? g.gate[col] : 0.f;
             if (EPI == EPI_ROPE_H16 && n0 + wn * 16 * TN + j * 16 >= g.rope_cols && g.rope_cols % 16 == 0 && g.seq % 4 == 0) {
                 // a tile of v columns: this lane's 4 rows are 4 consecutive keys of one batch (seq % 4 == 0), so
-                // they go to v^T as one 8-byte store per plane instead of four strided 2-byte ones
+                // they are one 8-byte store per half instead of four 2-byte ones
                 const int row0 = m0 + wm * 16 * TM + i * 16 + 4 * (lane >> 4);
                 if (row0 < g.m && col < g.n) {
-                    const int cv = col - g.rope_cols, b = row0 / g.seq, n = row0 % g.seq;
-                    const int64_t idx = int64_t(g.m) * g.rope_cols +
-                                        ((int64_t(b) * (g.rope_cols / 2 / g.hd) + cv / g.hd) * g.hd + cv % g.hd) * g.ldvt + n;
+                    const int cv = col - g.rope_cols, heads = g.rope_cols / 2 / kQkvHead;
+                    const int64_t idx = qkv_off(2, row0 / g.seq, cv / kQkvHead, row0 % g.seq, cv % kQkvHead, g.m / g.seq, heads, g.seq_pad);
                     f16x4v hi, lo;
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
@@ -126,7 +125,7 @@ VH_DEV void gemm_epilogue(const f32x4v (&acc)[TM][TN], const GemmArgs &g, int m0
                         lo[v] = l;
                     }
                     *reinterpret_cast<f16x4v *>(g.h16 + idx) = hi;
-                    *reinterpret_cast<f16x4v *>(g.h16 + g.lo_off + idx) = lo;
+                    *reinterpret_cast<f16x4v *>(g.h16 + idx + kPlaneLo) = lo;
                 }
                 continue;
             }
@@ -156,16 +155,11 @@ VH_DEV void gemm_epilogue(const f32x4v (&acc)[TM][TN], const GemmArgs &g, int m0
                     } else if (in) {
                         _Float16 hi, lo;
                         bad |= split_f16(r, hi, lo);
-                        int64_t idx;
-                        if (col < g.rope_cols) {
-                            idx = int64_t(row) * g.rope_cols + col;
-                        } else {  // v, transposed: [batch][head][d][key]
-                            const int cv = col - g.rope_cols, b = row / g.seq, n = row % g.seq;
-                            const int64_t vbase = int64_t(g.m) * g.rope_cols;
-                            idx = vbase + ((int64_t(b) * (g.rope_cols / 2 / g.hd) + cv / g.hd) * g.hd + cv % g.hd) * g.ldvt + n;
-                        }
+                        const int inner = g.rope_cols / 2, sec = col / inner, cq = col - sec * inner;
+                        const int64_t idx = qkv_off(sec, row / g.seq, cq / kQkvHead, row % g.seq, cq % kQkvHead, g.m / g.seq,
+                                                    inner / kQkvHead, g.seq_pad);
                         g.h16[idx] = hi;
-                        g.h16[g.lo_off + idx] = lo;
+                        g.h16[idx + kPlaneLo] = lo;
                     }
                 } else if (in) {
                     if (EPI == EPI_STORE) *dst = c;

@@ -91,47 +91,40 @@ VH_DEV void halves_store(f32x4v c, const GemmArgs &g, int row, int c0, bool &bad
         *reinterpret_cast<uint2 *>(o + kPlaneLo) = lo;
     }
 }
-// EPI_ROPE_H16's store of columns c0 .. c0 + 3 (already rotated): q | k rows as they are; v transposed per batch and head,
-// four lanes of a quad exchanging so that each holds four keys of one dimension (every lane of the wave takes part).
+// EPI_ROPE_H16's store of columns c0 .. c0 + 3 (already rotated) in qkv_off's layout; for v four lanes of a quad exchange so
+// that each holds four keys of one dimension (every lane of the wave takes part).
 VH_DEV void rope_h16_store(const f32x4v &c, const GemmArgs &g, int row, int c0, int lane, bool &bad) {
-    const bool rin = row < g.m;
+    const bool rin = row < g.m && c0 < g.n;
+    const int inner = g.rope_cols / 2, heads = inner / kQkvHead, B = g.m / g.seq, b = row / g.seq, n = row - b * g.seq;
     uint2 hi, lo;
     const bool ovf = split_f16x4(c, hi, lo);
-    bad |= rin && c0 < g.n && ovf;
+    bad |= rin && ovf;
+    auto put = [&](int64_t idx, const uint2 &h, const uint2 &l) {
+        *reinterpret_cast<uint2 *>(g.h16 + idx) = h;
+        *reinterpret_cast<uint2 *>(g.h16 + idx + kPlaneLo) = l;
+    };
     if (c0 < g.rope_cols) {
-        if (rin) {
-            const int64_t idx = int64_t(row) * g.rope_cols + c0;
-            *reinterpret_cast<uint2 *>(g.h16 + idx) = hi;
-            *reinterpret_cast<uint2 *>(g.h16 + g.lo_off + idx) = lo;
-        }
+        const int sec = c0 >= inner, cq = c0 - sec * inner;
+        if (rin) put(qkv_off(sec, b, cq / kQkvHead, n, cq % kQkvHead, B, heads, g.seq_pad), hi, lo);
         return;
     }
-    // [batch][head][d][key]
-    const int b = row / g.seq, n = row - b * g.seq, vh = g.rope_cols / 2 / g.hd;
-    const int64_t vbase = int64_t(g.m) * g.rope_cols;
+    const int cv = c0 - g.rope_cols;
     // element e: hi in the low half, lo in the high half
     uint32_t x[4] = {(hi.x & 0xFFFFu) | lo.x << 16, hi.x >> 16 | (lo.x & 0xFFFF0000u), (hi.y & 0xFFFFu) | lo.y << 16,
                      hi.y >> 16 | (lo.y & 0xFFFF0000u)};
     if (g.seq % 4 == 0) {
         quad_transpose(x, lane);
-        const int col = c0 + (lane & 3), cv = col - g.rope_cols, k0 = n - (lane & 3);
-        if (rin && col < g.n) {
-            const int64_t idx = vbase + ((int64_t(b) * vh + cv / g.hd) * g.hd + cv % g.hd) * g.ldvt + k0;
-            uint2 h, l;
-            h.x = (x[0] & 0xFFFFu) | (x[1] << 16); h.y = (x[2] & 0xFFFFu) | (x[3] << 16);
-            l.x = (x[0] >> 16) | (x[1] & 0xFFFF0000u); l.y = (x[2] >> 16) | (x[3] & 0xFFFF0000u);
-            *reinterpret_cast<uint2 *>(g.h16 + idx) = h;
-            *reinterpret_cast<uint2 *>(g.h16 + g.lo_off + idx) = l;
+        if (rin) {
+            const uint2 h = {(x[0] & 0xFFFFu) | (x[1] << 16), (x[2] & 0xFFFFu) | (x[3] << 16)};
+            const uint2 l = {(x[0] >> 16) | (x[1] & 0xFFFF0000u), (x[2] >> 16) | (x[3] & 0xFFFF0000u)};
+            put(qkv_off(2, b, cv / kQkvHead, n - (lane & 3), cv % kQkvHead + (lane & 3), B, heads, g.seq_pad), h, l);
         }
     } else if (rin) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int cv = c0 + e - g.rope_cols;
-            if (c0 + e < g.n) {
-                const int64_t idx = vbase + ((int64_t(b) * vh + cv / g.hd) * g.hd + cv % g.hd) * g.ldvt + n;
-                g.h16[idx] = __builtin_bit_cast(_Float16, uint16_t(x[e]));
-                g.h16[g.lo_off + idx] = __builtin_bit_cast(_Float16, uint16_t(x[e] >> 16));
-            }
+            const int64_t idx = qkv_off(2, b, cv / kQkvHead, n, cv % kQkvHead + e, B, heads, g.seq_pad);
+            g.h16[idx] = __builtin_bit_cast(_Float16, uint16_t(x[e]));
+            g.h16[idx + kPlaneLo] = __builtin_bit_cast(_Float16, uint16_t(x[e] >> 16));
         }
     }
 }

@@ -5,28 +5,6 @@
 
 namespace vh {
 
-typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void;
-
-VH_DEV u32x4s hh_rsrc(const void *p) {
-    const uint64_t a = reinterpret_cast<uint64_t>(p);
-    return u32x4s{uint32_t(a), uint32_t(a >> 32) & 0xFFFFu, 0x7FFFFFFFu, uint32_t(kBufFlags)};
-}
-// 16 (4) bytes per lane from the buffer to LDS address lds + 16 lane (4 lane). Asm, because the compiler would wait for
-// every DMA in flight before each LDS read it cannot tell apart from them; no register is loaded, and the waits are
-// wait_step's.
-VH_DEV void dma_b128(u32x4s r, uint32_t lds, int voff, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
-}
-VH_DEV void dma_b32(u32x4s r, uint32_t lds, int voff, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
-}
-// All but the newest N of this wave's DMAs have landed, and its LDS reads have returned.
-template <int N>
-VH_DEV void wait_step() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
-}
-
 // y = A W^T with A = hi + lo (g.a16, plane_off's layout of m rows of K halves and planes) and W f16 in fragment order
 // (launch_pack_f16: [n / 16][k / 32][lane][8]), or (Q8) the int8 values of Q8 weights as f16 in that order with their
 // block scales transposed, [K / 32][ceil64(n)]; K a multiple of 64. Each f16 x f16 product is exact in the f32
@@ -63,7 +41,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_hh(const _Float16 *__r
     gemm_tile(gridDim.x, gridDim.y, g.n > 2 * g.m, tm, tn);
     const int m0 = tm * RA * 16, n0 = tn * RW * 16, K32 = g.K / 32;
     const int mb = (g.m + 15) / 16 - m0 / 16, nb = (g.n + 15) / 16 - n0 / 16, ns64 = (g.n + 63) / 64 * 64;
-    const u32x4s ra = hh_rsrc(g.a16 + int64_t(m0) * g.K * 2), rw = hh_rsrc(w + int64_t(n0) * g.K), rs = hh_rsrc(Q8 ? static_cast<const void *>(scale_t) : w);
+    const u32x4s ra = dma_rsrc(g.a16 + int64_t(m0) * g.K * 2), rw = dma_rsrc(w + int64_t(n0) * g.K), rs = dma_rsrc(Q8 ? static_cast<const void *>(scale_t) : w);
     // this wave's fragments of a stage (block rows past the last read the last: their outputs are not stored)
     int ca[PA], cw[PB];
     uint32_t da[PA], dw[PB];

@@ -140,8 +140,8 @@ hipError_t launch_layernorm_rows(const float *x, int64_t R, int D, const float *
 // Any row norm of NormArgs (LayerNorm / modulation, optional mish and channel bias; the CosyVoice2 estimator's blocks).
 hipError_t launch_norm_rows(const NormArgs &a, hipStream_t s);
 hipError_t launch_dwconv(const float *x, const float *w, const float *b, float *y, int64_t R, int C, int K, int seq, hipStream_t s);
-hipError_t launch_f5_attn(const _Float16 *qkv16, int64_t lo_off, float *out, _Float16 *out16, int B, int N,
-                          int heads, int hd, int ldvt, int ldo, float scale, hipStream_t s);
+hipError_t launch_f5_attn(const _Float16 *qkv16, float *out, _Float16 *out16, int B, int N, int heads, int hd, int np, int ldo,
+                          float scale, hipStream_t s);
 // Qwen3-TTS codec decoder: streaming histories (dst != old), the causal depthwise conv, the transposed conv's
 // overlap-add (tail_old -> tail_new, K <= 2 stride, with an optional Snake output), the pre-transformer's RoPE + ring
 // append and windowed attention,

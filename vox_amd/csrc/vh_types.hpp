@@ -184,15 +184,13 @@ struct GemmArgs {
     // heads padded with zero dims to hd (the attention tiles' 64): the table's head dim and the dims that rotate,
     // d < rope_hd (0: hd)
     int32_t rope_hd;
-    // EPI_ROPE_H16: the rotated q | k and v as f16 halves (x = hi + lo) for the attention's matrix cores, written to
-    // h16 instead of y: plane hi then plane lo (lo_off halves apart), each = q | k rows [m][rope_cols] followed by
-    // v transposed per batch and head, [m / seq][heads][hd][ldvt] (ldvt >= seq, a multiple of 8); rope null: the
-    // same layout without the rotation
+    // EPI_ROPE_H16 (hd 64): the rotated q | k and v as f16 halves (x = hi + lo) for the attention's matrix cores, written to
+    // h16 in qkv_off's layout (seq_pad rows per batch and head, a multiple of 64) instead of y; rope null: the same layout
+    // without the rotation
     // EPI_GELU_H16: gelu(c + bias) into f16 planes h16 of ldy columns (plane_off's layout); the tanh
     // form, or the erf form when gelu_erf is set. EPI_SWIGLU_H16: EPI_SWIGLU's silu(gate) up written the same way.
     _Float16 *h16;
-    int64_t lo_off;
-    int32_t ldvt;
+    int32_t seq_pad;
     const _Float16 *a16;  // k_gemm_hh: A as f16 planes of K columns (plane_off's layout)
     // ASRC_CONV: x [m][lda] rows of `seq`-row batches; group g = blockIdx.z reads channels [g cig, (g + 1) cig) at
     // rows t + k - ksize / 2 of the same batch (causal: t + k - (ksize - 1)) (zeros outside) for A column k cig + i;

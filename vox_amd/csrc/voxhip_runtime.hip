@@ -2278,10 +2278,9 @@ struct F5 {
     int B = 0, N = 0;
     float *cat = nullptr, *h = nullptr, *a = nullptr, *nrm = nullptr, *at = nullptr, *ffb = nullptr;
     float *ada = nullptr, *fin = nullptr, *ts = nullptr, *x = nullptr, *out = nullptr, *rope = nullptr;
-    // q | k rows and v^T ([B heads hd][ldvt], key columns padded with zeros to ldvt) as f16 hi, then lo, planes
+    // q, k and v as f16 halves (qkv_off's layout, np rows per batch and head)
     _Float16 *qkv16 = nullptr;
-    int64_t lo_off = 0;
-    int ldvt = 0;
+    int np = 0;
     // split: the modulated rows, the attention output and the GELU output as f16 planes (R rows each)
     _Float16 *nrm16 = nullptr, *at16 = nullptr, *ffb16 = nullptr;
 };
@@ -2459,8 +2458,7 @@ void f5_free_step(F5 &F) {
     F.cat = F.h = F.a = F.nrm = F.at = F.ffb = F.ada = F.fin = F.ts = F.x = F.out = F.rope = nullptr;
     for (_Float16 *p : {F.qkv16, F.nrm16, F.at16, F.ffb16}) dfree(p);
     F.qkv16 = F.nrm16 = F.at16 = F.ffb16 = nullptr;
-    F.B = F.N = F.ldvt = 0;
-    F.lo_off = 0;
+    F.B = F.N = F.np = 0;
 }
 
 GemmArgs gemm_args(const GpuMat &m, const float *bias, float *y, int64_t lda, int64_t ldy, int64_t rows) {
@@ -2522,10 +2520,9 @@ void f5_enqueue(F5 &F, hipStream_t s) {
         const GpuMat &Mq = mat_at(L.qkv);
         GemmArgs gq = gemm_args(Mq, Mq.b, nullptr, D, 3 * INNER, R);
         gq.rope = F.rope; gq.seq = F.N; gq.hd = F.hp; gq.rope_hd = F.hd; gq.rope_cols = 2 * INNER; gq.rope_heads = F.pe;
-        gq.h16 = F.qkv16; gq.lo_off = F.lo_off; gq.ldvt = F.ldvt;
+        gq.h16 = F.qkv16; gq.seq_pad = F.np;
         f5_lin(F, Mq, EPI_ROPE_H16, F.nrm, F.nrm16, gq, s);
-        HIPCHECK(launch_f5_attn(F.qkv16, F.lo_off, F.split ? nullptr : F.at, F.at16, F.B, F.N, F.heads, F.hp,
-                                F.ldvt, INNER, scale, s));
+        HIPCHECK(launch_f5_attn(F.qkv16, F.split ? nullptr : F.at, F.at16, F.B, F.N, F.heads, F.hp, F.np, INNER, scale, s));
         const GpuMat &Mo = mat_at(L.o);
         GemmArgs go = gemm_args(Mo, Mo.b, F.h, INNER, D, R);
         go.gate = ada + 2 * D;
@@ -2651,10 +2648,10 @@ int voxhip_f5_begin(int id, int B, int N, const float *cat0, const float *rope) 
             F.at = dalloc_t<float>(R * INNER);
             F.ffb = dalloc_t<float>(R * size_t(F.ff));
         }
-        F.ldvt = (N + 63) / 64 * 64;  // whole key tiles, the padding zero
-        F.lo_off = int64_t(R * 2 * INNER) + int64_t(B) * int64_t(INNER) * F.ldvt;
-        F.qkv16 = dalloc_t<_Float16>(size_t(2 * F.lo_off));
-        HIPCHECK(hipMemset(F.qkv16, 0, size_t(2 * F.lo_off) * sizeof(_Float16)));  // the v^T padding stays zero
+        F.np = (N + 63) / 64 * 64;  // whole key tiles, the padding zero
+        const size_t qkv = size_t(3) * size_t(B) * size_t(F.np) * INNER * 2;
+        F.qkv16 = dalloc_t<_Float16>(qkv);
+        HIPCHECK(hipMemset(F.qkv16, 0, qkv * sizeof(_Float16)));  // the padding stays zero
         F.ada = dalloc_t<float>((size_t(F.depth) * 6 + 2) * D);  // the blocks' vectors, then fin: one GEMV's rows
         F.fin = F.ada + size_t(F.depth) * 6 * D;
         F.ts = dalloc_t<float>(D); F.x = dalloc_t<float>(size_t(N) * F.mel);
@@ -2777,8 +2774,7 @@ struct Cosy {
     float *in = nullptr, *a = nullptr, *b = nullptr, *h = nullptr, *cat = nullptr, *xn = nullptr, *at = nullptr,
           *ff = nullptr, *tb = nullptr, *x = nullptr, *out = nullptr;
     _Float16 *qkv16 = nullptr, *xn16 = nullptr, *at16 = nullptr, *ff16 = nullptr;
-    int64_t lo_off = 0;
-    int ldvt = 0;
+    int np = 0;
     // the step's launches as one graph over the buffers of this begin (captured by the first step after it)
     hipGraphExec_t step_graph = nullptr;
 };
@@ -2795,8 +2791,7 @@ void cosy_free_step(Cosy &E) {
     E.in = E.a = E.b = E.h = E.cat = E.xn = E.at = E.ff = E.tb = E.x = E.out = nullptr;
     for (_Float16 *p : {E.qkv16, E.xn16, E.at16, E.ff16}) dfree(p);
     E.qkv16 = E.xn16 = E.at16 = E.ff16 = nullptr;
-    E.T = E.ldvt = 0;
-    E.lo_off = 0;
+    E.T = E.np = 0;
 }
 
 F5Conv cosy_conv_up(const voxhip_f5_conv &c, int cin, int cout, bool k1, const char *what) {
@@ -2881,10 +2876,9 @@ void cosy_xblock(const Cosy &E, const CosyX &L, const CosyX *next, bool *normed,
     const GpuMat &Mq = mat_at(L.qkv);
     GemmArgs gq = gemm_args(Mq, Mq.b, nullptr, C, 3 * INNER, R);
     gq.rope = nullptr; gq.seq = E.T; gq.hd = kF5HeadDim; gq.rope_cols = 2 * INNER;
-    gq.h16 = E.qkv16; gq.lo_off = E.lo_off; gq.ldvt = E.ldvt;
+    gq.h16 = E.qkv16; gq.seq_pad = E.np;
     split_lin(E.split, Mq, EPI_ROPE_H16, E.xn, E.xn16, gq, s);
-    HIPCHECK(launch_f5_attn(E.qkv16, E.lo_off, E.split ? nullptr : E.at, E.at16, 2, E.T, E.heads, kF5HeadDim,
-                            E.ldvt, INNER, 1.0f / std::sqrt(float(E.hd)), s));
+    HIPCHECK(launch_f5_attn(E.qkv16, E.split ? nullptr : E.at, E.at16, 2, E.T, E.heads, kF5HeadDim, E.np, INNER, 1.0f / std::sqrt(float(E.hd)), s));
     const GpuMat &Mo = mat_at(L.o), &M1 = mat_at(L.ff1), &M2 = mat_at(L.ff2);
     if (E.split && block_tail_ok(R, C, INNER, L.ff)) {
         BlockTailArgs t{};
@@ -3027,10 +3021,10 @@ int voxhip_cosy_begin(int id, int T, const float *in0) {
             E.at = dalloc_t<float>(R * INNER);
             E.ff = dalloc_t<float>(R * FF);
         }
-        E.ldvt = (T + 63) / 64 * 64;  // whole key tiles, the padding zero
-        E.lo_off = int64_t(R * 2 * INNER) + int64_t(2) * int64_t(INNER) * E.ldvt;
-        E.qkv16 = dalloc_t<_Float16>(size_t(2 * E.lo_off));
-        HIPCHECK(hipMemset(E.qkv16, 0, size_t(2 * E.lo_off) * sizeof(_Float16)));  // the v^T padding stays zero
+        E.np = (T + 63) / 64 * 64;  // whole key tiles, the padding zero
+        const size_t qkv = size_t(3) * 2 * size_t(E.np) * INNER * 2;
+        E.qkv16 = dalloc_t<_Float16>(qkv);
+        HIPCHECK(hipMemset(E.qkv16, 0, qkv * sizeof(_Float16)));  // the padding stays zero
         E.tb = dalloc_t<float>((2 + E.mid_res.size()) * C);
         E.x = dalloc_t<float>(size_t(T) * E.M);
         E.out = dalloc_t<float>(R * E.M);
