@@ -1,5 +1,5 @@
-"""The fused out-projection + FFN of a 256-channel block (k_block_tail) at the edges of its 16-row blocks and of its widths
-(inner 256 / 512 / 1280 and ff 256 / 1024 / 2048 in steps of 256), beside widths that take the separate launches (ff 320,
+"""The fused out-projection + FFN of a 256-channel block (k_block_tail) at the edges of its 16-row blocks, of its widths
+(inner 256 / 512 / 1280 and ff 256 / 1024 / 2048 in steps of 256) and of its blocks per 16 rows (1, 2, 4), beside widths that take the separate launches (ff 320,
 inner 192), through a one-level flow estimator against the oracle. Tolerance: a chain of about 20 products and norms whose
 longest f32 sum has 2048 terms, sqrt(2048) 2^-24 = 2.7e-6 each, roots of squares added: 1.3e-5; the GELU's fit adds 1.2e-7."""
 import numpy as np
@@ -12,12 +12,17 @@ pytestmark = pytest.mark.gpu
 TOL = 1.3e-5
 
 
-@pytest.mark.parametrize("heads,ff,n_x", [(8, 1024, 2), (4, 256, 1), (20, 512, 2), (8, 2048, 1), (3, 1024, 1), (8, 320, 2)])
-def test_block_tail_widths(hip, oracle, heads, ff, n_x):
+SMALL = (1, 7, 8, 9, 17)  # 2 T rows: a part of a block, one short of it, whole, one over, a third
+
+
+@pytest.mark.parametrize("heads,ff,n_x,frames", [(8, 1024, 2, SMALL), (4, 256, 1, SMALL), (20, 512, 2, SMALL), (8, 2048, 1, SMALL),
+                                                 (3, 1024, 1, SMALL), (8, 320, 2, SMALL),
+                                                 (1, 1024, 1, (513, 1025))])  # 2 and 1 blocks per 16 rows
+def test_block_tail_widths(hip, oracle, heads, ff, n_x, frames):
     m = CosyModel(60 + heads, M=8, C=256, heads=heads, head_dim=64, n_mid=1, n_x=n_x, ff=ff, wtype=F16)
     est = m.create(hip)
     rng = np.random.default_rng(ff)
-    for T in (1, 7, 8, 9, 17):  # 2 T rows: a part of a block, one short of it, whole, one over, a third
+    for T in frames:
         in0, x, tb = m.inputs(rng, T)
         hip.cosy_begin(est, T, in0)
         for _ in range(2):  # the captured step and its replay

@@ -8,15 +8,31 @@ bool block_tail_ok(int64_t R, int C, int inner, int ff) {
     return C == kTailC && R > 0 && R <= INT32_MAX && inner > 0 && inner % 256 == 0 && ff > 0 && ff % 256 == 0 &&
            block_tail_smem(inner, ff) <= 160 * 1024;
 }
+// Blocks per 16 rows, each with a part of the FFN: as many as 256 CUs hold at once (a block's LDS fills one), where ff gives
+// each whole passes of 256. In the flow estimator's step 4 instead of 1: 1024 rows 18.2 -> 15.6 us a launch, 202 rows 18.8 ->
+// 13.7 (the step 2737 -> 2547 and 2235 -> 1939 us). Every block repeats the out-projection and its norm.
+static int block_tail_parts(int64_t R, int ff) {
+    const int64_t tiles = (R + 127) / 128 * 8;
+    for (int ns : {4, 2})
+        if (tiles * ns <= 256 && ff % (256 * ns) == 0) return ns;
+    return 1;
+}
+int64_t block_tail_ws(int64_t R) { return R <= 2048 ? (R + 15) / 16 * 16 * 4 * kTailC : 0; }  // 4 parts up to 1024 rows, 2 up to 2048
+template <int NS>
+static hipError_t block_tail(const BlockTailArgs &a, hipStream_t s) {
+    const size_t smem = block_tail_smem(a.inner, a.ff / NS);
+    const hipError_t e = ensure_smem(reinterpret_cast<const void *>(&k_block_tail<NS>), smem);
+    const unsigned grid = NS == 1 ? unsigned((a.R + 15) / 16) : unsigned((a.R + 127) / 128 * 8 * NS);
+    return e != hipSuccess ? e : launch(k_block_tail<NS>, dim3(grid), dim3(512), smem, s, a);
+}
 hipError_t launch_block_tail(const BlockTailArgs &a0, hipStream_t s) {
     BlockTailArgs a = a0;
     a.status = status_word();
     if (!block_tail_ok(a.R, kTailC, a.inner, a.ff) || !a.a16 || !a.wo || !a.w1 || !a.w2 || !a.lw || !a.lb || !a.x ||
         (a.nw && (!a.nb || !a.out16)) || !(a.eps > 0.0))
         return hipErrorInvalidValue;
-    const size_t smem = block_tail_smem(a.inner, a.ff);
-    const hipError_t e = ensure_smem(reinterpret_cast<const void *>(&k_block_tail), smem);
-    return e != hipSuccess ? e : launch(k_block_tail, dim3(unsigned((a.R + 15) / 16)), dim3(512), smem, s, a);
+    const int ns = a.ws && a.count ? block_tail_parts(a.R, a.ff) : 1;
+    return ns == 4 ? block_tail<4>(a, s) : ns == 2 ? block_tail<2>(a, s) : block_tail<1>(a, s);
 }
 
 }  // namespace vh

@@ -15,28 +15,37 @@ namespace vh {
 // go from L2 straight to registers, 8 steps ahead across all three products (2 KiB per step and wave, 128 KiB in flight per
 // CU), and the waves meet only at the norms and around h.
 //
-// What bounds it: the weights through one CU, 1.25 MB at inner 512, ff 1024 whatever the rows, at about 50 bytes a clock
-// (16 KiB a step in 0.13 us; without the GELU, or with half the MFMAs, it is 0.3 us faster). 16.8 us at 202 to 2048 rows, 20.2
-// at 4096, for the five launches it replaces (o, norm, ff1, ff2, norm), about 29 us in the estimator's step at 202 and 1024
-// rows.
+// NS > 1 blocks share 16 rows: each takes A Wo^T and LN(x) whole and 1 / NS of the columns of h, and the last of them to
+// finish adds the NS partial products h W2^T, in their order, and does the rest.
+//
+// What bounds it: the weights through one CU, at about 50 bytes a clock (16 KiB a step in 0.13 us; without the GELU, or with
+// half the MFMAs, it is 0.3 us faster): 1.25 MB at inner 512, ff 1024 with one block per 16 rows, 0.5 MB with four. The five
+// launches it replaces (o, norm, ff1, ff2, norm) took about 29 us in the estimator's step at 202 and at 1024 rows, one block per
+// 16 rows 18.8 and 18.2, four 13.7 and 15.6.
 constexpr int kTailC = 256, kTailRed = 8 * 16 * 2;  // doubles of one norm's partial moments
-inline size_t block_tail_smem(int inner, int ff) { return size_t(inner > ff ? inner : ff) * 64 + kTailC * 64 + 2 * kTailRed * sizeof(double); }
+inline size_t block_tail_smem(int inner, int ff) {  // ff: a block's part
+    return size_t(inner > ff ? inner : ff) * 64 + kTailC * 64 + 2 * kTailRed * sizeof(double);
+}
 
+template <int NS>
 __global__ __launch_bounds__(512, 2) void k_block_tail(BlockTailArgs a) {
     constexpr int PF = 8, FS = 1024;  // weight steps in flight; bytes of a fragment
     extern __shared__ __align__(16) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lr = lane & 15, lg = lane >> 4;
-    const int row = int(blockIdx.x) * 16 + lr, rc = min(row, a.R - 1), vo = lane * 16;
+    // blocks of one tile are 8 apart, on one XCD where blocks go round-robin
+    const int tile = NS == 1 ? int(blockIdx.x) : int(blockIdx.x) / (8 * NS) * 8 + int(blockIdx.x) % 8, part = NS == 1 ? 0 : int(blockIdx.x) / 8 % NS;
+    if (NS > 1 && tile * 16 >= a.R) return;
+    const int row = tile * 16 + lr, rc = min(row, a.R - 1), vo = lane * 16;
     const bool rin = row < a.R;
-    const int KI = a.inner / 32, KF = a.ff / 32, c0 = wave * 32 + 4 * lg;  // this lane's channels: c0 .. + 3, c0 + 16 .. + 19
-    uint8_t *act = lds, *xn = lds + max(a.inner, a.ff) * 64;               // A, then h; LN(x)
+    const int KI = a.inner / 32, KF = a.ff / 32, FF = a.ff / NS, c0 = wave * 32 + 4 * lg;  // this lane's channels: c0 .. + 3, c0 + 16 .. + 19
+    uint8_t *act = lds, *xn = lds + max(a.inner, FF) * 64;                 // A, then this block's part of h; LN(x)
     double *red = reinterpret_cast<double *>(xn + kTailC * 64);
     auto frag = [&](const _Float16 *w, int f, int K32) { return reinterpret_cast<const uint8_t *>(w) + int64_t(f) * K32 * FS + vo; };
     auto sync = [&] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
 
     // everything the first product needs is on its way before the first wait: A's 16 rows (2 KiB per 32 columns,
     // consecutive; 16 KiB per 256 columns), x, the parameters, the first weights
-    const uint8_t *src = reinterpret_cast<const uint8_t *>(a.a16) + int64_t(blockIdx.x) * a.inner * 64 + threadIdx.x * 16;
+    const uint8_t *src = reinterpret_cast<const uint8_t *>(a.a16) + int64_t(tile) * a.inner * 64 + threadIdx.x * 16;
     constexpr int AP = 4;
     u32x4 ar[AP];
 #pragma unroll
@@ -72,10 +81,10 @@ __global__ __launch_bounds__(512, 2) void k_block_tail(BlockTailArgs a) {
         *reinterpret_cast<u32x4 *>(act + i + threadIdx.x * 16) = *reinterpret_cast<const u32x4 *>(src + i);
 
     f32x4v acc[2], acx[2];
-    // acc = the product of the rows at `rows` (LDS, `steps` 32-column tiles) with this wave's two fragment rows at cur; the
-    // last PF steps fetch the first ones of the next product (next, null: none). The order within a step is pinned: the next
+    // acc = the product of the rows at `rows` (LDS, `steps` 32-column tiles) with this wave's two fragment rows (K32 tiles
+    // each) at cur; the last PF steps fetch the first ones of the next product (next). The order within a step is pinned: the next
     // tile's LDS reads, this one's MFMAs, the weights PF steps on, so a wait for weights leaves the newer ones in flight.
-    auto product = [&](auto has_next, const uint8_t *rows, int steps, const uint8_t *cur, const uint8_t *next, int next_steps) {
+    auto product = [&](auto has_next, const uint8_t *rows, int steps, const uint8_t *cur, int K32, const uint8_t *next, int next_K32) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[j] = acx[j] = f32x4v{0.f, 0.f, 0.f, 0.f};
         const uint8_t *r = rows + vo, *last = r + (steps - 1) * 2048;
@@ -98,7 +107,7 @@ __global__ __launch_bounds__(512, 2) void k_block_tail(BlockTailArgs a) {
             for (int u = 0; u < PF; ++u) {
                 step(u);
 #pragma unroll
-                for (int j = 0; j < 2; ++j) w[u][j] = *reinterpret_cast<const f16x8v *>(q + (j * steps + u) * FS);
+                for (int j = 0; j < 2; ++j) w[u][j] = *reinterpret_cast<const f16x8v *>(q + (j * K32 + u) * FS);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
@@ -106,7 +115,7 @@ __global__ __launch_bounds__(512, 2) void k_block_tail(BlockTailArgs a) {
             step(u);
             if constexpr (decltype(has_next)::value) {
 #pragma unroll
-                for (int j = 0; j < 2; ++j) w[u][j] = *reinterpret_cast<const f16x8v *>(next + (j * next_steps + u) * FS);
+                for (int j = 0; j < 2; ++j) w[u][j] = *reinterpret_cast<const f16x8v *>(next + (j * next_K32 + u) * FS);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -170,20 +179,20 @@ __global__ __launch_bounds__(512, 2) void k_block_tail(BlockTailArgs a) {
     };
 
     sync();
-    const uint8_t *w1 = frag(a.w1, 2 * wave, 8), *w2 = frag(a.w2, 2 * wave, KF);
-    product(std::true_type{}, act, KI, p, w1, 8);
+    const uint8_t *w1 = frag(a.w1, part * (FF / 16) + 2 * wave, 8), *w2 = frag(a.w2, 2 * wave, KF) + part * (FF / 32) * FS;
+    product(std::true_type{}, act, KI, p, KI, w1, 8);
 #pragma unroll
     for (int j = 0; j < 2; ++j) x[j] += acc[j] + (a.bo ? bias[j] : zero);
     norm(red, lw, lb, n);  // its barrier: every wave has read A, whose LDS h takes
 #pragma unroll
     for (int j = 0; j < 2; ++j) put(xn, c0 + 16 * j, n[j]);
     sync();
-    for (int f = 0; f < a.ff; f += 256) {
+    for (int f = 0; f < FF; f += 256) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) bias[j] = vec(a.b1, f + c0 + 16 * j);
-        const bool more = f + 256 < a.ff;
+        for (int j = 0; j < 2; ++j) bias[j] = vec(a.b1, part * FF + f + c0 + 16 * j);
+        const bool more = f + 256 < FF;
         const uint8_t *nw1 = w1 + 16 * 8 * FS;
-        product(std::true_type{}, xn, 8, w1, more ? nw1 : w2, more ? 8 : KF);
+        product(std::true_type{}, xn, 8, w1, 8, more ? nw1 : w2, more ? 8 : KF);
         w1 = nw1;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -200,7 +209,41 @@ __global__ __launch_bounds__(512, 2) void k_block_tail(BlockTailArgs a) {
         lb[j] = vec(a.nb, c0 + 16 * j);
     }
     sync();
-    product(std::false_type{}, act, KF, w2, nullptr, 0);
+    product(std::false_type{}, act, FF / 32, w2, KF, nullptr, 0);
+    if constexpr (NS > 1) {
+        // the last of the tile's blocks to get here adds the parts, in their order whoever it is. The parts go past the
+        // caches that other XCDs do not see (agent-scope stores and loads), written before the count (the wait).
+        float *ws = a.ws + int64_t(tile) * NS * kTailC * 16 + threadIdx.x;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                __hip_atomic_store(ws + part * kTailC * 16 + (4 * j + e) * 512, acc[j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        int *last = reinterpret_cast<int *>(red);  // the first norm's moments are read
+        if (threadIdx.x == 0) *last = __hip_atomic_fetch_add(a.count + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == NS - 1;
+        __syncthreads();
+        if (!*last) {
+            raise_status(a.status, bad, kStatusF16Range);
+            return;
+        }
+        if (threadIdx.x == 0) __hip_atomic_store(a.count + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+        float pv[NS][8];
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                pv[k][e] = __hip_atomic_load(ws + k * kTailC * 16 + e * 512, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc[j][e] = pv[0][4 * j + e];
+#pragma unroll
+                for (int k = 1; k < NS; ++k) acc[j][e] += pv[k][4 * j + e];
+            }
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         x[j] += acc[j] + (a.b2 ? bias[j] : zero);
@@ -209,7 +252,7 @@ __global__ __launch_bounds__(512, 2) void k_block_tail(BlockTailArgs a) {
     if (a.nw) {
         norm(red + kTailRed, lw, lb, n);
         if (rin) {
-            uint8_t *o = reinterpret_cast<uint8_t *>(a.out16) + int64_t(blockIdx.x) * kTailC * 64;
+            uint8_t *o = reinterpret_cast<uint8_t *>(a.out16) + int64_t(tile) * kTailC * 64;
 #pragma unroll
             for (int j = 0; j < 2; ++j) put(o, c0 + 16 * j, n[j]);
         }

@@ -2774,6 +2774,8 @@ struct Cosy {
     float *in = nullptr, *a = nullptr, *b = nullptr, *h = nullptr, *cat = nullptr, *xn = nullptr, *at = nullptr,
           *ff = nullptr, *tb = nullptr, *x = nullptr, *out = nullptr;
     _Float16 *qkv16 = nullptr, *xn16 = nullptr, *at16 = nullptr, *ff16 = nullptr;
+    float *tail_ws = nullptr;       // launch_block_tail's partial sums and counts (split models)
+    int32_t *tail_count = nullptr;
     int np = 0;
     // the step's launches as one graph over the buffers of this begin (captured by the first step after it)
     hipGraphExec_t step_graph = nullptr;
@@ -2791,6 +2793,10 @@ void cosy_free_step(Cosy &E) {
     E.in = E.a = E.b = E.h = E.cat = E.xn = E.at = E.ff = E.tb = E.x = E.out = nullptr;
     for (_Float16 *p : {E.qkv16, E.xn16, E.at16, E.ff16}) dfree(p);
     E.qkv16 = E.xn16 = E.at16 = E.ff16 = nullptr;
+    dfree(E.tail_ws);
+    dfree(E.tail_count);
+    E.tail_ws = nullptr;
+    E.tail_count = nullptr;
     E.T = E.np = 0;
 }
 
@@ -2885,7 +2891,7 @@ void cosy_xblock(const Cosy &E, const CosyX &L, const CosyX *next, bool *normed,
         t.a16 = E.at16; t.wo = Mo.w16; t.w1 = M1.w16; t.w2 = M2.w16;
         t.bo = Mo.b; t.b1 = M1.b; t.b2 = M2.b; t.lw = L.n3w; t.lb = L.n3b;
         if (next) { t.nw = next->n1w; t.nb = next->n1b; }
-        t.x = A; t.out16 = E.xn16; t.eps = double(1e-5f); t.R = int32_t(R); t.inner = INNER; t.ff = L.ff;
+        t.ws = E.tail_ws; t.count = E.tail_count; t.x = A; t.out16 = E.xn16; t.eps = double(1e-5f); t.R = int32_t(R); t.inner = INNER; t.ff = L.ff;
         HIPCHECK(launch_block_tail(t, s));
         *normed = next != nullptr;
         return;
@@ -3016,6 +3022,17 @@ int voxhip_cosy_begin(int id, int T, const float *in0) {
             E.xn16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(C))));
             E.at16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(INNER))));
             E.ff16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(FF))));
+            if (C == 256 && block_tail_ws(int64_t(R)) > 0) try {
+                E.tail_ws = dalloc_t<float>(size_t(block_tail_ws(int64_t(R))));
+                E.tail_count = dalloc_t<int32_t>((R + 15) / 16);
+                HIPCHECK(hipMemset(E.tail_count, 0, (R + 15) / 16 * sizeof(int32_t)));  // each launch leaves them zero
+            } catch (const Fail &) {  // no room: one block per 16 rows
+                (void)hipGetLastError();
+                dfree(E.tail_ws);
+                dfree(E.tail_count);
+                E.tail_ws = nullptr;
+                E.tail_count = nullptr;
+            }
         } else {
             E.xn = dalloc_t<float>(R * C);
             E.at = dalloc_t<float>(R * INNER);
