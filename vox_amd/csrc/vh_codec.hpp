@@ -92,88 +92,106 @@ __global__ __launch_bounds__(256) void k_convt_gather(const float *__restrict__ 
     y[i] = bias ? v + bias[o] : v;
 }
 
-// The pre-transformer's q / k rotation (rope_apply, kernels.cpp:740-757: pairs (d, d + hd / 2)) with the host table
-// rope [F][hd / 2][2] of positions pos0 + i, and the append of row i's keys and values to ring slot (pos0 + i) % R of
-// the layer's f32 ring [R][kv_heads hd]. grid F, block 256; qkv rows [F][ld] = q | k | v; the call's first position
-// pos0 is read from device memory (*pos), so a captured call replays at any position.
-__global__ __launch_bounds__(256) void k_codec_rope_ring(float *__restrict__ qkv, int32_t ld, int32_t heads, int32_t kvh,
-                                                         int32_t hd, const float *__restrict__ rope,
-                                                         float *__restrict__ ring_k, float *__restrict__ ring_v,
-                                                         int32_t R, const int64_t *__restrict__ pos) {
-    const int i = blockIdx.x, half = hd / 2, qd = heads * hd, kd = kvh * hd;
-    const int64_t pos0 = *pos;
-    float *row = qkv + int64_t(i) * ld;
-    const float *cs = rope + int64_t(i) * hd;
-    const int64_t slot = (pos0 + i) % R;
-    for (int e = threadIdx.x; e < (heads + kvh) * half; e += 256) {
-        const int h = e / half, d = e % half;
-        float *p = h < heads ? row + h * hd : row + qd + (h - heads) * hd;
-        const float a = p[d], b = p[d + half], c = cs[2 * d], s = cs[2 * d + 1];
-        const float r0 = a * c - b * s, r1 = b * c + a * s;
-        if (h < heads) {
-            p[d] = r0;
-            p[d + half] = r1;
-        } else {
-            float *kr = ring_k + slot * kd + (h - heads) * hd;
-            kr[d] = r0;
-            kr[d + half] = r1;
-        }
-    }
-    for (int e = threadIdx.x; e < kd; e += 256) ring_v[slot * kd + e] = row[qd + kd + e];
-}
-
-// Sliding-window attention of row i (position pos0 + i) and head h over the ring (kernels.cpp:809-828 with the window
-// of :814): keys of positions (p - W, p], scores scale (q . k), softmax, sum p v. One wave per (row, head): lanes take
-// keys for the scores (a key row read as float4s) and head dimensions for the output (the value rows read across the
-// wave, eight positions in flight). Ring slots advance from the first one without a division per position.
-// W <= 1024, hd <= 128, hd % 4 == 0.
-__global__ __launch_bounds__(64) void k_codec_attn(const float *__restrict__ qkv, int32_t ld, const float *__restrict__ ring_k,
-                                                   const float *__restrict__ ring_v, int32_t R, int32_t heads, int32_t kvh,
-                                                   int32_t hd, const int64_t *__restrict__ pos, int32_t W, float scale,
-                                                   float *__restrict__ ao) {
-    __shared__ float p[1024];
-    __shared__ __align__(16) float q[128];
-    const int i = blockIdx.x, h = blockIdx.y, lane = threadIdx.x, kd = kvh * hd, off = (h / (heads / kvh)) * hd;
+// The pre-transformer's attention of one call, from the q | k | v rows [F][ld] of its frames: the q / k rotation (rope_apply,
+// kernels.cpp:740-757: pairs (d, d + hd / 2)) with the host table rope [F][hd / 2][2] of positions pos0 + i; the append of row
+// i's key and value to ring slot (pos0 + i) % R of the layer's f32 ring [R][kv_heads hd]; and the sliding-window attention of
+// row i (kernels.cpp:809-828 with the window of :814): keys of positions (p - W, p], scores scale (q . k), softmax, sum p v. The
+// call's own keys are rotated again by each block that needs them, from the rows, so no block waits for another's append,
+// and the appended slots are in no row's window (R >= W + F - 1). The first position pos0 is read from device memory (*pos), so a
+// captured call replays at any position. W <= 1024, hd <= 128, hd % 4 == 0, F <= 16.
+// One block per (row, head): a thread takes a key for the scores, then a dimension and every (256 / DT)th key for the output;
+// the ring's keys and values are on their way before anything waits. Bound by that latency: one wave reading the values eight
+// positions at a time took 6.5 us for a window of 72, after 3.8 us for the rotation and append in a launch of its own; 10.3 ->
+// 6.0 us.
+constexpr int kCodecRows = 16;
+template <int DT>
+__global__ __launch_bounds__(256) void k_codec_attn(const float *__restrict__ qkv, int32_t ld, float *ring_k, float *ring_v,
+                                                    const float *__restrict__ rope, int32_t R, int32_t heads, int32_t kvh, int32_t hd,
+                                                    const int64_t *__restrict__ pos, int32_t W, float scale, float *__restrict__ ao) {
+    constexpr int G = 256 / DT, VC = 24;  // key groups of the output, keys of a group in flight
+    __shared__ float p[1024], red[4], part[G][DT];
+    __shared__ __align__(16) float q[128], kc[kCodecRows][128];
+    const int i = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, d = tid % DT, grp = tid / DT;
+    const int qd = heads * hd, kd = kvh * hd, hk = h / (heads / kvh), off = hk * hd, half = hd / 2;
     const int64_t pos0 = *pos;
     const int64_t last = pos0 + i, first = last - W + 1 > 0 ? last - W + 1 : 0;
-    const int n = int(last - first + 1), s0 = int(first % R);
-    for (int d = lane; d < hd; d += 64) q[d] = qkv[int64_t(i) * ld + h * hd + d];
+    const int n = int(last - first + 1), s0 = int(first % R), nring = n - 1 - i > 0 ? n - 1 - i : 0;  // keys before the call's
+    const int r0 = i + 1 - (n - nring);  // the first of the call's rows in the window
+    auto slot_of = [&](int j) { return s0 + j < R ? s0 + j : s0 + j - R; };
+    auto value = [&](int j) {
+        return j < nring ? ring_v[int64_t(slot_of(j)) * kd + off + d] : qkv[int64_t(r0 + j - nring) * ld + qd + kd + off + d];
+    };
+    f32x4 kr[DT / 4];  // this thread's key, if the ring's
+    if (tid < nring) {
+        const f32x4 *k = reinterpret_cast<const f32x4 *>(ring_k + int64_t(slot_of(tid)) * kd + off);
+#pragma unroll
+        for (int e = 0; e < DT / 4; ++e) kr[e] = k[min(e, hd / 4 - 1)];
+    }
+    float v[VC];
+    if (d < hd) {
+#pragma unroll
+        for (int c = 0; c < VC; ++c) v[c] = grp + G * c < n ? value(grp + G * c) : 0.f;
+    }
+    for (int e = tid; e < (i + 2) * half; e += 256) {  // the call's keys up to row i, then q
+        const int r = e / half, x = e % half;
+        const bool key = r <= i;
+        const float *src = key ? qkv + int64_t(r) * ld + qd + off : qkv + int64_t(i) * ld + h * hd;
+        const float *cs = rope + int64_t(key ? r : i) * hd;
+        const float a = src[x], b = src[x + half], c = cs[2 * x], sn = cs[2 * x + 1];
+        float *o = key ? kc[r] : q;
+        o[x] = a * c - b * sn;
+        o[x + half] = b * c + a * sn;
+    }
     __syncthreads();
+    if (h % (heads / kvh) == 0 && tid < hd) {  // row i's slot, by the first query head of each kv head
+        const int64_t slot = last % R;
+        ring_k[slot * kd + off + tid] = kc[i][tid];
+        ring_v[slot * kd + off + tid] = qkv[int64_t(i) * ld + qd + kd + off + tid];
+    }
+    const f32x4 *qv = reinterpret_cast<const f32x4 *>(q);
     float mx = -INFINITY;
-    for (int j = lane; j < n; j += 64) {
-        int slot = s0 + j;
-        if (slot >= R) slot -= R;
-        const f32x4 *kr = reinterpret_cast<const f32x4 *>(ring_k + int64_t(slot) * kd + off);
-        const f32x4 *qv = reinterpret_cast<const f32x4 *>(q);
+    for (int j = tid; j < n; j += 256) {
         float dot = 0.f;
-        for (int d4 = 0; d4 < hd / 4; ++d4) {
-            const f32x4 a = kr[d4], b = qv[d4];
-            dot += b[0] * a[0] + b[1] * a[1] + b[2] * a[2] + b[3] * a[3];
+        auto term = [&](const f32x4 &a, const f32x4 &b) { dot += b[0] * a[0] + b[1] * a[1] + b[2] * a[2] + b[3] * a[3]; };
+        if (j < nring && j == tid) {
+#pragma unroll
+            for (int e = 0; e < DT / 4; ++e)
+                if (e < hd / 4) term(kr[e], qv[e]);
+        } else {
+            const f32x4 *k = j < nring ? reinterpret_cast<const f32x4 *>(ring_k + int64_t(slot_of(j)) * kd + off)
+                                       : reinterpret_cast<const f32x4 *>(kc[r0 + j - nring]);
+            for (int e = 0; e < hd / 4; ++e) term(k[e], qv[e]);
         }
         p[j] = scale * dot;
         mx = fmaxf(mx, p[j]);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
+    mx = wave_max(mx);
+    if (tid % 64 == 0) red[tid / 64] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     float sum = 0.f;
-    for (int j = lane; j < n; j += 64) {
+    for (int j = tid; j < n; j += 256) {
         p[j] = expf(p[j] - mx);
         sum += p[j];
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
+    sum = wave_sum(sum);
+    __syncthreads();  // every wave has read red
+    if (tid % 64 == 0) red[tid / 64] = sum;
     __syncthreads();
-    const float inv = 1.0f / sum;
-    for (int d = lane; d < hd; d += 64) {
-        const float *vb = ring_v + off + d;
-        float acc = 0.f;
-        int slot = s0;
-#pragma unroll 8
-        for (int j = 0; j < n; ++j) {
-            acc += p[j] * vb[int64_t(slot) * kd];
-            if (++slot == R) slot = 0;
-        }
-        ao[int64_t(i) * heads * hd + h * hd + d] = acc * inv;
+    const float inv = 1.0f / ((red[0] + red[1]) + (red[2] + red[3]));
+    float acc = 0.f;
+    if (d < hd) {
+#pragma unroll
+        for (int c = 0; c < VC; ++c) acc += grp + G * c < n ? p[grp + G * c] * v[c] : 0.f;
+        for (int j = grp + G * VC; j < n; j += G) acc += p[j] * value(j);
+    }
+    part[grp][d] = acc;
+    __syncthreads();
+    if (tid < hd) {
+        float o = part[0][tid];
+#pragma unroll
+        for (int g = 1; g < G; ++g) o += part[g][tid];
+        ao[int64_t(i) * heads * hd + h * hd + tid] = o * inv;
     }
 }
 

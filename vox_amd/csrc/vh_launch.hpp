@@ -158,10 +158,8 @@ hipError_t launch_ola(const float *tmp, const float *tail_old, float *tail_new, 
 // nn::ConvT's padded overlap-add (gather form) from the GEMM output z [T][K co] to y [To][co] (+ bias when not null).
 hipError_t launch_convt_gather(const float *z, const float *bias, float *y, int T, int To, int stride, int K, int pad, int co,
                                hipStream_t s);
-hipError_t launch_codec_rope_ring(float *qkv, int ld, int F, int heads, int kvh, int hd, const float *rope, float *ring_k,
-                                  float *ring_v, int R, const int64_t *pos, hipStream_t s);
-hipError_t launch_codec_attn(const float *qkv, int ld, const float *ring_k, const float *ring_v, int R, int F, int heads, int kvh,
-                             int hd, const int64_t *pos, int W, float scale, float *ao, hipStream_t s);
+hipError_t launch_codec_attn(const float *qkv, int ld, float *ring_k, float *ring_v, const float *rope, int R, int F, int heads,
+                             int kvh, int hd, const int64_t *pos, int W, float scale, float *ao, hipStream_t s);
 hipError_t launch_scale_acc(float *h, const float *t, const float *sc, int64_t rows, int H, hipStream_t s);
 hipError_t launch_clamp1(float *y, int64_t n, hipStream_t s);
 hipError_t launch_stream_conv(int wt, int epi, const uint8_t *w, const float *scale, const float *x, const GemmArgs &g,

@@ -3243,10 +3243,8 @@ int64_t codec_enqueue(Codec &E, CodecSt &St, int T, hipStream_t s) {
     for (int li = 0; li < E.layers; ++li) {
         const LayerDev &d = X.L[size_t(li)];
         gemv(mat_at(d.qkv), T, PRO_RMS, EPI_STORE, E.h, H, T, E.qkv, QW, X.norms + d.ln1, E.eps, nullptr, s, nullptr, E.pre);
-        HIPCHECK(launch_codec_rope_ring(E.qkv, QW, T, E.heads, E.kvh, E.hd, E.rope, St.kr[size_t(li)], St.vr[size_t(li)], E.R,
-                                        St.pos_dev, s));
-        HIPCHECK(launch_codec_attn(E.qkv, QW, St.kr[size_t(li)], St.vr[size_t(li)], E.R, T, E.heads, E.kvh, E.hd, St.pos_dev, E.W,
-                                   scale, E.ao, s));
+        HIPCHECK(launch_codec_attn(E.qkv, QW, St.kr[size_t(li)], St.vr[size_t(li)], E.rope, E.R, T, E.heads, E.kvh, E.hd, St.pos_dev,
+                                   E.W, scale, E.ao, s));
         // the layer scales (null: none) ride on the residual epilogue: h += scale (W x + b)
         gemv(mat_at(d.o), T, PRO_X, EPI_ACC, E.ao, qd, T, E.h, H, nullptr, 0.f, nullptr, s, nullptr, nullptr, nullptr, nullptr,
              nullptr, E.sa[size_t(li)]);
