@@ -133,7 +133,7 @@ VH_DEV void rope_h16_store(const f32x4v &c, const GemmArgs &g, int row, int c0, 
 // then holds four consecutive columns C[row][c0 .. c0 + 3] in c (row = lane % 16, c0 = 4 (lane / 16) of the tile), so a
 // RoPE or SwiGLU pair is in one lane and a store is 16 bytes of a row (8 of an f16 plane) instead of four 4-byte (2-byte)
 // stores to four rows. The sums and the elementwise formulas are gemm_epilogue's. vec (epi_vec): rows and parameters may
-// be accessed 16 bytes at a time where the four columns exist. All lanes of a wave call it (the v^T exchange).
+// be accessed 16 bytes at a time where the four columns exist. All lanes of a wave call it (the exchange of v).
 template <int EPI>
 VH_DEV void epi_tile(f32x4v c, const GemmArgs &g, int row, int c0, bool vec, int lane, bool &bad) {
     const bool rin = row < g.m, full = vec && c0 + 3 < g.n;

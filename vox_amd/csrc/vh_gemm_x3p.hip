@@ -33,8 +33,11 @@ static bool x3p_ok(int asrc, const GemmArgs &g) {
 //   against 10.2 us. From 100 of them on K is not split (1920 x 96, K 672, 120 tiles: 7.5 us against 8.9 with 2 slices
 //   and their reduce).
 // - fewer: K slices up to about 200 blocks, of at least 128 columns (32 x 768, K 5376: 11.3 us with 14 slices, 11.7 with
-//   21, 12.2 with 7; 160 x 384, K 2688: 10.1 with 7, 11.2 with 14). Where K is short or the epilogue cannot follow a
-//   reduce, 32 x 32 tiles of 4 waves instead (160 x 384, K 384: 5.0 us against 5.7 with 32 x 64, 6.6 with 2 slices).
+//   21, 12.2 with 7; 160 x 384, K 2688: 10.1 with 7, 11.2 with 14). Up to K 768, or where the epilogue cannot follow a reduce,
+//   32 x 32 tiles of 4 waves instead, since the reduce is a launch of 4.5 us (160 x 384, K 384: 5.0 us against 5.7 with 32 x 64,
+//   6.6 with 2 slices; the flow estimator's 202 x 256, K 768: 8.2 against 5.0 + 4.6 with 6 slices; 16 x 1026, K 512 as a matmul
+//   call 52 us against 56). At K 1024 it was faster still in the codec, but one chain of that length rounds more than the
+//   slices did (1.7e-6 against 1.4e-6 of the samples).
 enum { kT64x64, kT64x96, kT32x64, kT32x32 };
 struct X3Plan {
     int tile, splits, kchunk;
@@ -44,7 +47,7 @@ static X3Plan x3p_plan(const GemmArgs &g, int groups, bool reducible) {
     if (tiles(64, 64) >= 200) return {g.n == 96 ? kT64x96 : kT64x64, 1, 0};
     const int64_t t = tiles(32, 64);
     if (t >= 100) return {kT32x64, 1, 0};
-    if (!reducible || groups != 1 || !g.ws || g.K < 512) return {kT32x32, 1, 0};
+    if (!reducible || groups != 1 || !g.ws || g.K <= 768) return {kT32x32, 1, 0};
     const int64_t want = std::min<int64_t>((200 + t - 1) / t, g.K / 128);
     int kchunk = int(((g.K + want - 1) / want + 63) / 64 * 64);
     const int splits = (g.K + kchunk - 1) / kchunk;
