@@ -17,7 +17,9 @@ static int block_tail_parts(int64_t R, int ff) {
         if (tiles * ns <= 256 && ff % (256 * ns) == 0) return ns;
     return 1;
 }
-int64_t block_tail_ws(int64_t R) { return R <= 2048 ? (R + 15) / 16 * 16 * 4 * kTailC : 0; }  // 4 parts up to 1024 rows, 2 up to 2048
+// Tiles times parts are at most 256, tiles at most 128.
+int64_t block_tail_ws() { return 256 * 16 * kTailC; }
+int64_t block_tail_counts() { return 128; }
 template <int NS>
 static hipError_t block_tail(const BlockTailArgs &a, hipStream_t s) {
     const size_t smem = block_tail_smem(a.inner, a.ff / NS);

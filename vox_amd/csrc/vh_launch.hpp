@@ -76,8 +76,9 @@ hipError_t launch_pack_planes(const _Float16 *hi, const _Float16 *lo, int64_t m,
 // The row-local part of a transformer block as one launch, where block_tail_ok (256 channels, inner and ff multiples of
 // 256 that fit LDS).
 bool block_tail_ok(int64_t R, int C, int inner, int ff);
-// Floats of its ws at R rows (count: one int per 16 rows, zeroed once); ws and count null: one block per 16 rows.
-int64_t block_tail_ws(int64_t R);
+// Floats of its ws and ints of its count (zeroed once), whatever the rows; null: one block per 16 rows.
+int64_t block_tail_ws();
+int64_t block_tail_counts();
 hipError_t launch_block_tail(const BlockTailArgs &a, hipStream_t s);
 // Forces launch_gemm_hh's block tile (0: its shape policy); voxhip_bench_gemm_hh only.
 void set_gemm_hh_tile(int tile);

@@ -277,7 +277,7 @@ struct BlockTailArgs {
     _Float16 *out16;
     double eps;
     int32_t R, inner, ff;                        // inner and ff multiples of 256
-    float *ws;                                   // block_tail_ws(R) floats: partial sums of blocks that share rows
+    float *ws;                                   // block_tail_ws() floats: partial sums of blocks that share rows
     int32_t *count;                              // per 16 rows, zero between launches
     int32_t *status;
 };

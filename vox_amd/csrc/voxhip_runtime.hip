@@ -2774,7 +2774,9 @@ struct Cosy {
     float *in = nullptr, *a = nullptr, *b = nullptr, *h = nullptr, *cat = nullptr, *xn = nullptr, *at = nullptr,
           *ff = nullptr, *tb = nullptr, *x = nullptr, *out = nullptr;
     _Float16 *qkv16 = nullptr, *xn16 = nullptr, *at16 = nullptr, *ff16 = nullptr;
-    float *tail_ws = nullptr;       // launch_block_tail's partial sums and counts (split models)
+    // launch_block_tail's partial sums and counts (split models of its width), of any step: made by create, since two more
+    // allocations and a clear cost begin 0.6 ms
+    float *tail_ws = nullptr;
     int32_t *tail_count = nullptr;
     int np = 0;
     // the step's launches as one graph over the buffers of this begin (captured by the first step after it)
@@ -2793,10 +2795,6 @@ void cosy_free_step(Cosy &E) {
     E.in = E.a = E.b = E.h = E.cat = E.xn = E.at = E.ff = E.tb = E.x = E.out = nullptr;
     for (_Float16 *p : {E.qkv16, E.xn16, E.at16, E.ff16}) dfree(p);
     E.qkv16 = E.xn16 = E.at16 = E.ff16 = nullptr;
-    dfree(E.tail_ws);
-    dfree(E.tail_count);
-    E.tail_ws = nullptr;
-    E.tail_count = nullptr;
     E.T = E.np = 0;
 }
 
@@ -3001,6 +2999,17 @@ int voxhip_cosy_create(const voxhip_cosy_desc *d) {
         prepare(E->up_x);
         for (const auto &v : E->mid_x) prepare(v);
         E->split = split;
+        if (split && C == 256) try {
+            E->tail_ws = dalloc_t<float>(size_t(block_tail_ws()));
+            E->tail_count = dalloc_t<int32_t>(size_t(block_tail_counts()));
+            HIPCHECK(hipMemset(E->tail_count, 0, size_t(block_tail_counts()) * sizeof(int32_t)));  // each launch leaves them zero
+        } catch (const Fail &) {  // no room: one block per 16 rows
+            (void)hipGetLastError();
+            dfree(E->tail_ws);
+            dfree(E->tail_count);
+            E->tail_ws = nullptr;
+            E->tail_count = nullptr;
+        }
         g.cosy.push_back(E.release());
         return int(g.cosy.size()) - 1;
     }, -1);
@@ -3022,17 +3031,6 @@ int voxhip_cosy_begin(int id, int T, const float *in0) {
             E.xn16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(C))));
             E.at16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(INNER))));
             E.ff16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(FF))));
-            if (C == 256 && block_tail_ws(int64_t(R)) > 0) try {
-                E.tail_ws = dalloc_t<float>(size_t(block_tail_ws(int64_t(R))));
-                E.tail_count = dalloc_t<int32_t>((R + 15) / 16);
-                HIPCHECK(hipMemset(E.tail_count, 0, (R + 15) / 16 * sizeof(int32_t)));  // each launch leaves them zero
-            } catch (const Fail &) {  // no room: one block per 16 rows
-                (void)hipGetLastError();
-                dfree(E.tail_ws);
-                dfree(E.tail_count);
-                E.tail_ws = nullptr;
-                E.tail_count = nullptr;
-            }
         } else {
             E.xn = dalloc_t<float>(R * C);
             E.at = dalloc_t<float>(R * INNER);
