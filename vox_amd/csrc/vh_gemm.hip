@@ -91,11 +91,6 @@ static int split_plan(const GemmArgs &g, int *kchunk) {
         if (const int splits = plan(kSplitMaxSmall)) return splits;
     return plan(8);
 }
-template <int EPI>
-static hipError_t splitk_reduce(const GemmArgs &g, int splits, hipStream_t s) {
-    const int64_t threads = int64_t(g.m) * ((g.n + 3) / 4);
-    return launch(k_gemm_splitk_reduce<EPI>, dim3(unsigned((threads + 255) / 256)), dim3(256), 0, s, g, int32_t(splits));
-}
 template <int WT, int EPI>
 static hipError_t gemm_splitk(const uint8_t *w, const float *scale, const float *A, const GemmArgs &g, hipStream_t s, bool *done) {
     *done = false;
@@ -109,7 +104,7 @@ static hipError_t gemm_splitk(const uint8_t *w, const float *scale, const float 
         hipError_t e = gemm_run_h16<WT, EPI_STORE, 2, 2>(w, scale, A, gs, s);
         if (e != hipSuccess) return e;
         *done = true;
-        return splitk_reduce<EPI>(g, splits, s);
+        return launch_splitk_reduce<EPI>(g, splits, s);
     }
 }
 
@@ -131,7 +126,7 @@ static hipError_t gemm_tile(const uint8_t *w, const float *scale, const float *A
             if (splits) {
                 hipError_t e = WT == WT_F32 ? f32w_run<EPI_STORE, ASRC_ROWS>(w, A, gs, splits, s)
                                             : gemm_run<WT, EPI_STORE, ASRC_ROWS, 2>(w, scale, A, gs, splits, s);
-                return e != hipSuccess ? e : splitk_reduce<EPI>(g, splits, s);
+                return e != hipSuccess ? e : launch_splitk_reduce<EPI>(g, splits, s);
             }
         }
         if constexpr (WT == WT_F32) return f32w_run<EPI, ASRC_ROWS>(w, A, g, 1, s);
@@ -214,7 +209,7 @@ hipError_t launch_conv_gemm(int epi, const float *w, const float *A, const GemmA
         if (splits) {
             hipError_t e = f32w_run<EPI_STORE, ASRC_CONV>(wb, A, gs, splits, s);
             if (e != hipSuccess) return e;
-            return epi == EPI_STORE ? splitk_reduce<EPI_STORE>(g, splits, s) : splitk_reduce<EPI_ACC>(g, splits, s);
+            return epi == EPI_STORE ? launch_splitk_reduce<EPI_STORE>(g, splits, s) : launch_splitk_reduce<EPI_ACC>(g, splits, s);
         }
     }
     if (epi == EPI_MISH) return f32w_run<EPI_MISH, ASRC_CONV>(wb, A, g, groups, s);
@@ -234,7 +229,7 @@ static hipError_t stream_conv(const uint8_t *w, const float *scale, const float 
     if (splits) {
         hipError_t e = WT == WT_F32 ? f32w_run<EPI_STORE, ASRC_STREAM>(w, x, gs, splits, s)
                                     : gemm_run<WT, EPI_STORE, ASRC_STREAM, 2>(w, scale, x, gs, splits, s);
-        return e != hipSuccess ? e : splitk_reduce<EPI>(g, splits, s);
+        return e != hipSuccess ? e : launch_splitk_reduce<EPI>(g, splits, s);
     }
     if constexpr (WT == WT_F32) return f32w_run<EPI, ASRC_STREAM>(w, x, g, 1, s);
     return gemm_run<WT, EPI, ASRC_STREAM, 2>(w, scale, x, g, 1, s);

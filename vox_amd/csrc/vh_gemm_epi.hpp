@@ -2,6 +2,7 @@
 // split-K reduce that applies them.
 #pragma once
 #include "vh_gemm.hpp"
+#include "vh_launch.hpp"
 
 namespace vh {
 
@@ -322,35 +323,61 @@ VH_DEV void store_partial(const f32x4v &v, float *ws, const GemmArgs &g, int row
     }
 }
 
-// The split-K partial slices ws[z][m][n] added in z order, then bias and the epilogue: one thread per four columns of a
-// row. Eight slices' loads are in flight at once (past `splits` they read slice 0 and are left out). Bound by its launch
-// and one round trip of loads. grid ceil(m ceil(n / 4) / 256).
-template <int EPI>
+// The split-K partial slices ws[z][m][n] added in z order, then bias and the epilogue: one thread per U columns of a row, eight
+// slices' loads in flight at once (past `splits` they read slice 0 and are left out). U 4 where n is a multiple of 4; else one
+// column (a gate | up pair of SWIGLU), since four columns then are sixteen 4-byte loads and a chain of scalar stores a thread
+// (9 x 1026, K 3072 in 24 slices, product and reduce: 16.5 us with four columns, 11.1 with one). Bound by its launch and one
+// round trip of loads. grid ceil(m ceil(n / U) / 256).
+template <int EPI, int U>
 __global__ __launch_bounds__(256) void k_gemm_splitk_reduce(GemmArgs g, int32_t splits) {
-    const int nq = (g.n + 3) / 4;
+    static_assert(U == 4 || U == (EPI == EPI_SWIGLU ? 2 : 1), "four columns, or the epilogue's least");
+    const int nq = (g.n + U - 1) / U;
     const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (t >= int64_t(g.m) * nq) return;
-    const int row = int(t / nq), c0 = int(t % nq) * 4;
+    const int row = int(t / nq), c0 = int(t % nq) * U;
     const int64_t slice = int64_t(g.m) * g.n;
     const float *p = g.ws + int64_t(row) * g.n + c0;
     f32x4v v = {0.f, 0.f, 0.f, 0.f};
     for (int z0 = 0; z0 < splits; z0 += 8) {
         f32x4v x[8];
-        if (g.n % 4 == 0) {
 #pragma unroll
-            for (int z = 0; z < 8; ++z) x[z] = *reinterpret_cast<const f32x4v *>(p + (z0 + z < splits ? z0 + z : 0) * slice);
-        } else {
-#pragma unroll
-            for (int z = 0; z < 8; ++z)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) x[z][e] = c0 + e < g.n ? p[(z0 + z < splits ? z0 + z : 0) * slice + e] : 0.f;
+        for (int z = 0; z < 8; ++z) {
+            const float *q = p + (z0 + z < splits ? z0 + z : 0) * slice;
+            if constexpr (U == 4) {
+                x[z] = *reinterpret_cast<const f32x4v *>(q);
+            } else {
+                x[z] = f32x4v{q[0], U == 2 ? q[U - 1] : 0.f, 0.f, 0.f};
+            }
         }
 #pragma unroll
         for (int z = 0; z < 8; ++z)
             if (z0 + z < splits) v += x[z];
     }
-    bool bad = false;
-    epi_tile<EPI>(v, g, row, c0, epi_vec<EPI>(g), 0, bad);
+    if constexpr (U == 4) {
+        bool bad = false;
+        epi_tile<EPI>(v, g, row, c0, epi_vec<EPI>(g), 0, bad);
+    } else {
+#pragma unroll
+        for (int e = 0; e < U; ++e) v[e] += g.bias ? g.bias[c0 + e] : 0.f;
+        if constexpr (EPI == EPI_SWIGLU) {
+            g.y[int64_t(row) * g.ldy + c0 / 2] = silu(v[0]) * v[1];
+        } else {
+            constexpr bool kAcc = EPI == EPI_ACC || EPI == EPI_GATED_ACC || EPI == EPI_ACC_SNAKE, kSnake = EPI == EPI_SNAKE || EPI == EPI_ACC_SNAKE;
+            const int64_t idx = int64_t(row) * g.ldy + c0;
+            f32x4v o2 = {0.f, 0.f, 0.f, 0.f};
+            g.y[idx] = epi_value<EPI>(v[0], kAcc ? g.y[idx] : 0.f, EPI == EPI_GATED_ACC ? g.gate[c0] : kSnake ? g.snake_a[c0] : 0.f,
+                                      kSnake ? g.snake_ib[c0] : 0.f, o2, 0);
+            if constexpr (EPI == EPI_ACC_SNAKE) g.snake_y[idx] = o2[0];
+        }
+    }
+}
+template <int EPI>
+hipError_t launch_splitk_reduce(const GemmArgs &g, int splits, hipStream_t s) {
+    constexpr int U = EPI == EPI_SWIGLU ? 2 : 1;
+    const int u = g.n % 4 == 0 ? 4 : U;
+    const dim3 grid(unsigned((int64_t(g.m) * ((g.n + u - 1) / u) + 255) / 256));
+    if (u == 4) return launch(k_gemm_splitk_reduce<EPI, 4>, grid, dim3(256), 0, s, g, int32_t(splits));
+    return launch(k_gemm_splitk_reduce<EPI, U>, grid, dim3(256), 0, s, g, int32_t(splits));
 }
 template <int EPI>
 constexpr bool kReduceEpi = EPI == EPI_STORE || EPI == EPI_ACC || EPI == EPI_GATED_ACC || EPI == EPI_SWIGLU || EPI == EPI_SNAKE ||

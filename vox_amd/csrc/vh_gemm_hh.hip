@@ -93,9 +93,7 @@ static hipError_t hh_split_or_run(const _Float16 *w, const float *scale_t, const
     const int splits = hh_split(g, &gs.kchunk);
     if (!splits) return hh_wt<EPI>(hh_tile(g, scale_t != nullptr), w, scale_t, g, s);
     const hipError_t e = hh_wt<EPI_STORE>(kH32x64, w, scale_t, gs, s);
-    if (e != hipSuccess) return e;
-    const int64_t threads = int64_t(g.m) * ((g.n + 3) / 4);
-    return launch(k_gemm_splitk_reduce<EPI>, dim3(unsigned((threads + 255) / 256)), dim3(256), 0, s, g, int32_t(splits));
+    return e != hipSuccess ? e : launch_splitk_reduce<EPI>(g, splits, s);
 }
 
 hipError_t launch_gemm_hh_acc_rms(const _Float16 *w, const float *scale_t, const GemmArgs &g0, const float *gamma, float eps,

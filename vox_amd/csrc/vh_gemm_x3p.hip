@@ -78,9 +78,7 @@ static hipError_t x3p_run(const float *A, const GemmArgs &g, int groups, hipStre
         GemmArgs gs = g;
         gs.kchunk = p.kchunk;
         const hipError_t e = x3p_tiles<EPI_STORE, ASRC>(p.tile, A, gs, p.splits, s);
-        if (e != hipSuccess) return e;
-        const int64_t threads = int64_t(g.m) * ((g.n + 3) / 4);
-        return launch(k_gemm_splitk_reduce<EPI>, dim3(unsigned((threads + 255) / 256)), dim3(256), 0, s, g, int32_t(p.splits));
+        return e != hipSuccess ? e : launch_splitk_reduce<EPI>(g, p.splits, s);
     }
     return hipErrorInvalidValue;  // no plan splits such a product
 }
