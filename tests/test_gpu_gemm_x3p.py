@@ -39,6 +39,15 @@ def test_matmul_f32(hip, m, n, K):
     assert np.all(err <= bound(x, w) + 2.0 ** -23 * np.abs(want)), float(np.max(err))
 
 
+@pytest.mark.parametrize("m,n,K", [
+    (33, 2753, 2048), (64, 4094, 2120), (33, 6081, 4096),  # 64 x 64 tiles in 5, 4 and 2 slices, a short last one
+    (80, 2433, 2056), (400, 514, 5376),                    # 32 x 64 tiles, odd rows of them, in two slices
+    (200, 1347, 3080),                                     # in three
+    (64, 2113, 1096), (80, 2433, 2040)])                   # 66 tiles: three slices; K one step short of two
+def test_matmul_f32_long_k(hip, m, n, K):
+    test_matmul_f32(hip, m, n, K)
+
+
 def test_codec_96_channels(hip, oracle):
     # a decoder whose last block has 96 channels at 6,656 rows a call: its convolutions fill the CUs with 64 x 96 tiles, the
     # first block of tiles of each reads the history

@@ -30,14 +30,21 @@ static bool x3p_ok(int asrc, const GemmArgs &g) {
 //   waves and 46 with 64 x 96 of 4 waves); 64 x 96 where n is an odd multiple of 96 up to 96 itself (30720 x 96, K 672:
 //   24.6 against 31.3 us, a third of the second 64-column tile being padding).
 // - below that 32 x 64 tiles of 8 waves: 333 x 64 x 16 groups, K 1984: 16.9 against 23.4 us; 1024 x 256, K 768: 8.4
-//   against 10.2 us. From 100 of them on K is not split (1920 x 96, K 672, 120 tiles: 7.5 us against 8.9 with 2 slices
-//   and their reduce).
+//   against 10.2 us. From 100 of them on a K below 2048 is not split (1920 x 96, K 672, 120 tiles: 7.5 us against 8.9 with 2
+//   slices and their reduce).
 // - fewer: K slices up to about 200 blocks, of at least 128 columns (32 x 768, K 5376: 11.3 us with 14 slices, 11.7 with
-//   21, 12.2 with 7; 160 x 384, K 2688: 10.1 with 7, 11.2 with 14). Up to K 768, or where the epilogue cannot follow a reduce,
+//   21, 12.2 with 7; 160 x 384, K 2688: 10.1 with 7, 11.2 with 14), and at most 256 blocks, a round of the CUs (64 x 2112,
+//   K 5376, 66 tiles: 23.4 us with 3 slices, 29.9 with 4). Up to K 768, or where the epilogue cannot follow a reduce,
 //   32 x 32 tiles of 4 waves instead, since the reduce is a launch of 4.5 us (160 x 384, K 384: 5.0 us against 5.7 with 32 x 64,
 //   6.6 with 2 slices; the flow estimator's 202 x 256, K 768: 8.2 against 5.0 + 4.6 with 6 slices; 16 x 1026, K 512 as a matmul
 //   call 52 us against 56). At K 1024 it was faster still in the codec, but one chain of that length rounds more than the
 //   slices did (1.7e-6 against 1.4e-6 of the samples).
+// - a long K from 86 tiles on, where a round of them holds two slices or none: 64 x 64 tiles in slices up to 256 blocks where
+//   they pad no rows, up to 64 of them from K 2048 (33 x 3072, K 5376: 22.8 us against 28.8 with 32 x 64 in 2 slices and 24.7-26.7
+//   by k_gemm_x3; 128 x 1472, K 3072 18.4 against 21.8 and 22.0; 64 x 1024 x K 2048, 32 tiles, no gain), up to 96 from K 4096
+//   (64 x 6144, K 5376: 40.4 against 45.2 unsplit; at K 2048 23.2 against 21.8). Odd counts of row tiles: two slices of 32 x 64
+//   up to 128 tiles from K 2048 (400 x 512, K 5376: 29.5 us, unsplit 45.3, k_gemm_x3 31.2; K 2048: 16.6, 19.5, 19.1), three up to
+//   170 from K 3072 (400 x 768, K 5376: 39.6 us, unsplit 46.2, k_gemm_x3 44.1; at K 2048 20.7 against 19.7).
 enum { kT64x64, kT64x96, kT32x64, kT32x32 };
 struct X3Plan {
     int tile, splits, kchunk;
@@ -45,14 +52,23 @@ struct X3Plan {
 static X3Plan x3p_plan(const GemmArgs &g, int groups, bool reducible) {
     auto tiles = [&](int bm, int bn) { return int64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * groups; };
     if (tiles(64, 64) >= 200) return {g.n == 96 ? kT64x96 : kT64x64, 1, 0};
-    const int64_t t = tiles(32, 64);
-    if (t >= 100) return {kT32x64, 1, 0};
-    if (!reducible || groups != 1 || !g.ws || g.K <= 768) return {kT32x32, 1, 0};
-    const int64_t want = std::min<int64_t>((200 + t - 1) / t, g.K / 128);
-    int kchunk = int(((g.K + want - 1) / want + 63) / 64 * 64);
-    const int splits = (g.K + kchunk - 1) / kchunk;
-    if (splits < 2 || int64_t(splits) * g.m * g.n > g.ws_cap) return {kT32x32, 1, 0};
-    return {kT32x64, splits, kchunk};
+    const int64_t t = tiles(32, 64), t64 = tiles(64, 64);
+    const bool split = reducible && groups == 1 && g.ws;
+    X3Plan whole{t >= 100 ? kT32x64 : kT32x32, 1, 0}, p{kT32x64, 1, 0};
+    int64_t want = 1;
+    if (split && t > 85 && t == 2 * t64 && ((t64 <= 64 && g.K >= 2048) || (t64 <= 96 && g.K >= 4096))) {
+        p.tile = kT64x64;
+        want = 256 / t64;
+    } else if (split && t >= 100) {
+        if (t <= 128 && g.K >= 2048) want = 2;
+        else if (t > 128 && t <= 170 && g.K >= 3072) want = 3;
+    } else if (split && g.K > 768) {
+        want = std::min<int64_t>({(200 + t - 1) / t, 256 / t, g.K / 128});
+    }
+    if (want < 2) return whole;
+    p.kchunk = int(((g.K + want - 1) / want + 63) / 64 * 64);
+    p.splits = (g.K + p.kchunk - 1) / p.kchunk;
+    return p.splits < 2 || int64_t(p.splits) * g.m * g.n > g.ws_cap ? whole : p;
 }
 
 template <int EPI, int ASRC, int WM, int WN, int TM, int TN>
