@@ -101,7 +101,9 @@ int voxhip_upload(const voxhip_mat *parts, int n_parts);
  * and use integer dots; Q8 with m > 8 and F32/F16/BF16 use f32 activations. Returns 1 or 0. */
 int voxhip_matmul(int mat, const float *x, int64_t m, float *y);
 /* voxhip_matmul on device-resident rows, allocating nothing: d_y [m][rows] = d_x [m][cols] . W^T (+ bias), with the
- * arithmetic of voxhip_matmul (the same kernels and m-dependent paths). No counterpart in the reference: it is for
+ * arithmetic of voxhip_matmul (the same m-dependent paths; F32 weights of more than 4 rows are read as stored, where
+ * voxhip_matmul reads a copy laid out for the matrix cores: the same products, summed in another order). A call gives the
+ * same bits whatever calls came before it. No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc). It calls no hipMalloc / hipFree: the split-K partial sums and the int path's once-quantized
  * input rows live in a fixed 6.3 MiB array in the library's code object (one copy per device, held until the

@@ -584,8 +584,8 @@ bool ffn_quant_epilogue(const GpuMat &gu, const GpuMat &dn, int64_t m_total, int
 }
 
 // One matrix pass: y (=, +=, swiglu) W * prologue(x) for mc rows. On the GEMM path the prologue runs as its own
-// kernel into pre ([mc][cols]; xnorm instead when the normed rows are wanted). sc: the pass's scratch (null: the
-// library's).
+// kernel into pre ([mc][cols]; xnorm instead when the normed rows are wanted). scp: the pass's scratch (null: the
+// library's; set by the no-alloc call alone).
 // acc (one row on the int path): the fused FFN's pending sums, added to x (PRO_RMS) or to y before the product
 // (EPI_ACC, which also clears the rows it consumed).
 // qout (EPI_SWIGLU on pre-quantized rows): the SwiGLU output goes to these quantized rows instead of y; qin (PRO_X):
@@ -622,7 +622,9 @@ void gemv(const GpuMat &m, int64_t m_total, int pro, int epi, const float *x, in
         ga.ws = sc.ws; ga.ws_cap = sc.ws_cap;
         ga.gate = yscale;  // a row scale of the GEMV is the GEMM's gated residual (y += gate[col] (c + bias))
         ga.f32_wide = f32_wide(m);
-        ga.wx = m.wx;
+        // the no-alloc call (its own scratch) always reads the weights as stored: it cannot lay them out, its bits must not
+        // depend on whether another call did, and a caller's graph may hold its launches for good
+        ga.wx = scp ? nullptr : m.wx;
         HIPCHECK(launch_gemm(gemv_type(m), yscale ? EPI_GATED_ACC : epi, m.w, m.s, A, ga, s));
         return;
     }
