@@ -846,12 +846,22 @@ void prepare_w16(GpuMat &m, hipStream_t s) {
     m.w16 = w16;
     m.st = st;
 }
-void prepare_planes(Xfmr &X, int first, int count, int64_t m_total, int mc, hipStream_t s) {
-    for (int li = first; li < first + count; ++li)
-        if (planes_layer(X, li, m_total, mc, false)) {
-            const LayerDev &L = X.L[size_t(li)];
-            for (int id : {L.qkv, L.o, L.gu, L.down}) prepare_w16(g.mats[size_t(id)], s);
+// Lays out what a pass of mc rows reads, before its launches are enqueued or captured: every entry point does it before every
+// pass, so that a call's kernels do not depend on the calls before it. One matrix; then the matrices of layers first ..
+// first + count - 1 (the row table set).
+void prepare_mat(GpuMat &m, int64_t m_total, int mc, hipStream_t s) {
+    if (gemm_path(m, m_total, mc)) prepare_x3(m, s);
+}
+void prepare_layers(Xfmr &X, int first, int count, int64_t m_total, int mc, bool fused, hipStream_t s) {
+    const bool pass_attn = pass_attn_of(X, mc, fused);
+    for (int li = first; li < first + count; ++li) {
+        const LayerDev &L = X.L[size_t(li)];
+        const bool planes = pass_attn && planes_layer(X, li, m_total, mc, false);
+        for (int id : {L.qkv, L.o, L.gu, L.down}) {
+            if (planes) prepare_w16(g.mats[size_t(id)], s);
+            else prepare_mat(g.mats[size_t(id)], m_total, mc, s);
         }
+    }
 }
 
 // x0 (optional): the input rows ([mc][H]) when they are not in X.h yet. The first layer's q|k|v GEMV then reads them
@@ -1066,6 +1076,7 @@ int forward_rows(Xfmr &X, int64_t m, RowsOf rows_of, const float *x, int in_proj
         std::memcpy(pin, x + c0 * xc, size_t(mc * xc) * 4);
         if (Pm) {
             float *xin = ensure_xin(X, int64_t(chunk) * xc);
+            prepare_mat(mat_at(in_proj), m_total, mc, g.stream);
             HIPCHECK(copy_h2d(xin, pin, size_t(mc * xc) * 4, g.stream));
             gemv(*Pm, m_total, PRO_X, EPI_STORE, xin, xc, mc, X.h, H, nullptr, 0.f, nullptr, g.stream);
         } else {
@@ -1075,10 +1086,7 @@ int forward_rows(Xfmr &X, int64_t m, RowsOf rows_of, const float *x, int in_proj
         for (int i = 0; i < mc && fused; ++i)
             for (int j = 0; j < i; ++j)
                 if (rr[size_t(i)].k == rr[size_t(j)].k) { fused = false; break; }
-        for (int li = first_layer; li < first_layer + n_layers; ++li)
-            for (int id : {X.L[size_t(li)].qkv, X.L[size_t(li)].o, X.L[size_t(li)].gu, X.L[size_t(li)].down})
-                if (gemm_path(g.mats[size_t(id)], m_total, mc)) prepare_x3(g.mats[size_t(id)], g.stream);
-        if (pass_attn_of(X, mc, fused)) prepare_planes(X, first_layer, n_layers, m_total, mc, g.stream);
+        prepare_layers(X, first_layer, n_layers, m_total, mc, fused, g.stream);
         run_layers(X, mc, m_total, first_layer, n_layers, fused);
         if (hidden_out) {
             HIPCHECK(copy_d2h(pin, X.h, size_t(mc * H) * 4, g.stream));
@@ -1088,6 +1096,7 @@ int forward_rows(Xfmr &X, int64_t m, RowsOf rows_of, const float *x, int in_proj
         if (final_all || last) {
             const int r0 = final_all ? 0 : mc - 1, mr = final_all ? mc : 1;
             if (out_last || head >= 0) {
+                if (head >= 0) prepare_mat(mat_at(head), mr, mr, g.stream);
                 enqueue_final(X, r0, mr, head, g.stream);
                 if (out_last) {
                     HIPCHECK(copy_d2h(pin, X.xnorm, size_t(mr * H) * 4, g.stream));
@@ -1449,7 +1458,7 @@ int voxhip_matmul(int mat, const float *x, int64_t m, float *y) {
         GpuMat &M = mat_at(mat);
         if (m <= 0) return 1;
         const int chunk = rows_per_pass(M, m);
-        if (gemm_path(M, m, int(std::min<int64_t>(chunk, m)))) prepare_x3(M, g.stream);
+        prepare_mat(M, m, int(std::min<int64_t>(chunk, m)), g.stream);
         const size_t xb = size_t(chunk) * size_t(M.cols) * 4, yb = size_t(chunk) * size_t(M.rows) * 4;
         float *pin = pinned(std::max(xb, yb) + 64);
         float *dx = dev_scratch(g.dbuf_x, g.dbuf_x_bytes, xb), *dy = dev_scratch(g.dbuf_y, g.dbuf_y_bytes, yb);
@@ -1546,7 +1555,7 @@ int voxhip_convt(int mat, int32_t K, int32_t stride, int32_t pad, int32_t out_pa
         HIPCHECK(copy_h2d(dx, pin, xb + bb, g.stream));
         // z = x W^T, frames in passes of the matrix's pass height, then the padded overlap-add + bias
         const int chunk = rows_per_pass(M, T);
-        if (gemm_path(M, T, int(std::min<int64_t>(chunk, T)))) prepare_x3(M, g.stream);
+        prepare_mat(M, T, int(std::min<int64_t>(chunk, T)), g.stream);
         for (int64_t c0 = 0; c0 < T; c0 += chunk) {
             const int mc = int(std::min<int64_t>(chunk, T - c0));
             gemv(M, T, PRO_X, EPI_STORE, dx + c0 * cin, cin, mc, dz + c0 * KO, KO, nullptr, 0.f, nullptr, g.stream);
@@ -1853,7 +1862,13 @@ void prepare_decode(Xfmr &X, Seq &S, int64_t pos0, int64_t m, int head, const vo
     std::vector<RowRef> rr(static_cast<size_t>(m));
     for (int64_t i = 0; i < m; ++i) rr[size_t(i)] = row_of(S, pos0 + i);
     set_rows(X, rr);
+    prepare_layers(X, 0, X.layers, m, int(m), m == 1, g.stream);
     if (cfg) set_sample_cfgs(X, cfg, 1);
+}
+// The same for a step of one row for each of B sequences, whose rows are set: its head runs on every row.
+void prepare_steps(Xfmr &X, int B, int head) {
+    prepare_layers(X, 0, X.layers, B, B, true, g.stream);
+    if (head >= 0) prepare_mat(mat_at(head), B, B, g.stream);
 }
 
 uint64_t gemv_stream_bytes(const Xfmr &X) {
@@ -1906,6 +1921,7 @@ int voxhip_decode_steps_dev(int xfmr, const int32_t *seqs, const int64_t *pos, i
         }
         prepare_head(X, head, cfgs != nullptr);
         set_rows(X, rr);
+        prepare_steps(X, int(B), head);
         if (cfgs) set_sample_cfgs(X, cfgs, int(B));
         vh::prof_stage(X.name.c_str());
         if (vh::prof_on()) {  // stamped launches are not captured
@@ -3963,6 +3979,7 @@ int voxhip_bench_decode_steps(int xfmr, const int32_t *seqs, const int64_t *pos,
         }
         prepare_head(X, head, cfgs != nullptr);
         set_rows(X, rr);
+        prepare_steps(X, int(B), head);
         if (cfgs) set_sample_cfgs(X, cfgs, int(B));
         bench_decode_impl(X, key, int(B), true, ps, d_x, head, cfgs != nullptr, d_tokens, warmup, steps, out);
         return 1;
