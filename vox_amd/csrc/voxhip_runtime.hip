@@ -181,6 +181,9 @@ struct Ctx {
     std::vector<Seq> seqs;
     std::unordered_map<void *, uint64_t> allocs;
     uint64_t vram_used = 0, vram_limit = 0;
+    // a weight copy (GpuMat::w16, st, wx; F5Conv::wx) found no room: no more are made until the limit changes or a matrix is
+    // freed, so that a call does not try again each time
+    bool copies_off = false;
     voxhip_stats stats{};
     std::string last_error;
     bool warned = false;
@@ -238,6 +241,7 @@ void *dalloc(size_t bytes) {
                    " MiB requested");
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();  // the failure is reported here, not by the next launch
     if (e != hipSuccess) throw Fail(std::string("hipMalloc of ") + std::to_string(bytes >> 20) + " MiB failed: " + hipGetErrorString(e));
     g.allocs[p] = bytes;
     g.vram_used += bytes;
@@ -251,6 +255,16 @@ void dfree(void *p) {
 }
 template <class T>
 T *dalloc_t(size_t n) { return static_cast<T *>(dalloc(n * sizeof(T))); }
+// Room for a weight copy, or null. The copies only make products faster: without one they read the weights as stored.
+void *dalloc_copy(size_t bytes) {
+    if (g.copies_off) return nullptr;
+    try {
+        return dalloc(bytes);
+    } catch (const Fail &) {
+        g.copies_off = true;
+        return nullptr;
+    }
+}
 
 float *pinned(size_t bytes) {
     if (g.pin_bytes < bytes) {
@@ -379,18 +393,12 @@ float host_absmax(const float *w, size_t n) {
     return mx;
 }
 
-// The layout of F32 weights that k_gemm_x3p reads (rows of K weights per group, one group after the other), or null when
-// it cannot be allocated: the products then keep k_gemm_x3. Not during a capture.
+// The layout of F32 weights that k_gemm_x3p reads (rows of K weights per group, one group after the other), or null without
+// room: the products then keep k_gemm_x3. Not during a capture.
 void *pack_x3(const float *w, int64_t rows, int64_t K, int groups, hipStream_t s) {
     const int64_t one = vh::pack_x3_bytes(rows, K);
-    uint8_t *p = nullptr;
-    try {
-        p = static_cast<uint8_t *>(dalloc(size_t(one * groups)));
-    } catch (const Fail &) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    for (int i = 0; i < groups; ++i) {
+    uint8_t *p = static_cast<uint8_t *>(dalloc_copy(size_t(one * groups)));
+    for (int i = 0; p && i < groups; ++i) {
         const hipError_t e = vh::launch_pack_x3(w + int64_t(i) * rows * K, rows, K, p + one * i, s);
         if (e != hipSuccess) {
             dfree(p);
@@ -826,13 +834,9 @@ bool planes_layer(const Xfmr &X, int li, int64_t m_total, int mc, bool need_read
 void prepare_w16(GpuMat &m, hipStream_t s) {
     if (m.w16) return;
     const bool q8 = m.type == VOXHIP_Q8;
-    _Float16 *w16 = nullptr;
-    float *st = nullptr;
-    try {
-        w16 = dalloc_t<_Float16>(size_t(pack_f16_halves(m.rows, m.cols)));
-        if (q8) st = dalloc_t<float>(size_t(scale_t_floats(m.rows, m.cols)));
-    } catch (const Fail &) {
-        (void)hipGetLastError();  // a failed hipMalloc leaves its error for the next query
+    _Float16 *w16 = static_cast<_Float16 *>(dalloc_copy(size_t(pack_f16_halves(m.rows, m.cols)) * sizeof(_Float16)));
+    float *st = w16 && q8 ? static_cast<float *>(dalloc_copy(size_t(scale_t_floats(m.rows, m.cols)) * sizeof(float))) : nullptr;
+    if (!w16 || (q8 && !st)) {
         dfree(w16);
         return;
     }
@@ -845,6 +849,27 @@ void prepare_w16(GpuMat &m, hipStream_t s) {
     }
     m.w16 = w16;
     m.st = st;
+}
+// The same for all of a model's matrices: without room for every one, those just made go back.
+bool prepare_w16_all(const std::vector<int> &ids, hipStream_t s) {
+    std::vector<int> made;
+    for (int id : ids) {
+        GpuMat &m = g.mats[size_t(id)];
+        if (m.w16) continue;
+        prepare_w16(m, s);
+        if (m.w16) {
+            made.push_back(id);
+            continue;
+        }
+        HIPCHECK(hipStreamSynchronize(s));
+        for (int k : made) {
+            GpuMat &d = g.mats[size_t(k)];
+            dfree(d.w16); dfree(d.st);
+            d.w16 = nullptr; d.st = nullptr;
+        }
+        return false;
+    }
+    return true;
 }
 // Lays out what a pass of mc rows reads, before its launches are enqueued or captured: every entry point does it before every
 // pass, so that a call's kernels do not depend on the calls before it. One matrix; then the matrices of layers first ..
@@ -1411,6 +1436,7 @@ const char *voxhip_last_error(void) {
 void voxhip_set_vram_limit(uint64_t bytes) {
     std::lock_guard<std::mutex> lk(g.mu);
     g.vram_limit = bytes;
+    g.copies_off = false;
 }
 void voxhip_mem_info_get(voxhip_mem_info *out) {
     std::lock_guard<std::mutex> lk(g.mu);
@@ -2303,6 +2329,14 @@ struct F5 {
     _Float16 *nrm16 = nullptr, *at16 = nullptr, *ffb16 = nullptr;
 };
 
+// The convolutions on the conv GEMM.
+template <class Fn>
+void each_conv(F5 &F, Fn fn) {
+    fn(F.pos1);
+    fn(F.pos2);
+    if (F.vdim) fn(F.v_embed);
+}
+
 F5 &f5_at(int id) {
     if (id < 0 || size_t(id) >= g.f5.size() || !g.f5[size_t(id)]) throw Fail("bad F5 handle " + std::to_string(id));
     return *g.f5[size_t(id)];
@@ -2439,12 +2473,14 @@ F5Conv upload_conv_gemm(const voxhip_f5_conv &c, const char *what) {
     d.wide = f32_wide(host_absmax(w.data(), w.size()));
     d.w = dalloc_t<float>(w.size());
     h2d(d.w, w.data(), w.size() * 4);
-    if (!d.wide) d.wx = pack_x3(d.w, cog, d.kpad, c.groups, g.stream);
     if (c.b) {
         d.b = dalloc_t<float>(size_t(c.cout));
         h2d(d.b, c.b, size_t(c.cout) * 4);
     }
     return d;
+}
+void prepare_conv(F5Conv &c, hipStream_t s) {
+    if (!c.wide && !c.wx) c.wx = pack_x3(c.w, c.cout / c.groups, c.kpad, c.groups, s);
 }
 F5Conv upload_conv(const voxhip_f5_conv &c, int dim) {
     if (c.cin != dim || c.cout != dim) throw Fail("F5 position convolution: cin = cout = dim");
@@ -2602,15 +2638,6 @@ int voxhip_f5_create(const voxhip_f5_desc *d) {
         } catch (const Fail &) {
             F->ada_all = -1;
         }
-        F->split = D % 64 == 0 && FF % 64 == 0;  // the attention width (heads x 64) always is
-        for (const F5Block &fb : F->blocks)
-            for (int id : {fb.qkv, fb.o, fb.ff1, fb.ff2}) F->split = F->split && mat_at(id).type == VOXHIP_F16;
-        if (F->split)
-            for (const F5Block &fb : F->blocks)
-                for (int id : {fb.qkv, fb.o, fb.ff1, fb.ff2}) {
-                    prepare_w16(mat_at(id), g.stream);
-                    F->split = F->split && mat_at(id).w16;
-                }
         F->pos1 = upload_conv(d->pos1, D);
         F->pos2 = upload_conv(d->pos2, D);
         if (d->vocos_dim > 0) {  // Vocos (f5.cpp:333-346): the linears are matrix handles, the rest host arrays
@@ -2638,11 +2665,17 @@ int voxhip_f5_create(const voxhip_f5_desc *d) {
             }
             F->vdim = VD; F->vinter = VI; F->vout = VO; F->v_head = d->v_head;
         }
-        std::vector<int> ids{F->in_proj, F->proj_out};  // the linears that multiply rows, where they are F32
+        bool planes = D % 64 == 0 && FF % 64 == 0;  // the attention width (heads x 64) always is
+        std::vector<int> ids;
         for (const F5Block &fb : F->blocks) ids.insert(ids.end(), {fb.qkv, fb.o, fb.ff1, fb.ff2});
+        for (int id : ids) planes = planes && mat_at(id).type == VOXHIP_F16;
+        // weight copies last: they take the room that is left
+        F->split = planes && prepare_w16_all(ids, g.stream);
+        ids.insert(ids.end(), {F->in_proj, F->proj_out});
         for (const F5VBlock &vb : F->vblocks) ids.insert(ids.end(), {vb.pw1, vb.pw2});
         if (F->vdim) ids.push_back(F->v_head);
-        for (int id : ids) prepare_x3(mat_at(id), g.stream);
+        for (int id : ids) prepare_x3(mat_at(id), g.stream);  // the linears that multiply rows, where they are F32
+        each_conv(*F, [](F5Conv &c) { prepare_conv(c, g.stream); });
         g.f5.push_back(F.release());
         return int(g.f5.size()) - 1;
     }, -1);
@@ -2801,6 +2834,19 @@ struct Cosy {
     hipGraphExec_t step_graph = nullptr;
 };
 
+template <class Fn>
+void each_conv(Cosy &E, Fn fn) {
+    auto res = [&](CosyRes &r) {
+        fn(r.c1);
+        fn(r.c2);
+        fn(r.res);
+    };
+    res(E.down_res);
+    res(E.up_res);
+    for (CosyRes &r : E.mid_res) res(r);
+    for (F5Conv *c : {&E.down_conv, &E.up_out, &E.final_conv, &E.final_proj}) fn(*c);
+}
+
 Cosy &cosy_at(int id) {
     if (id < 0 || size_t(id) >= g.cosy.size() || !g.cosy[size_t(id)]) throw Fail("bad flow estimator handle " + std::to_string(id));
     return *g.cosy[size_t(id)];
@@ -2849,7 +2895,6 @@ CosyX cosy_x_up(const voxhip_cosy_x &x, int C, int heads, int hd) {
     o.qkv = stack_rows_heads({x.q, x.k, x.v}, heads, hd, kF5HeadDim);
     o.o = pad_head_cols(x.o, heads, hd, kF5HeadDim);
     o.ff1 = x.ff1; o.ff2 = x.ff2; o.ff = x.ff_dim;
-    for (int id : {o.qkv, o.o, o.ff1, o.ff2}) prepare_x3(mat_at(id), g.stream);  // where they are F32
     return o;
 }
 
@@ -2992,41 +3037,26 @@ int voxhip_cosy_create(const voxhip_cosy_desc *d) {
         E->final_proj = cosy_conv_up(d->final_proj, C, M, true, "final_proj");
         E->fn_w = upload_vec(d->fn_w, C, "final block norm weight");
         E->fn_b = upload_vec(d->fn_b, C, "final block norm bias");
-        bool split = C % 64 == 0 && E->inner % 64 == 0;
-        for (const auto *v : {&E->down_x, &E->up_x})
-            for (const CosyX &x : *v) split = split && x.ff % 64 == 0;
-        for (const auto &v : E->mid_x)
-            for (const CosyX &x : v) split = split && x.ff % 64 == 0;
-        auto all_f16 = [&](const std::vector<CosyX> &v) {
-            for (const CosyX &x : v)
-                for (int id : {x.qkv, x.o, x.ff1, x.ff2})
-                    if (mat_at(id).type != VOXHIP_F16) return false;
-            return true;
+        bool planes = C % 64 == 0 && E->inner % 64 == 0;
+        std::vector<int> ids;
+        auto add = [&](const std::vector<CosyX> &v) {
+            for (const CosyX &x : v) {
+                ids.insert(ids.end(), {x.qkv, x.o, x.ff1, x.ff2});
+                planes = planes && x.ff % 64 == 0;
+            }
         };
-        split = split && all_f16(E->down_x) && all_f16(E->up_x);
-        for (const auto &v : E->mid_x) split = split && all_f16(v);
-        auto prepare = [&](const std::vector<CosyX> &v) {
-            for (const CosyX &x : v)
-                for (int id : {x.qkv, x.o, x.ff1, x.ff2})
-                    if (split) {
-                        prepare_w16(mat_at(id), g.stream);
-                        split = split && mat_at(id).w16;
-                    }
-        };
-        prepare(E->down_x);
-        prepare(E->up_x);
-        for (const auto &v : E->mid_x) prepare(v);
-        E->split = split;
-        if (split && C == 256) try {
-            E->tail_ws = dalloc_t<float>(size_t(block_tail_ws()));
-            E->tail_count = dalloc_t<int32_t>(size_t(block_tail_counts()));
-            HIPCHECK(hipMemset(E->tail_count, 0, size_t(block_tail_counts()) * sizeof(int32_t)));  // each launch leaves them zero
-        } catch (const Fail &) {  // no room: one block per 16 rows
-            (void)hipGetLastError();
-            dfree(E->tail_ws);
-            dfree(E->tail_count);
-            E->tail_ws = nullptr;
-            E->tail_count = nullptr;
+        add(E->down_x);
+        add(E->up_x);
+        for (const auto &v : E->mid_x) add(v);
+        for (int id : ids) planes = planes && mat_at(id).type == VOXHIP_F16;
+        // weight copies last: they take the room that is left
+        E->split = planes && prepare_w16_all(ids, g.stream);
+        for (int id : ids) prepare_x3(mat_at(id), g.stream);  // where they are F32
+        each_conv(*E, [](F5Conv &c) { prepare_conv(c, g.stream); });
+        if (E->split && C == 256) {  // without room: one block per 16 rows
+            E->tail_ws = static_cast<float *>(dalloc_copy(size_t(block_tail_ws()) * sizeof(float)));
+            E->tail_count = static_cast<int32_t *>(dalloc_copy(size_t(block_tail_counts()) * sizeof(int32_t)));
+            if (E->tail_count) HIPCHECK(hipMemset(E->tail_count, 0, size_t(block_tail_counts()) * sizeof(int32_t)));  // each launch leaves them zero
         }
         g.cosy.push_back(E.release());
         return int(g.cosy.size()) - 1;
@@ -3688,6 +3718,7 @@ int voxhip_mat_free(int mat) {
         for (Xfmr *X : g.xf)
             if (X) drop_graphs(*X);
         free_mat(mat);
+        g.copies_off = false;
         return 1;
     }, 0);
 }
