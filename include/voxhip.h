@@ -87,7 +87,11 @@ void voxhip_stats_get(voxhip_stats *out);                  /* gpu_stats (gpu.hpp
 /* GpuStats::last_error (gpu.hpp:16): copied under the library lock into a buffer of the calling thread, valid
  * until that thread's next voxhip_last_error call (a failure on another thread cannot change it). */
 const char *voxhip_last_error(void);
-void voxhip_set_vram_limit(uint64_t bytes);                /* gpu_set_vram_limit (gpu.hpp:34) */
+/* gpu_set_vram_limit (gpu.hpp:34). Beside the matrices the library keeps copies of some weights in the order its matrix-core
+ * kernels read them, and counts them as used. They only take room that nothing else needs: an allocation that finds none
+ * (the limit, or the device's memory) takes theirs, and the products then read the weights as stored, more slowly, until the
+ * limit is set again or a matrix is freed. */
+void voxhip_set_vram_limit(uint64_t bytes);
 void voxhip_mem_info_get(voxhip_mem_info *out);            /* gpu_mem_info (gpu.hpp:36) */
 
 /* ---------------------------------------------------------------- matrices */

@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 from conftest import rel_err
-from models import F16, CosyModel, F5Model
+import pyoracle as po
+from models import F16, CodecModel, CosyModel, F5Model, Model
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +95,71 @@ def test_create_gives_back_copies_that_do_not_all_fit(hip, oracle, limit, kind):
     c.begin(hip, h, oracle)
     c.step(hip, h)
     c.end(hip, h)
+
+
+@pytest.mark.parametrize("kind", [Dit, Flow])
+def test_begin_takes_the_room_of_copies(hip, oracle, limit, kind):
+    # a limit under which create finds room for every copy, and begin's buffers only in their place
+    c = kind()
+    used = hip.mem_info().used
+    h = c.create(hip)
+    whole = hip.mem_info().used - used
+    c.begin(hip, h, oracle)
+    c.step(hip, h)
+    c.end(hip, h)
+    limit(whole + (1 << 19))
+    h = c.create(hip)
+    full = hip.mem_info().used
+    c.begin(hip, h, oracle)
+    assert hip.mem_info().used < full - c.linears // 2
+    first = c.step(hip, h)
+    assert np.array_equal(c.step(hip, h), first)
+    c.end(hip, h)
+    hip.lib().voxhip_set_vram_limit(0)  # room again: the next begin lays the weights out again
+    used = hip.mem_info().used
+    c.begin(hip, h, oracle)
+    assert hip.mem_info().used > used + c.linears
+    c.step(hip, h)
+    c.end(hip, h)
+
+
+def test_allocation_takes_the_room_of_copies_in_use(hip, oracle, limit):
+    # models with a begun step, captured graphs and states: an allocation that needs their copies' room gets it, and they go on
+    dit, flow = Dit(), Flow()
+    hd, hf = dit.create(hip), flow.create(hip)
+    dit.begin(hip, hd, oracle)
+    flow.begin(hip, hf, oracle)
+    lm = Model(72, 2, 512, 8, 2, 64, 1024, wtype=F16, head_rows=96)
+    xf, head = hip.xfmr_create(lm.hx, "copies"), hip.upload(lm.head[1])
+    seq = hip.seq_create(xf, 64)
+    x = np.random.default_rng(5).standard_normal((20, 512)).astype(np.float32)
+    dec = CodecModel(73)
+    codec = dec.create(hip)
+    z = (np.random.default_rng(6).standard_normal((8, dec.cc["codebook_dim"])) * 0.5).astype(np.float32)
+    pcm = po.codec_forward(po.CodecState(dec.ox, 64), z)
+
+    def all_steps(st):
+        dit.step(hip, hd)
+        flow.step(hip, hf)
+        out, logits = hip.forward(xf, seq, 0, x, 512, head=head)
+        assert rel_err(out, oracle.transformer_forward(lm.ox, lm.oracle_kv(64), x)) < 1e-3
+        got = np.concatenate([hip.codec_forward(codec, st, z[i:i + 2]) for i in (0, 2, 4, 6)])
+        assert rel_err(got, pcm) < 1e-4, rel_err(got, pcm)
+    st = [hip.codec_state_new(codec) for _ in range(2)]
+    for _ in range(3):  # eager, captured, replayed
+        dit.step(hip, hd)
+        flow.step(hip, hf)
+        hip.forward(xf, seq, 0, x, 512, head=head)
+    all_steps(st[0])
+    limit(1 << 19)
+    used = hip.mem_info().used
+    big = hip.DevBuf(dit.linears + flow.linears)  # fits in the copies' place alone
+    assert hip.mem_info().used < used + (1 << 19)
+    all_steps(st[1])
+    with pytest.raises(hip.VoxHipError, match="VRAM limit"):
+        hip.DevBuf(64 << 20)  # nothing left to give back
+    big.free()
+    dit.end(hip, hd)
+    flow.end(hip, hf)
+    for s in st:
+        hip.codec_state_free(s)

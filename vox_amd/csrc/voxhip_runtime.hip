@@ -181,8 +181,8 @@ struct Ctx {
     std::vector<Seq> seqs;
     std::unordered_map<void *, uint64_t> allocs;
     uint64_t vram_used = 0, vram_limit = 0;
-    // a weight copy (GpuMat::w16, st, wx; F5Conv::wx) found no room: no more are made until the limit changes or a matrix is
-    // freed, so that a call does not try again each time
+    // a weight copy (GpuMat::w16, st, wx; F5Conv::wx) found no room, or all went for something required: no more are made until
+    // the limit changes or a matrix is freed, so that calls do not make and drop them in turn
     bool copies_off = false;
     voxhip_stats stats{};
     std::string last_error;
@@ -233,19 +233,30 @@ int32_t *status_word() { return g.status_dev; }
 namespace {
 
 // ------------------------------------------------------------------ device memory with accounting
-void *dalloc(size_t bytes) {
+// Gives back every weight copy (below, with the objects that read them): whether there was one.
+bool release_copies();
+
+// required: what a call cannot do without; the weight copies make room for it.
+void *dalloc(size_t bytes, bool required = true) {
     if (bytes == 0) bytes = 16;
-    if (g.vram_limit && g.vram_used + bytes > g.vram_limit)
-        throw Fail("VRAM limit reached: " + std::to_string(g.vram_limit >> 20) + " MiB allowed, " +
-                   std::to_string(g.vram_used >> 20) + " MiB in use, " + std::to_string((bytes + (1u << 20) - 1) >> 20) +
-                   " MiB requested");
-    void *p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) (void)hipGetLastError();  // the failure is reported here, not by the next launch
-    if (e != hipSuccess) throw Fail(std::string("hipMalloc of ") + std::to_string(bytes >> 20) + " MiB failed: " + hipGetErrorString(e));
-    g.allocs[p] = bytes;
-    g.vram_used += bytes;
-    return p;
+    for (;;) {
+        std::string why;
+        if (g.vram_limit && g.vram_used + bytes > g.vram_limit) {
+            why = "VRAM limit reached: " + std::to_string(g.vram_limit >> 20) + " MiB allowed, " +
+                  std::to_string(g.vram_used >> 20) + " MiB in use, " + std::to_string((bytes + (1u << 20) - 1) >> 20) + " MiB requested";
+        } else {
+            void *p = nullptr;
+            const hipError_t e = hipMalloc(&p, bytes);
+            if (e == hipSuccess) {
+                g.allocs[p] = bytes;
+                g.vram_used += bytes;
+                return p;
+            }
+            (void)hipGetLastError();  // the failure is reported here, not by the next launch
+            why = std::string("hipMalloc of ") + std::to_string(bytes >> 20) + " MiB failed: " + hipGetErrorString(e);
+        }
+        if (!required || !release_copies()) throw Fail(why);
+    }
 }
 void dfree(void *p) {
     if (!p) return;
@@ -259,7 +270,7 @@ T *dalloc_t(size_t n) { return static_cast<T *>(dalloc(n * sizeof(T))); }
 void *dalloc_copy(size_t bytes) {
     if (g.copies_off) return nullptr;
     try {
-        return dalloc(bytes);
+        return dalloc(bytes, false);
     } catch (const Fail &) {
         g.copies_off = true;
         return nullptr;
@@ -1436,7 +1447,11 @@ const char *voxhip_last_error(void) {
 void voxhip_set_vram_limit(uint64_t bytes) {
     std::lock_guard<std::mutex> lk(g.mu);
     g.vram_limit = bytes;
+    if (!g.copies_off) return;
     g.copies_off = false;
+    if (hipStreamSynchronize(g.stream) != hipSuccess) return;
+    for (Xfmr *X : g.xf)
+        if (X) drop_graphs(*X);  // captured without copies
 }
 void voxhip_mem_info_get(voxhip_mem_info *out) {
     std::lock_guard<std::mutex> lk(g.mu);
@@ -2310,7 +2325,7 @@ struct F5 {
     F5Conv pos1, pos2;
     // every block linear F16 and dim, inner, ff multiples of 64: the block's activations travel between kernels as
     // f16 halves (hi, lo planes) and the linears take k_gemm_hh; otherwise f32 rows and k_gemm_h16 / k_gemm_f32
-    bool split = false;
+    bool planes = false, split = false;  // the model could; it has the copies k_gemm_hh reads
     // Vocos (vdim 0: none): embed conv, norms, blocks, head; buffers of the last vocode length vT
     int vdim = 0, vinter = 0, vout = 0, v_head = -1;
     F5Conv v_embed;
@@ -2320,13 +2335,13 @@ struct F5 {
     float *vm = nullptr, *vx = nullptr, *vy = nullptr, *vh = nullptr, *vhead = nullptr;
     // step buffers of begin(B, N): rows R = B N
     int B = 0, N = 0;
+    // nrm, at, ffb: the modulated rows, the attention output and the GELU output, as f32 rows or (split) as f16 planes; a begun
+    // step can go from split to f32 rows between two steps
     float *cat = nullptr, *h = nullptr, *a = nullptr, *nrm = nullptr, *at = nullptr, *ffb = nullptr;
     float *ada = nullptr, *fin = nullptr, *ts = nullptr, *x = nullptr, *out = nullptr, *rope = nullptr;
     // q, k and v as f16 halves (qkv_off's layout, np rows per batch and head)
     _Float16 *qkv16 = nullptr;
     int np = 0;
-    // split: the modulated rows, the attention output and the GELU output as f16 planes (R rows each)
-    _Float16 *nrm16 = nullptr, *at16 = nullptr, *ffb16 = nullptr;
 };
 
 // The convolutions on the conv GEMM.
@@ -2507,11 +2522,15 @@ float *upload_vec(const float *v, int n, const char *what) {
     return d;
 }
 
+// Room for m rows of K f32 values, or as many as f16 planes (4 bytes a value either way, the planes of whole 16 rows).
+float *rows_or_planes(int64_t m, int64_t K) { return dalloc_t<float>(size_t(planes_halves(m, K) / 2)); }
+_Float16 *planes_of(bool split, float *p) { return split ? reinterpret_cast<_Float16 *>(p) : nullptr; }
+
 void f5_free_step(F5 &F) {
     for (float *p : {F.cat, F.h, F.a, F.nrm, F.at, F.ffb, F.ada, F.ts, F.x, F.out, F.rope}) dfree(p);  // fin is in ada
     F.cat = F.h = F.a = F.nrm = F.at = F.ffb = F.ada = F.fin = F.ts = F.x = F.out = F.rope = nullptr;
-    for (_Float16 *p : {F.qkv16, F.nrm16, F.at16, F.ffb16}) dfree(p);
-    F.qkv16 = F.nrm16 = F.at16 = F.ffb16 = nullptr;
+    dfree(F.qkv16);
+    F.qkv16 = nullptr;
     F.B = F.N = F.np = 0;
 }
 
@@ -2566,34 +2585,48 @@ void f5_enqueue(F5 &F, hipStream_t s) {
         HIPCHECK(launch_conv_gemm(c == 0 ? EPI_MISH : EPI_MISH_ACC, cv.w, c == 0 ? F.h : F.a, ga, cv.groups, s));
     }
     const float scale = 1.0f / std::sqrt(float(F.hd));
+    _Float16 *nrm16 = planes_of(F.split, F.nrm), *at16 = planes_of(F.split, F.at), *ffb16 = planes_of(F.split, F.ffb);
     for (int i = 0; i < F.depth; ++i) {
         const F5Block &L = F.blocks[size_t(i)];
         const float *ada = F.ada + size_t(i) * 6 * D;  // shift, scale, gate (msa), shift, scale, gate (mlp)
         float *nrm = F.split ? nullptr : F.nrm;
-        HIPCHECK(launch_f5_modulate(F.h, R, D, ada + D, ada, nrm, F.nrm16, s));
+        HIPCHECK(launch_f5_modulate(F.h, R, D, ada + D, ada, nrm, nrm16, s));
         const GpuMat &Mq = mat_at(L.qkv);
         GemmArgs gq = gemm_args(Mq, Mq.b, nullptr, D, 3 * INNER, R);
         gq.rope = F.rope; gq.seq = F.N; gq.hd = F.hp; gq.rope_hd = F.hd; gq.rope_cols = 2 * INNER; gq.rope_heads = F.pe;
         gq.h16 = F.qkv16; gq.seq_pad = F.np;
-        f5_lin(F, Mq, EPI_ROPE_H16, F.nrm, F.nrm16, gq, s);
-        HIPCHECK(launch_f5_attn(F.qkv16, F.split ? nullptr : F.at, F.at16, F.B, F.N, F.heads, F.hp, F.np, INNER, scale, s));
+        f5_lin(F, Mq, EPI_ROPE_H16, F.nrm, nrm16, gq, s);
+        HIPCHECK(launch_f5_attn(F.qkv16, F.split ? nullptr : F.at, at16, F.B, F.N, F.heads, F.hp, F.np, INNER, scale, s));
         const GpuMat &Mo = mat_at(L.o);
         GemmArgs go = gemm_args(Mo, Mo.b, F.h, INNER, D, R);
         go.gate = ada + 2 * D;
-        f5_lin(F, Mo, EPI_GATED_ACC, F.at, F.at16, go, s);
-        HIPCHECK(launch_f5_modulate(F.h, R, D, ada + 4 * D, ada + 3 * D, nrm, F.nrm16, s));
+        f5_lin(F, Mo, EPI_GATED_ACC, F.at, at16, go, s);
+        HIPCHECK(launch_f5_modulate(F.h, R, D, ada + 4 * D, ada + 3 * D, nrm, nrm16, s));
         const GpuMat &M1 = mat_at(L.ff1), &M2 = mat_at(L.ff2);
         GemmArgs g1 = gemm_args(M1, M1.b, F.split ? nullptr : F.ffb, D, F.ff, R);
-        g1.h16 = F.ffb16;
+        g1.h16 = ffb16;
         if (F.split) g1.ldy = F.ff;
-        f5_lin(F, M1, F.split ? EPI_GELU_H16 : EPI_GELU, F.nrm, F.nrm16, g1, s);
+        f5_lin(F, M1, F.split ? EPI_GELU_H16 : EPI_GELU, F.nrm, nrm16, g1, s);
         GemmArgs g2 = gemm_args(M2, M2.b, F.h, F.ff, D, R);
         g2.gate = ada + 5 * D;
-        f5_lin(F, M2, EPI_GATED_ACC, F.ffb, F.ffb16, g2, s);
+        f5_lin(F, M2, EPI_GATED_ACC, F.ffb, ffb16, g2, s);
     }
     HIPCHECK(launch_f5_modulate(F.h, R, D, F.fin, F.fin + D, F.nrm, nullptr, s));  // final modulation: (scale, shift)
     const GpuMat &Mp = mat_at(F.proj_out);
     f5_gemm(Mp, EPI_STORE, F.nrm, gemm_args(Mp, Mp.b, F.out, D, F.mel, R), s);
+}
+
+// Lays out the weights a step and the vocoder read, as far as there is room (create and begin; nothing to do once it is done).
+void lay_out(F5 &F) {
+    if (g.copies_off) return;
+    std::vector<int> ids;
+    for (const F5Block &fb : F.blocks) ids.insert(ids.end(), {fb.qkv, fb.o, fb.ff1, fb.ff2});
+    F.split = F.planes && prepare_w16_all(ids, g.stream);
+    ids.insert(ids.end(), {F.in_proj, F.proj_out});
+    for (const F5VBlock &vb : F.vblocks) ids.insert(ids.end(), {vb.pw1, vb.pw2});
+    if (F.vdim) ids.push_back(F.v_head);
+    for (int id : ids) prepare_x3(mat_at(id), g.stream);  // the linears that multiply rows, where they are F32
+    each_conv(F, [](F5Conv &c) { prepare_conv(c, g.stream); });
 }
 }  // namespace
 
@@ -2665,17 +2698,10 @@ int voxhip_f5_create(const voxhip_f5_desc *d) {
             }
             F->vdim = VD; F->vinter = VI; F->vout = VO; F->v_head = d->v_head;
         }
-        bool planes = D % 64 == 0 && FF % 64 == 0;  // the attention width (heads x 64) always is
-        std::vector<int> ids;
-        for (const F5Block &fb : F->blocks) ids.insert(ids.end(), {fb.qkv, fb.o, fb.ff1, fb.ff2});
-        for (int id : ids) planes = planes && mat_at(id).type == VOXHIP_F16;
-        // weight copies last: they take the room that is left
-        F->split = planes && prepare_w16_all(ids, g.stream);
-        ids.insert(ids.end(), {F->in_proj, F->proj_out});
-        for (const F5VBlock &vb : F->vblocks) ids.insert(ids.end(), {vb.pw1, vb.pw2});
-        if (F->vdim) ids.push_back(F->v_head);
-        for (int id : ids) prepare_x3(mat_at(id), g.stream);  // the linears that multiply rows, where they are F32
-        each_conv(*F, [](F5Conv &c) { prepare_conv(c, g.stream); });
+        F->planes = D % 64 == 0 && FF % 64 == 0;  // the attention width (heads x 64) always is
+        for (const F5Block &fb : F->blocks)
+            for (int id : {fb.qkv, fb.o, fb.ff1, fb.ff2}) F->planes = F->planes && mat_at(id).type == VOXHIP_F16;
+        lay_out(*F);  // last: the copies take the room that is left
         g.f5.push_back(F.release());
         return int(g.f5.size()) - 1;
     }, -1);
@@ -2687,18 +2713,13 @@ int voxhip_f5_begin(int id, int B, int N, const float *cat0, const float *rope) 
         F5 &F = f5_at(id);
         if (B <= 0 || N <= 0 || !cat0 || !rope || int64_t(B) * N > INT32_MAX / 8) throw Fail("bad F5 step shape");
         f5_free_step(F);
+        lay_out(F);
         const size_t R = size_t(B) * size_t(N), D = size_t(F.dim), INNER = size_t(F.heads) * F.hp;
         const size_t W = 2 * size_t(F.mel) + F.text;
         F.cat = dalloc_t<float>(R * W); F.h = dalloc_t<float>(R * D); F.a = dalloc_t<float>(R * D);
-        F.nrm = dalloc_t<float>(R * D);
-        if (F.split) {
-            F.nrm16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(D))));
-            F.at16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(INNER))));
-            F.ffb16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), F.ff)));
-        } else {
-            F.at = dalloc_t<float>(R * INNER);
-            F.ffb = dalloc_t<float>(R * size_t(F.ff));
-        }
+        F.nrm = rows_or_planes(int64_t(R), int64_t(D));
+        F.at = rows_or_planes(int64_t(R), int64_t(INNER));
+        F.ffb = rows_or_planes(int64_t(R), F.ff);
         F.np = (N + 63) / 64 * 64;  // whole key tiles, the padding zero
         const size_t qkv = size_t(3) * size_t(B) * size_t(F.np) * INNER * 2;
         F.qkv16 = dalloc_t<_Float16>(qkv);
@@ -2819,12 +2840,13 @@ struct Cosy {
     float *fn_w = nullptr, *fn_b = nullptr;
     // every transformer linear F16 and C, inner, ff multiples of 64: the block activations travel as f16 halves
     // and the linears take k_gemm_hh; otherwise f32 rows
-    bool split = false;
-    // step buffers of begin(T): rows R = 2 T
+    bool planes = false, split = false;  // the model could; it has the copies k_gemm_hh reads
+    // step buffers of begin(T): rows R = 2 T; xn, at and ff (the normed rows, the attention output, the GELU output) as f32 rows
+    // or (split) as f16 planes
     int T = 0;
     float *in = nullptr, *a = nullptr, *b = nullptr, *h = nullptr, *cat = nullptr, *xn = nullptr, *at = nullptr,
           *ff = nullptr, *tb = nullptr, *x = nullptr, *out = nullptr;
-    _Float16 *qkv16 = nullptr, *xn16 = nullptr, *at16 = nullptr, *ff16 = nullptr;
+    _Float16 *qkv16 = nullptr;
     // launch_block_tail's partial sums and counts (split models of its width), of any step: made by create, since two more
     // allocations and a clear cost begin 0.6 ms
     float *tail_ws = nullptr;
@@ -2852,13 +2874,16 @@ Cosy &cosy_at(int id) {
     return *g.cosy[size_t(id)];
 }
 
-void cosy_free_step(Cosy &E) {
+void drop_step_graph(Cosy &E) {
     if (E.step_graph) (void)hipGraphExecDestroy(E.step_graph);
     E.step_graph = nullptr;
+}
+void cosy_free_step(Cosy &E) {
+    drop_step_graph(E);
     for (float *p : {E.in, E.a, E.b, E.h, E.cat, E.xn, E.at, E.ff, E.tb, E.x, E.out}) dfree(p);
     E.in = E.a = E.b = E.h = E.cat = E.xn = E.at = E.ff = E.tb = E.x = E.out = nullptr;
-    for (_Float16 *p : {E.qkv16, E.xn16, E.at16, E.ff16}) dfree(p);
-    E.qkv16 = E.xn16 = E.at16 = E.ff16 = nullptr;
+    dfree(E.qkv16);
+    E.qkv16 = nullptr;
     E.T = E.np = 0;
 }
 
@@ -2938,31 +2963,32 @@ void cosy_xblock(const Cosy &E, const CosyX &L, const CosyX *next, bool *normed,
     const int C = E.C, INNER = E.inner;
     const int64_t R = int64_t(2) * E.T;
     float *xn = E.split ? nullptr : E.xn;
-    if (!*normed) cosy_norm(E, A, L.n1w, L.n1b, false, nullptr, xn, E.xn16, s);
+    _Float16 *xn16 = planes_of(E.split, E.xn), *at16 = planes_of(E.split, E.at), *ff16 = planes_of(E.split, E.ff);
+    if (!*normed) cosy_norm(E, A, L.n1w, L.n1b, false, nullptr, xn, xn16, s);
     *normed = false;
     const GpuMat &Mq = mat_at(L.qkv);
     GemmArgs gq = gemm_args(Mq, Mq.b, nullptr, C, 3 * INNER, R);
     gq.rope = nullptr; gq.seq = E.T; gq.hd = kF5HeadDim; gq.rope_cols = 2 * INNER;
     gq.h16 = E.qkv16; gq.seq_pad = E.np;
-    split_lin(E.split, Mq, EPI_ROPE_H16, E.xn, E.xn16, gq, s);
-    HIPCHECK(launch_f5_attn(E.qkv16, E.split ? nullptr : E.at, E.at16, 2, E.T, E.heads, kF5HeadDim, E.np, INNER, 1.0f / std::sqrt(float(E.hd)), s));
+    split_lin(E.split, Mq, EPI_ROPE_H16, E.xn, xn16, gq, s);
+    HIPCHECK(launch_f5_attn(E.qkv16, E.split ? nullptr : E.at, at16, 2, E.T, E.heads, kF5HeadDim, E.np, INNER, 1.0f / std::sqrt(float(E.hd)), s));
     const GpuMat &Mo = mat_at(L.o), &M1 = mat_at(L.ff1), &M2 = mat_at(L.ff2);
     if (E.split && block_tail_ok(R, C, INNER, L.ff)) {
         BlockTailArgs t{};
-        t.a16 = E.at16; t.wo = Mo.w16; t.w1 = M1.w16; t.w2 = M2.w16;
+        t.a16 = at16; t.wo = Mo.w16; t.w1 = M1.w16; t.w2 = M2.w16;
         t.bo = Mo.b; t.b1 = M1.b; t.b2 = M2.b; t.lw = L.n3w; t.lb = L.n3b;
         if (next) { t.nw = next->n1w; t.nb = next->n1b; }
-        t.ws = E.tail_ws; t.count = E.tail_count; t.x = A; t.out16 = E.xn16; t.eps = double(1e-5f); t.R = int32_t(R); t.inner = INNER; t.ff = L.ff;
+        t.ws = E.tail_ws; t.count = E.tail_count; t.x = A; t.out16 = xn16; t.eps = double(1e-5f); t.R = int32_t(R); t.inner = INNER; t.ff = L.ff;
         HIPCHECK(launch_block_tail(t, s));
         *normed = next != nullptr;
         return;
     }
-    split_lin(E.split, Mo, EPI_ACC, E.at, E.at16, gemm_args(Mo, Mo.b, A, INNER, C, R), s);
-    cosy_norm(E, A, L.n3w, L.n3b, false, nullptr, xn, E.xn16, s);
+    split_lin(E.split, Mo, EPI_ACC, E.at, at16, gemm_args(Mo, Mo.b, A, INNER, C, R), s);
+    cosy_norm(E, A, L.n3w, L.n3b, false, nullptr, xn, xn16, s);
     GemmArgs g1 = gemm_args(M1, M1.b, E.split ? nullptr : E.ff, C, L.ff, R);
-    g1.h16 = E.ff16; g1.gelu_erf = 1;
-    split_lin(E.split, M1, E.split ? EPI_GELU_H16 : EPI_GELU_ERF, E.xn, E.xn16, g1, s);
-    split_lin(E.split, M2, EPI_ACC, E.ff, E.ff16, gemm_args(M2, M2.b, A, L.ff, C, R), s);
+    g1.h16 = ff16; g1.gelu_erf = 1;
+    split_lin(E.split, M1, E.split ? EPI_GELU_H16 : EPI_GELU_ERF, E.xn, xn16, g1, s);
+    split_lin(E.split, M2, EPI_ACC, E.ff, ff16, gemm_args(M2, M2.b, A, L.ff, C, R), s);
 }
 
 void cosy_xblocks(const Cosy &E, const std::vector<CosyX> &v, float *A, hipStream_t s) {
@@ -2994,6 +3020,26 @@ void cosy_enqueue(Cosy &E, hipStream_t s) {
     cosy_conv(E, E.final_conv, EPI_STORE, cur, C, oth, C, s);
     cosy_norm(E, oth, E.fn_w, E.fn_b, true, nullptr, oth, nullptr, s);
     cosy_conv(E, E.final_proj, EPI_STORE, oth, C, E.out, M, s);
+}
+
+std::vector<CosyX> cosy_blocks(const Cosy &E) {
+    std::vector<CosyX> v = E.down_x;
+    v.insert(v.end(), E.up_x.begin(), E.up_x.end());
+    for (const auto &m : E.mid_x) v.insert(v.end(), m.begin(), m.end());
+    return v;
+}
+// As lay_out(F5 &), and k_block_tail's partial sums (without them one block per 16 rows).
+void lay_out(Cosy &E) {
+    if (g.copies_off) return;
+    std::vector<int> ids;
+    for (const CosyX &x : cosy_blocks(E)) ids.insert(ids.end(), {x.qkv, x.o, x.ff1, x.ff2});
+    E.split = E.planes && prepare_w16_all(ids, g.stream);
+    for (int id : ids) prepare_x3(mat_at(id), g.stream);  // where they are F32
+    each_conv(E, [](F5Conv &c) { prepare_conv(c, g.stream); });
+    if (!E.split || E.C != 256 || E.tail_count) return;
+    if (!E.tail_ws) E.tail_ws = static_cast<float *>(dalloc_copy(size_t(block_tail_ws()) * sizeof(float)));
+    if (E.tail_ws) E.tail_count = static_cast<int32_t *>(dalloc_copy(size_t(block_tail_counts()) * sizeof(int32_t)));
+    if (E.tail_count) HIPCHECK(hipMemset(E.tail_count, 0, size_t(block_tail_counts()) * sizeof(int32_t)));  // each launch leaves them zero
 }
 }  // namespace
 
@@ -3037,27 +3083,12 @@ int voxhip_cosy_create(const voxhip_cosy_desc *d) {
         E->final_proj = cosy_conv_up(d->final_proj, C, M, true, "final_proj");
         E->fn_w = upload_vec(d->fn_w, C, "final block norm weight");
         E->fn_b = upload_vec(d->fn_b, C, "final block norm bias");
-        bool planes = C % 64 == 0 && E->inner % 64 == 0;
-        std::vector<int> ids;
-        auto add = [&](const std::vector<CosyX> &v) {
-            for (const CosyX &x : v) {
-                ids.insert(ids.end(), {x.qkv, x.o, x.ff1, x.ff2});
-                planes = planes && x.ff % 64 == 0;
-            }
-        };
-        add(E->down_x);
-        add(E->up_x);
-        for (const auto &v : E->mid_x) add(v);
-        for (int id : ids) planes = planes && mat_at(id).type == VOXHIP_F16;
-        // weight copies last: they take the room that is left
-        E->split = planes && prepare_w16_all(ids, g.stream);
-        for (int id : ids) prepare_x3(mat_at(id), g.stream);  // where they are F32
-        each_conv(*E, [](F5Conv &c) { prepare_conv(c, g.stream); });
-        if (E->split && C == 256) {  // without room: one block per 16 rows
-            E->tail_ws = static_cast<float *>(dalloc_copy(size_t(block_tail_ws()) * sizeof(float)));
-            E->tail_count = static_cast<int32_t *>(dalloc_copy(size_t(block_tail_counts()) * sizeof(int32_t)));
-            if (E->tail_count) HIPCHECK(hipMemset(E->tail_count, 0, size_t(block_tail_counts()) * sizeof(int32_t)));  // each launch leaves them zero
+        E->planes = C % 64 == 0 && E->inner % 64 == 0;
+        for (const CosyX &x : cosy_blocks(*E)) {
+            E->planes = E->planes && x.ff % 64 == 0;
+            for (int id : {x.qkv, x.o, x.ff1, x.ff2}) E->planes = E->planes && mat_at(id).type == VOXHIP_F16;
         }
+        lay_out(*E);  // last: the copies take the room that is left
         g.cosy.push_back(E.release());
         return int(g.cosy.size()) - 1;
     }, -1);
@@ -3071,19 +3102,14 @@ int voxhip_cosy_begin(int id, int T, const float *in0) {
             throw Fail("bad flow estimator length");
         HIPCHECK(hipStreamSynchronize(g.stream));
         cosy_free_step(E);
+        lay_out(E);
         const size_t R = size_t(2) * size_t(T), C = size_t(E.C), INNER = size_t(E.inner), FF = size_t(std::max(E.ffmax, 1));
         E.in = dalloc_t<float>(R * 4 * E.M);
         E.a = dalloc_t<float>(R * C); E.b = dalloc_t<float>(R * C); E.h = dalloc_t<float>(R * C);
         E.cat = dalloc_t<float>(R * 2 * C);
-        if (E.split) {
-            E.xn16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(C))));
-            E.at16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(INNER))));
-            E.ff16 = dalloc_t<_Float16>(size_t(planes_halves(int64_t(R), int64_t(FF))));
-        } else {
-            E.xn = dalloc_t<float>(R * C);
-            E.at = dalloc_t<float>(R * INNER);
-            E.ff = dalloc_t<float>(R * FF);
-        }
+        E.xn = rows_or_planes(int64_t(R), int64_t(C));
+        E.at = rows_or_planes(int64_t(R), int64_t(INNER));
+        E.ff = rows_or_planes(int64_t(R), int64_t(FF));
         E.np = (T + 63) / 64 * 64;  // whole key tiles, the padding zero
         const size_t qkv = size_t(3) * 2 * size_t(E.np) * INNER * 2;
         E.qkv16 = dalloc_t<_Float16>(qkv);
@@ -3344,6 +3370,62 @@ int64_t codec_enqueue(Codec &E, CodecSt &St, int T, hipStream_t s) {
     HIPCHECK(launch_clamp1(E.S[4], len, s));
     return len;
 }
+
+// Every product of a call takes the packed weights, as far as there is room (create and a new state; a call's launches are
+// captured).
+void lay_out(const Codec &E) {
+    if (g.copies_off) return;
+    std::vector<int> ids{E.pre_conv.mat, E.pt_in, E.pt_out, E.conv0.mat, E.fin.mat};
+    for (const LayerDev &d : xf_at(E.xf).L) ids.insert(ids.end(), {d.qkv, d.o, d.gu, d.down});
+    for (const CodecUp &u : E.ups) ids.insert(ids.end(), {u.tr, u.pw1, u.pw2});
+    for (const CodecBlk &b : E.blocks) {
+        ids.push_back(b.tr);
+        for (int u = 0; u < 3; ++u) ids.insert(ids.end(), {b.c1[u].mat, b.c2[u].mat});
+    }
+    for (int id : ids) prepare_x3(mat_at(id), g.stream);
+}
+
+// After the work in flight, every copy and every graph that may read one; models go on with the weights as stored. The copies
+// are read by g.stream's work and this library's graphs only (the no-alloc call, whose launches a caller may capture, never
+// reads one), and no caller of dalloc holds one across the call. Not during a capture.
+bool release_copies() {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (!g.ok || hipStreamIsCapturing(g.stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
+    if (hipStreamSynchronize(g.stream) != hipSuccess) return false;
+    bool any = false;
+    auto drop = [&](auto *&p) {
+        any = any || p;
+        dfree(p);
+        p = nullptr;
+    };
+    for (Xfmr *X : g.xf)
+        if (X) drop_graphs(*X);
+    for (CodecSt *S : g.cstates) {
+        if (!S) continue;
+        for (auto &kv : S->graphs) (void)hipGraphExecDestroy(kv.second);
+        S->graphs.clear();
+    }
+    for (F5 *F : g.f5) {
+        if (!F) continue;
+        F->split = false;
+        each_conv(*F, [&](F5Conv &c) { drop(c.wx); });
+    }
+    for (Cosy *E : g.cosy) {
+        if (!E) continue;
+        drop_step_graph(*E);
+        E->split = false;
+        each_conv(*E, [&](F5Conv &c) { drop(c.wx); });
+        drop(E->tail_ws);
+        drop(E->tail_count);
+    }
+    for (GpuMat &m : g.mats) {
+        drop(m.w16);
+        drop(m.st);
+        drop(m.wx);
+    }
+    g.copies_off = true;
+    return any;
+}
 }  // namespace
 
 namespace {
@@ -3487,15 +3569,7 @@ int voxhip_codec_create(const voxhip_codec_desc *d) {
         E->pre = dalloc_t<float>(F * size_t(std::max(E->H, E->I)));
         E->rope = dalloc_t<float>(F * size_t(E->hd));
         E->z = dalloc_t<float>(F * size_t(E->cdim));
-        // every product of a call takes the packed weights (its launches are captured: nothing is laid out later)
-        std::vector<int> ids{E->pre_conv.mat, E->pt_in, E->pt_out, E->conv0.mat, E->fin.mat};
-        for (const LayerDev &d : xf_at(E->xf).L) ids.insert(ids.end(), {d.qkv, d.o, d.gu, d.down});
-        for (const CodecUp &u : E->ups) ids.insert(ids.end(), {u.tr, u.pw1, u.pw2});
-        for (const CodecBlk &b : E->blocks) {
-            ids.push_back(b.tr);
-            for (int u = 0; u < 3; ++u) ids.insert(ids.end(), {b.c1[u].mat, b.c2[u].mat});
-        }
-        for (int id : ids) prepare_x3(mat_at(id), g.stream);
+        lay_out(*E);  // last: the copies take the room that is left
         g.codecs.push_back(E.release());
         return int(g.codecs.size()) - 1;
     }, -1);
@@ -3514,6 +3588,7 @@ int voxhip_codec_state_new(int codec) {
     return guard_int([&] {
         require_ok();
         const Codec &E = codec_at(codec);
+        lay_out(E);
         std::unique_ptr<CodecSt> S(new CodecSt());
         S->codec = codec;
         S->pre = hist_new((E.pre_conv.K - 1) * E.pre_conv.dil, E.pre_conv.cin);
