@@ -716,11 +716,15 @@ void ensure_rows(Xfmr &X, int rows) {
     if (X.cap_rows >= rows) return;
     if (X.cap_rows) HIPCHECK(hipStreamSynchronize(g.stream));
     drop_graphs(X);
-    for (float *p : {X.h, X.qkv, X.q, X.g, X.xnorm, X.pre, X.pm, X.pl, X.po}) dfree(p);
-    dfree(X.pa16); dfree(X.pb16);
-    dfree(X.rows_dev); dfree(X.scfg_dev); dfree(X.token_dev);
+    auto drop = [](auto *&p) { dfree(p); p = nullptr; };
+    for (float **p : {&X.h, &X.qkv, &X.q, &X.g, &X.xnorm, &X.pre, &X.pm, &X.pl, &X.po}) drop(*p);
+    drop(X.pa16); drop(X.pb16);
+    drop(X.rows_dev); drop(X.scfg_dev); drop(X.token_dev);
     if (X.rows_host) (void)hipHostFree(X.rows_host);
     if (X.scfg_host) (void)hipHostFree(X.scfg_host);
+    X.rows_host = nullptr;
+    X.scfg_host = nullptr;
+    X.cap_rows = 0;  // until every buffer is there: an allocation below may throw
     const size_t M = size_t(rows), qd = size_t(X.heads) * X.hd, kd = size_t(X.kvh) * X.hd;
     X.h = dalloc_t<float>(M * X.H);
     X.qkv = dalloc_t<float>(M * (qd + 2 * kd));
@@ -749,6 +753,8 @@ float *ensure_logits(Xfmr &X, int64_t elems) {
     if (X.logits_elems < elems) {
         HIPCHECK(hipStreamSynchronize(g.stream));
         dfree(X.logits);
+        X.logits = nullptr;
+        X.logits_elems = 0;
         X.logits = dalloc_t<float>(size_t(elems));
         X.logits_elems = elems;
         drop_graphs(X);
@@ -759,6 +765,8 @@ float *ensure_xin(Xfmr &X, int64_t elems) {
     if (X.xin_elems < elems) {
         HIPCHECK(hipStreamSynchronize(g.stream));
         dfree(X.xin);
+        X.xin = nullptr;
+        X.xin_elems = 0;
         X.xin = dalloc_t<float>(size_t(elems));
         X.xin_elems = elems;
         drop_graphs(X);  // a captured frame loop reads the old input buffer
@@ -1077,6 +1085,7 @@ RowRef row_of(const Seq &S, int64_t pos) {
 void check_seq_for(Xfmr &X, int xid, const Seq &S) {
     if (S.xfmr != xid && (S.layers < X.layers || S.kvh != X.kvh || S.hd != X.hd)) throw Fail("sequence belongs to another transformer shape");
     ensure_rope(X, S.cap);  // the RoPE table must cover every position the sequence can hold
+    ensure_rows(X, kMaxM);  // there since the create, unless a growth found no room
 }
 
 // Generic host-pointer forward for up to any m rows of one sequence (or B rows of B sequences).
@@ -1753,6 +1762,8 @@ int voxhip_sample_logits(const float *logits, int32_t n, const voxhip_sample_cfg
         }
         if (n_history > 0 && size_t(n_history) > g.hist_cap) {
             dfree(g.hist_dev);
+            g.hist_dev = nullptr;
+            g.hist_cap = 0;
             g.hist_dev = dalloc_t<int32_t>(size_t(n_history));
             g.hist_cap = size_t(n_history);
         }
@@ -2017,6 +2028,8 @@ void lm_buffers(Xfmr &X, int64_t max_len, int64_t V, bool want_logp) {
     if (X.lm_dec_cap < max_len) {
         HIPCHECK(hipStreamSynchronize(g.stream));
         dfree(X.lm_dec);
+        X.lm_dec = nullptr;
+        X.lm_dec_cap = 0;
         X.lm_dec = dalloc_t<int32_t>(size_t(max_len));
         X.lm_dec_cap = max_len;
         changed = true;
@@ -2024,6 +2037,8 @@ void lm_buffers(Xfmr &X, int64_t max_len, int64_t V, bool want_logp) {
     if (want_logp && X.lm_logp_cap < max_len * V) {
         HIPCHECK(hipStreamSynchronize(g.stream));
         dfree(X.lm_logp);
+        X.lm_logp = nullptr;
+        X.lm_logp_cap = 0;
         X.lm_logp = dalloc_t<float>(size_t(max_len * V));
         X.lm_logp_cap = max_len * V;
         changed = true;
@@ -2763,7 +2778,11 @@ int voxhip_f5_vocos(int id, const float *mel, int T, float *head) {
         const int VD = F.vdim;
         if (F.vT < T) {
             HIPCHECK(hipStreamSynchronize(g.stream));
-            for (float *p : {F.vm, F.vx, F.vy, F.vh, F.vhead}) dfree(p);
+            for (float **p : {&F.vm, &F.vx, &F.vy, &F.vh, &F.vhead}) {
+                dfree(*p);
+                *p = nullptr;
+            }
+            F.vT = 0;  // until every buffer is there: an allocation below may throw
             F.vm = dalloc_t<float>(size_t(T) * F.mel); F.vx = dalloc_t<float>(size_t(T) * VD); F.vy = dalloc_t<float>(size_t(T) * VD);
             F.vh = dalloc_t<float>(size_t(T) * F.vinter); F.vhead = dalloc_t<float>(size_t(T) * F.vout);
             F.vT = T;
