@@ -1,5 +1,5 @@
 """The F32-weight GEMM on packed split-f16 weights (k_gemm_x3p) through matmul, at the edges of its tiles and plans:
-64 x 64 and 64 x 96 tiles on full grids, 32 x 64 and 32 x 32 below, K slices and their reduce, ragged rows, columns and
+64 x 64 tiles on full grids, 32 x 64 and 32 x 32 below, K slices and their reduce, ragged rows, columns and
 K (whose padding holds zeros)."""
 import numpy as np
 import pytest
@@ -49,7 +49,7 @@ def test_matmul_f32_long_k(hip, m, n, K):
 
 
 def test_codec_96_channels(hip, oracle):
-    # a decoder whose last block has 96 channels at 6,656 rows a call: its convolutions fill the CUs with 64 x 96 tiles, the
+    # a decoder whose last block has 96 channels at 6,656 rows a call: its convolutions fill the CUs with 64 x 64 tiles, the
     # first block of tiles of each reads the history
     cc = dict(models.CODEC_TINY, decoder_dim=384, upsample_rates=[8, 13])
     m = models.CodecModel(77, cc)
@@ -61,6 +61,32 @@ def test_codec_96_channels(hip, oracle):
         got, want = hip.codec_forward(codec, st, z), po.codec_forward(ost, z)
         assert rel_err(got, want) < 1e-3, rel_err(got, want)
     hip.codec_state_free(st)
+
+
+@pytest.mark.parametrize("cols", [68, 96, 100])
+def test_conv_tiles_ragged_in_columns(hip, oracle, cols):
+    # a DiT step whose grouped position convolutions fill the CUs (832 rows, 8 groups of `cols` channels) with 64 x 64 tiles whose
+    # last columns are padding. Tolerance: 8 products in a chain, the longest sum 800 terms, roots of squares added, sqrt(8 x
+    # 800) 2^-24 = 4.8e-6, three times that. An oracle that has lost the weights' lo halves in those convolutions is beyond it.
+    tol = 1.5e-5
+
+    def model(lossy):
+        m = models.F5Model(50 + cols, 8 * cols, 1, 1, ff_mult=1, K=3, groups=8, wtype=models.F32)
+        if lossy:
+            m.ox = po.F5(m.dim, 1, 1, 64, 1, m.mel, m.text, m.pe, *(po.Mat(*m.mats[k]) for k in ("in_proj", "norm_out", "proj_out")),
+                         [{k: po.Mat(*v) for k, v in b.items()} for b in m.blocks],
+                         *(po.Conv((c[0] * 1024).astype(np.float16).astype(np.float32) / 1024, *c[1:]) for c in m.pos))
+        return m
+    m = model(False)
+    h = m.create(hip)
+    cat0, x, ts, rope = m.inputs(np.random.default_rng(cols), 1, 832)
+    hip.f5_begin(h, 1, 832, cat0, rope)
+    got = hip.f5_step(h, x, ts, 1, 832, m.mel)
+    hip.f5_end(h)
+    want = oracle.f5_step(m.ox, 1, 832, m.with_x(cat0, x, 1), ts, rope)
+    lost = oracle.f5_step(model(True).ox, 1, 832, m.with_x(cat0, x, 1), ts, rope)
+    assert rel_err(lost, want) > 2 * tol, rel_err(lost, want)
+    assert rel_err(got, want) < tol, rel_err(got, want)
 
 
 def test_overflow_flag(hip):

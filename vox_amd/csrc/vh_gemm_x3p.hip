@@ -27,8 +27,8 @@ static bool x3p_ok(int asrc, const GemmArgs &g) {
 
 // The block tile and the K slices of a product, from its count of tiles:
 // - 200 tiles of 64 x 64 or more fill the 256 CUs: 64 x 64 of 8 waves (2560 x 384, K 2688: 31.8 us against 52 with 4
-//   waves and 46 with 64 x 96 of 4 waves); 64 x 96 where n is an odd multiple of 96 up to 96 itself (30720 x 96, K 672:
-//   24.6 against 31.3 us, a third of the second 64-column tile being padding).
+//   waves and 46 with 64 x 96 of 4 waves; also where 64 x 96 would pad a third less: 30720 x 96 in the codec, K 672 34.5 against
+//   38.4 us, K 96 17.0 against 21.1; 3840 x 80 x 8 groups, K 560 42.1 against 49.4).
 // - below that 32 x 64 tiles of 8 waves: 333 x 64 x 16 groups, K 1984: 16.9 against 23.4 us; 1024 x 256, K 768: 8.4
 //   against 10.2 us. From 100 of them on a K below 2048 is not split (1920 x 96, K 672, 120 tiles: 7.5 us against 8.9 with 2
 //   slices and their reduce).
@@ -45,13 +45,13 @@ static bool x3p_ok(int asrc, const GemmArgs &g) {
 //   (64 x 6144, K 5376: 40.4 against 45.2 unsplit; at K 2048 23.2 against 21.8). Odd counts of row tiles: two slices of 32 x 64
 //   up to 128 tiles from K 2048 (400 x 512, K 5376: 29.5 us, unsplit 45.3, k_gemm_x3 31.2; K 2048: 16.6, 19.5, 19.1), three up to
 //   170 from K 3072 (400 x 768, K 5376: 39.6 us, unsplit 46.2, k_gemm_x3 44.1; at K 2048 20.7 against 19.7).
-enum { kT64x64, kT64x96, kT32x64, kT32x32 };
+enum { kT64x64, kT32x64, kT32x32 };
 struct X3Plan {
     int tile, splits, kchunk;
 };
 static X3Plan x3p_plan(const GemmArgs &g, int groups, bool reducible) {
     auto tiles = [&](int bm, int bn) { return int64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * groups; };
-    if (tiles(64, 64) >= 200) return {g.n == 96 ? kT64x96 : kT64x64, 1, 0};
+    if (tiles(64, 64) >= 200) return {kT64x64, 1, 0};
     const int64_t t = tiles(32, 64), t64 = tiles(64, 64);
     const bool split = reducible && groups == 1 && g.ws;
     X3Plan whole{t >= 100 ? kT32x64 : kT32x32, 1, 0}, p{kT32x64, 1, 0};
@@ -81,7 +81,6 @@ template <int EPI, int ASRC>
 static hipError_t x3p_tiles(int tile, const float *A, const GemmArgs &g, int z, hipStream_t s) {
     switch (tile) {
         case kT64x64: return x3p_tile<EPI, ASRC, 2, 4, 2, 1>(A, g, z, s);
-        case kT64x96: return x3p_tile<EPI, ASRC, 2, 2, 2, 3>(A, g, z, s);
         case kT32x64: return x3p_tile<EPI, ASRC, 2, 4, 1, 1>(A, g, z, s);
         default: return x3p_tile<EPI, ASRC, 2, 2, 1, 1>(A, g, z, s);
     }
