@@ -95,10 +95,10 @@ VH_DEV u32x4s dma_rsrc(const void *p) {
 // every DMA in flight before each LDS read it cannot tell apart from them; no register is loaded, and the waits are
 // wait_step's.
 VH_DEV void dma_b128(u32x4s r, uint32_t lds, int voff, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory", "m0");
 }
 VH_DEV void dma_b32(u32x4s r, uint32_t lds, int voff, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory", "m0");
 }
 // All but the newest N of this wave's DMAs have landed, and its LDS reads have returned.
 template <int N>
