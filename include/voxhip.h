@@ -490,7 +490,8 @@ int voxhip_bench_gemv_q8(int64_t rows, int64_t cols, int copies, int warmup, int
  * shape: y [m][n] = (A_hi + A_lo) [m][K] . W [n][K]^T, A_hi ~N(0, 1) and A_lo ~N(0, 1e-3) as f16 planes, W ~N(0,
  * 0.02) as f16 or (q8 != 0) in its q8 form (int8 values widened to f16, per-32 block scales). tile 0 takes the
  * library's shape policy; 1..4 force one of its block tiles (rows of A x rows of W: 32x32, 32x64, 64x64, 64x128 of
- * 8 waves); every tile gives the same bits (the same MFMA sequence per output). The inputs are those of
+ * 8 waves); every tile gives the same bits (the same MFMA sequence per output). -1: the policy with the library's split-K
+ * workspace, as the models' passes run it (a long K on a small grid in slices, summed by a second launch). The inputs are those of
  * voxhip_mat_synthetic(F16, m, K, 11, 0x90, 0, 1) (A_hi), (F16, m, K, 12, 0x91, 0, 1e-3) (A_lo) and (F16 or Q8, n, K,
  * 13, 0x92, 0, 0.02) (W). Average microseconds per launch; y_out (host, may be NULL) receives y of
  * the last launch. K must be a multiple of 64. No reference counterpart (benchmark helper). */

@@ -14,13 +14,17 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("m,n,K", [
     (1, 1, 64), (1, 130, 128), (15, 33, 64), (16, 64, 192), (17, 63, 128), (31, 4, 320), (32, 32, 64),
     (33, 65, 192), (63, 127, 64), (64, 128, 128), (65, 129, 192), (129, 257, 64),  # one past each tile, n off the fours
-    (33, 100, 2112), (70, 72, 4864),                                              # split K, a short last slice
+    (33, 100, 2112), (70, 72, 4864), (33, 101, 2112),                             # split K, a short last slice, n off the fours
     (640, 2052, 64), (1290, 1030, 64)])                                           # the grids of the wide tiles
 def test_gemm_hh_edges(hip, m, n, K, q8):
     a, w = _operands(hip, m, n, K, q8)
     want = a @ w.T
     bound = (K / 32 + 32) * 2.0 ** -24 * (np.abs(a) @ np.abs(w).T)
-    for tile in range(5):
+    for tile in range(-1, 5):  # -1: K split as in the models
         got = hip.bench_gemm_hh(m, n, K, q8=q8, tile=tile, warmup=0, iters=1, out=True)[1]
         worst = float(np.max(np.abs(got - want) / bound))
         assert worst <= 1.0, (m, n, K, q8, tile, worst)
+        if tile == -1:
+            sliced = got
+        elif tile == 0 and K >= 2112:  # the sums of slices round differently: K was split
+            assert not np.array_equal(got, sliced)

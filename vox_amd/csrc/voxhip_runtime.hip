@@ -4251,7 +4251,7 @@ int voxhip_bench_gemm_hh(int64_t m, int64_t n, int64_t K, int q8, int tile, int 
     return guard_int([&] {
         require_ok();
         if (vh::prof_on()) throw Fail("the benchmark entry points time launches, which VOX_PROFILE=gpu serialises");
-        if (m <= 0 || n <= 0 || K <= 0 || K % 64 || tile < 0 || tile > 4 || warmup < 0 || iters <= 0 || !us_per_launch)
+        if (m <= 0 || n <= 0 || K <= 0 || K % 64 || tile < -1 || tile > 4 || warmup < 0 || iters <= 0 || !us_per_launch)
             throw Fail("bad bench arguments");
         if (m > (int64_t(1) << 20) || n > (int64_t(1) << 20) || m * K > (int64_t(1) << 28) || n * K > (int64_t(1) << 28))
             throw Fail("bench_gemm_hh: shape too large");
@@ -4299,7 +4299,11 @@ int voxhip_bench_gemm_hh(int64_t m, int64_t n, int64_t K, int q8, int tile, int 
             ga.a16 = planes;
             ga.y = y;
             ga.ldy = int32_t(n);
-            vh::set_gemm_hh_tile(tile);
+            if (tile < 0) {
+                ga.ws = g.gemm_ws;
+                ga.ws_cap = kGemmWsFloats;
+            }
+            vh::set_gemm_hh_tile(std::max(tile, 0));
             for (int i = 0; i < warmup; ++i) HIPCHECK(launch_gemm_hh(EPI_STORE, pack, st, ga, g.stream));
             HIPCHECK(hipEventCreate(&e0));
             HIPCHECK(hipEventCreate(&e1));

@@ -858,7 +858,7 @@ def bench_gemv_q8(rows, cols, copies, warmup, iters):
 
 def bench_gemm_hh(m, n, K, q8=False, tile=0, warmup=3, iters=20, out=False):
     """Average microseconds of one split-f16 MFMA GEMM launch on an (m, n, K) product (tile 0: the library's policy,
-    1..4 a forced block tile: 32x32, 32x64, 64x64, 64x128); with out, also y [m][n] of the last launch."""
+    1..4 a forced block tile: 32x32, 32x64, 64x64, 64x128; -1: the policy with K split as in the models); with out, also y [m][n] of the last launch."""
     us = C.c_double()
     y = np.empty((m, n), np.float32) if out else None
     _check(lib().voxhip_bench_gemm_hh(m, n, K, int(bool(q8)), tile, warmup, iters, C.byref(us),
