@@ -4,12 +4,15 @@
 
 namespace vh {
 
+// The LDS is that of one block per 16 rows: launches without ws take it at any length. No length is too long: against the
+// separate launches the estimator's step gains 1.26x at 20 frames, 1.21x at 512, 1.17-1.20x up to 2048 and 1.04-1.11x from
+// there to 5000, where blocks come in several rounds.
 bool block_tail_ok(int64_t R, int C, int inner, int ff) {
     return C == kTailC && R > 0 && R <= INT32_MAX && inner > 0 && inner % 256 == 0 && ff > 0 && ff % 256 == 0 &&
            block_tail_smem(inner, ff) <= 160 * 1024;
 }
-// Blocks per 16 rows, each with a part of the FFN: as many as 256 CUs hold at once (a block's LDS fills one), where ff gives
-// each whole passes of 256. In the flow estimator's step 4 instead of 1: 1024 rows 18.2 -> 15.6 us a launch, 202 rows 18.8 ->
+// Blocks per 16 rows, each with a part of the FFN: as many as 256 CUs hold at once (one each: its 146 registers leave a SIMD
+// three waves, and a block is two a SIMD), where ff gives each whole passes of 256. In the flow estimator's step 4 instead of 1: 1024 rows 18.2 -> 15.6 us a launch, 202 rows 18.8 ->
 // 13.7 (the step 2737 -> 2547 and 2235 -> 1939 us). Every block repeats the out-projection and its norm.
 static int block_tail_parts(int64_t R, int ff) {
     const int64_t tiles = (R + 127) / 128 * 8;

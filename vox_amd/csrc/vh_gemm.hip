@@ -160,9 +160,6 @@ static hipError_t gemm_epi(int epi, const uint8_t *w, const float *scale, const 
         case EPI_GELU_ERF: return gemm_tile<WT, EPI_GELU_ERF>(w, scale, A, g, s);
         case EPI_ACC_SNAKE:
             return g.snake_a && g.snake_ib && g.snake_y ? gemm_tile<WT, EPI_ACC_SNAKE>(w, scale, A, g, s) : hipErrorInvalidValue;
-        case EPI_ROPE:
-            if (!g.rope || g.hd <= 0 || g.hd % 2 || g.seq <= 0 || g.rope_cols % (2 * g.hd)) return hipErrorInvalidValue;
-            return gemm_tile<WT, EPI_ROPE>(w, scale, A, g, s);
         case EPI_ROPE_H16:
             return rope_h16_ok(g) ? gemm_tile<WT, EPI_ROPE_H16>(w, scale, A, g, s) : hipErrorInvalidValue;
         default: return hipErrorInvalidValue;
@@ -174,7 +171,7 @@ hipError_t launch_gemm(int wt, int epi, const uint8_t *w, const float *scale, co
     g.status = status_word();
     if (g.m <= 0) return hipSuccess;
     if (g.K % 8 || g.n <= 0 || g.lda % 4) return hipErrorInvalidValue;
-    if ((epi == EPI_SWIGLU || epi == EPI_ROPE) && g.n % 2) return hipErrorInvalidValue;
+    if (epi == EPI_SWIGLU && g.n % 2) return hipErrorInvalidValue;
     if (wt == WT_F32 && g.wx && gemm_args_ok(epi, g)) {
         bool done = false;
         const hipError_t e = launch_gemm_x3p(ASRC_ROWS, epi, A, g, 1, s, &done);

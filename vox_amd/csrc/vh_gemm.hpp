@@ -138,7 +138,7 @@ VH_DEV void gemm_epilogue(const f32x4v (&acc)[TM][TN], const GemmArgs &g, int m0
                 if (EPI == EPI_SWIGLU) {
                     const float up = __shfl_xor(c, 1, kWave);  // column col ^ 1 of the same row
                     if (in && (col & 1) == 0) g.y[int64_t(row) * g.ldy + col / 2] = silu(c) * up;
-                } else if (EPI == EPI_ROPE || EPI == EPI_ROPE_H16) {
+                } else if (EPI == EPI_ROPE_H16) {
                     const float o = __shfl_xor(c, 1, kWave);  // the pair partner (2j <-> 2j + 1)
                     float r = c;
                     if (col < g.rope_cols && g.rope) {
@@ -150,9 +150,7 @@ VH_DEV void gemm_epilogue(const f32x4v (&acc)[TM][TN], const GemmArgs &g, int m0
                             r = (col & 1) ? c * cc + o * sn : c * cc - o * sn;
                         }
                     }
-                    if (EPI == EPI_ROPE) {
-                        if (in) *dst = r;
-                    } else if (in) {
+                    if (in) {
                         _Float16 hi, lo;
                         bad |= split_f16(r, hi, lo);
                         const int inner = g.rope_cols / 2, sec = col / inner, cq = col - sec * inner;
@@ -204,9 +202,8 @@ VH_DEV void gemm_store_partial(const f32x4v (&acc)[TM][TN], const GemmArgs &g, i
 
 // Epilogues: EPI_STORE y = c + bias; EPI_ACC y += c + bias; EPI_SWIGLU W rows are (gate u, up u) pairs, y[u] =
 // silu(gate) * up; EPI_GATED_ACC y += gate[col] * (c + bias); EPI_GELU y = gelu_tanh(c + bias); EPI_MISH
-// y = mish(c + bias); EPI_MISH_ACC y += mish(c + bias); EPI_GELU_ERF y = gelu_erf(c + bias); EPI_ROPE y = c + bias
-// with the pairs of q | k rotated;
-// EPI_ROPE_H16 writes its results as f16 halves (hi, lo) for the attention's split-f16 products.
+// y = mish(c + bias); EPI_MISH_ACC y += mish(c + bias); EPI_GELU_ERF y = gelu_erf(c + bias); EPI_ROPE_H16
+// c + bias with the pairs of q | k rotated, as f16 halves (hi, lo) for the attention's split-f16 products.
 // ASRC_CONV: W (F32) and y columns are those of group blockIdx.z.
 template <int WT, int EPI, int ASRC, int TM, int TN>
 __global__ __launch_bounds__(256) void k_gemm_f32(const uint8_t *__restrict__ w, const float *__restrict__ scale,

@@ -150,7 +150,7 @@ VH_DEV void epi_tile(f32x4v c, const GemmArgs &g, int row, int c0, bool vec, int
         if (rin && c0 < g.n) halves_store<EPI>(c, g, row, c0, bad);
         return;
     }
-    if constexpr (EPI == EPI_ROPE || EPI == EPI_ROPE_H16) {
+    if constexpr (EPI == EPI_ROPE_H16) {
         if (c0 < g.rope_cols && g.rope && rin) {
             const int n = row % g.seq, inner = g.rope_cols / 2, rhd = g.rope_hd ? g.rope_hd : g.hd;
 #pragma unroll
@@ -164,10 +164,8 @@ VH_DEV void epi_tile(f32x4v c, const GemmArgs &g, int row, int c0, bool vec, int
                 }
             }
         }
-        if constexpr (EPI == EPI_ROPE_H16) {
-            rope_h16_store(c, g, row, c0, lane, bad);
-            return;
-        }
+        rope_h16_store(c, g, row, c0, lane, bad);
+        return;
     }
     if (!rin) return;
     const int64_t idx = int64_t(row) * g.ldy + c0;
@@ -218,7 +216,7 @@ VH_DEV bool epi_vec(const GemmArgs &g) {
 template <int EPI, int TM, int TN>
 struct EpiOps {
     static constexpr bool kAcc = EPI == EPI_ACC || EPI == EPI_GATED_ACC || EPI == EPI_MISH_ACC || EPI == EPI_ACC_SNAKE;
-    static constexpr bool kRope = EPI == EPI_ROPE || EPI == EPI_ROPE_H16;
+    static constexpr bool kRope = EPI == EPI_ROPE_H16;
     static constexpr bool kP0 = EPI == EPI_GATED_ACC || EPI == EPI_SNAKE || EPI == EPI_ACC_SNAKE;
     static constexpr bool kP1 = EPI == EPI_SNAKE || EPI == EPI_ACC_SNAKE;
     f32x4v bias[TN], p0[kP0 ? TN : 1], p1[kP1 ? TN : 1], y[kAcc ? TM : 1][kAcc ? TN : 1], cs[kRope ? TM : 1][kRope ? TN : 1];

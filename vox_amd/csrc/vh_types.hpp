@@ -16,8 +16,8 @@ enum { EPI_STORE = 0, EPI_ACC = 1, EPI_SWIGLU = 2 };
 // GemvArgs::yq / yqs / yqsum for the next pass (which takes them as its PRO_Q rows) instead of stored as floats
 enum { EPI_SWIGLU_Q = 13 };
 // GEMM-only epilogues (F5 DiT, Vocos, the codec): y += gate * c; y = gelu_tanh(c); y = mish(c); y += mish(c); RoPE on
-// q|k columns; y = gelu_erf(c); y = snake(c); y += c, then snake(y) into snake_y as well
-enum { EPI_GATED_ACC = 3, EPI_GELU = 4, EPI_MISH = 5, EPI_MISH_ACC = 6, EPI_ROPE = 7, EPI_ROPE_H16 = 8, EPI_GELU_H16 = 9,
+// q|k columns into f16 halves; y = gelu_erf(c); y = snake(c); y += c, then snake(y) into snake_y as well
+enum { EPI_GATED_ACC = 3, EPI_GELU = 4, EPI_MISH = 5, EPI_MISH_ACC = 6, EPI_ROPE_H16 = 8, EPI_GELU_H16 = 9,
        EPI_GELU_ERF = 10, EPI_SNAKE = 11, EPI_SWIGLU_H16 = 12, EPI_ACC_SNAKE = 14 };
 // GEMM A operand: rows of a matrix, or the implicit im2col rows of a grouped "same" Conv1d
 enum { ASRC_ROWS = 0, ASRC_CONV = 1, ASRC_STREAM = 2 };
@@ -177,7 +177,7 @@ struct GemmArgs {
     int64_t lda, ldy;
     int32_t m, n, K;
     const float *gate;  // EPI_GATED_ACC: [n]
-    // EPI_ROPE: table [seq][hd/2][2] (cos, sin) at position row % seq; pairs (2j, 2j + 1) of the columns below
+    // EPI_ROPE_H16: table [seq][hd/2][2] (cos, sin) at position row % seq; pairs (2j, 2j + 1) of the columns below
     // rope_cols rotate (q | k heads), heads >= rope_heads of each of q and k are left as they are
     const float *rope;
     int32_t seq, hd, rope_cols, rope_heads;

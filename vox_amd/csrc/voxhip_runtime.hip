@@ -834,8 +834,8 @@ bool any_hd(const Xfmr &X) { return X.hd != 64 && X.hd != 128; }
 
 // Planes passes: a prefill pass of one sequence on the f32-activation GEMM whose four matrices are F16 or Q8 with K a
 // multiple of 64 runs its GEMMs on f16 halves of their inputs that the producers write (the RMSNorms, the attention,
-// the SwiGLU epilogue), so no GEMM block splits its A tile again, and Q8 weights as their int8 values widened to f16
-// once (planes_weights). The products and their order are those of the f32-activation GEMM.
+// the SwiGLU epilogue), so no GEMM block splits its A tile again, on weights laid out once (prepare_w16; Q8 as its int8
+// values). The products are those of the f32-activation GEMM, summed in another order.
 bool planes_mat(const GpuMat &m, int64_t m_total, int mc) {
     return (m.type == VOXHIP_F16 || m.type == VOXHIP_Q8) && m.cols % 64 == 0 && gemm_path(m, m_total, mc);
 }
@@ -3150,7 +3150,7 @@ int voxhip_cosy_step(int id, const float *x, const float *tb, float *out) {
         if (!x || !tb || !out) throw Fail("missing argument");
         h2d(E.x, x, size_t(E.T) * E.M * 4);
         h2d(E.tb, tb, (2 + E.mid_res.size()) * size_t(E.C) * 4);
-        // the step's ~560 launches as one graph: the buffers of this begin, the weights and the scratch are fixed
+        // the step's launches (about 300) as one graph: the buffers of this begin, the weights and the scratch are fixed
         vh::prof_stage("flow.est");
         if (vh::prof_on()) cosy_enqueue(E, g.stream);  // stamped launches are not captured
         else if (!E.step_graph) {
