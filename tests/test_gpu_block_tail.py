@@ -20,9 +20,7 @@ SMALL = (1, 7, 8, 9, 17)  # 2 T rows: a part of a block, one short of it, whole,
 
 
 @pytest.mark.parametrize("heads,ff,n_x,frames", [(8, 1024, 2, SMALL), (4, 256, 1, SMALL), (20, 512, 2, SMALL), (8, 2048, 1, SMALL),
-                                                 (3, 1024, 1, SMALL), (8, 320, 2, SMALL),
-                                                 (4, 1024, 1, (512, 513, 1024, 1025))])  # 64 tiles of 16 rows: 4 blocks each
-# (all 256 of ws), 72 and 128: 2 (all 128 counts), 136: 1
+                                                 (3, 1024, 1, SMALL), (8, 320, 2, SMALL)])
 def test_block_tail_widths(hip, oracle, heads, ff, n_x, frames):
     m = CosyModel(60 + heads, M=8, C=256, heads=heads, head_dim=64, n_mid=1, n_x=n_x, ff=ff, wtype=F16)
     est = m.create(hip)
@@ -36,6 +34,20 @@ def test_block_tail_widths(hip, oracle, heads, ff, n_x, frames):
             assert rel_err(got, want) < TOL, (heads, ff, T, rel_err(got, want))
             x = rng.standard_normal(x.shape).astype(np.float32)
         hip.cosy_end(est)
+
+
+@pytest.mark.parametrize("T", [512, 513, 1024, 1025])  # 64 tiles of 16 rows: 4 blocks each (all 256 of ws), 72 and 128: 2
+def test_block_tail_lengths(hip, oracle, T):           # (all 128 counts), 136: 1
+    m = CosyModel(64, M=8, C=256, heads=4, head_dim=64, n_mid=0, n_x=1, ff=1024, wtype=F16)
+    est = m.create(hip)
+    in0, x, tb = m.inputs(np.random.default_rng(T), T)
+    hip.cosy_begin(est, T, in0)
+    got = hip.cosy_step(est, x, tb, T, m.M)
+    want = oracle.cosy_step(m.ox, T, m.with_x(in0, x), tb)
+    assert rel_err(got, want) < TOL, (T, rel_err(got, want))
+    for _ in range(3):  # replays: the counts are zero again, the parts added in their order
+        assert np.array_equal(hip.cosy_step(est, x, tb, T, m.M), got)
+    hip.cosy_end(est)
 
 
 CHILD = r"""

@@ -9,6 +9,14 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-3  # keys and values of 16 bits
 
 
+def limit_to_use(hip, more):
+    """The VRAM limit at what is in use without any weight copy (an allocation past every limit takes theirs), and so much more."""
+    hip.lib().voxhip_set_vram_limit(int(hip.mem_info().used + 1))
+    with pytest.raises(hip.VoxHipError, match="VRAM limit"):
+        hip.DevBuf(1 << 40)
+    hip.lib().voxhip_set_vram_limit(int(hip.mem_info().used + more))
+
+
 def test_row_scratch_after_a_refused_growth(hip, oracle):
     mdl = Model(860, 2, 256, 4, 2, 64, 512, wtype=F16, head_rows=64)
     xf, head = hip.xfmr_create(mdl.hx, "t"), hip.upload(mdl.head[1])
@@ -16,7 +24,7 @@ def test_row_scratch_after_a_refused_growth(hip, oracle):
     rng = np.random.default_rng(1)
     x = rng.standard_normal((600, 256)).astype(np.float32)
     hip.forward(xf, seq, 0, x[:16], 256, head=head)
-    hip.lib().voxhip_set_vram_limit(int(hip.mem_info().used + (1 << 20)))
+    limit_to_use(hip, 1 << 20)
     try:
         with pytest.raises(hip.VoxHipError, match="VRAM limit"):
             hip.forward(xf, seq, 0, x, 256, head=head)  # 512 rows a pass: scratch of several MiB
@@ -43,7 +51,7 @@ def test_vocoder_after_a_refused_length(hip, oracle):
     h = m.create(hip)
     mel = np.random.default_rng(2).standard_normal((20000, m.mel)).astype(np.float32)
     hip.f5_vocos(h, mel[:40])
-    hip.lib().voxhip_set_vram_limit(int(hip.mem_info().used + (1 << 20)))
+    limit_to_use(hip, 1 << 20)
     try:
         with pytest.raises(hip.VoxHipError, match="VRAM limit"):
             hip.f5_vocos(h, mel)

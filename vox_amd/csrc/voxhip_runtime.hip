@@ -897,6 +897,7 @@ void prepare_mat(GpuMat &m, int64_t m_total, int mc, hipStream_t s) {
     if (gemm_path(m, m_total, mc)) prepare_x3(m, s);
 }
 void prepare_layers(Xfmr &X, int first, int count, int64_t m_total, int mc, bool fused, hipStream_t s) {
+    if (mc <= 4) return;  // no pass of so few rows takes the GEMM
     const bool pass_attn = pass_attn_of(X, mc, fused);
     for (int li = first; li < first + count; ++li) {
         const LayerDev &L = X.L[size_t(li)];
@@ -3150,7 +3151,7 @@ int voxhip_cosy_step(int id, const float *x, const float *tb, float *out) {
         if (!x || !tb || !out) throw Fail("missing argument");
         h2d(E.x, x, size_t(E.T) * E.M * 4);
         h2d(E.tb, tb, (2 + E.mid_res.size()) * size_t(E.C) * 4);
-        // the step's launches (about 300) as one graph: the buffers of this begin, the weights and the scratch are fixed
+        // the step's launches (about 260) as one graph: the buffers of this begin, the weights and the scratch are fixed
         vh::prof_stage("flow.est");
         if (vh::prof_on()) cosy_enqueue(E, g.stream);  // stamped launches are not captured
         else if (!E.step_graph) {
@@ -3698,7 +3699,7 @@ int voxhip_codec_forward(int codec, int state, const float *z, int F, float *pcm
         h2d(E.z, z, size_t(F) * size_t(E.cdim) * 4);
         h2d(E.rope, cs.data(), cs.size() * 4);
         h2d(St.pos_dev, &St.len, sizeof(int64_t));
-        // the call's ~150 launches as one graph per (F, parity): the buffers, the weights and the scratch are fixed,
+        // the call's launches (about 130) as one graph per (F, parity): the buffers, the weights and the scratch are fixed,
         // the position comes from pos_dev
         const int key = 2 * F + St.parity;
         vh::prof_stage("codec");
