@@ -15,7 +15,7 @@ namespace vh {
 // two barriers a step, about 1.2 us each whatever the block count. Here a K step of 64 takes 0.45 us with 120 blocks; large
 // grids are bound by the split's VALU work and the LDS and L1 reads together. Eight waves per 64 x 64 tile
 // (32 x 16 outputs each) halve each wave's share of the split. Measured, k_gemm_x3 against this kernel (us):
-// 2560 x 384, K 2688 (streaming conv) 95.6 -> 31.8; 10240 x 192, K 1344 62.4 -> 29.7; 30720 x 96, K 672 52.6 -> 24.6;
+// 2560 x 384, K 2688 (streaming conv) 95.6 -> 31.8; 10240 x 192, K 1344 62.4 -> 29.7; 30720 x 96, K 672 with Snake 55.9 -> 35.3;
 // 333 x 64 x 16 groups, K 1984 78.3 -> 16.9; 1024 x 256, K 768 14.9 -> 8.3; 160 x 384, K 384 14.1 -> 5.0.
 //
 // Block: WM x WN waves of 16 TM x 16 TN outputs; W is the MFMA's A operand, the activations its B (epi_tile's layout).
