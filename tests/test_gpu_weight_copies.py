@@ -163,3 +163,20 @@ def test_allocation_takes_the_room_of_copies_in_use(hip, oracle, limit):
     flow.end(hip, hf)
     for s in st:
         hip.codec_state_free(s)
+
+
+def test_allocation_past_every_copy_leaves_them(hip, oracle, limit):
+    dit = Dit()
+    h = dit.create(hip)
+    dit.begin(hip, h, oracle)
+    first = dit.step(hip, h)
+    limit(0)
+    used = hip.mem_info().used
+    with pytest.raises(hip.VoxHipError, match="VRAM limit"):
+        hip.DevBuf(1 << 40)
+    hip.lib().voxhip_set_vram_limit(0)
+    with pytest.raises(hip.VoxHipError, match="hipMalloc"):
+        hip.DevBuf(1 << 42)
+    assert hip.mem_info().used == used
+    assert np.array_equal(dit.step(hip, h), first)
+    dit.end(hip, h)

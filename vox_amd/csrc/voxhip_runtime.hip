@@ -233,8 +233,8 @@ int32_t *status_word() { return g.status_dev; }
 namespace {
 
 // ------------------------------------------------------------------ device memory with accounting
-// Gives back every weight copy (below, with the objects that read them): whether there was one.
-bool release_copies();
+// Gives back every weight copy (below, with the objects that read them) where that makes room for `bytes`: whether it did.
+bool release_copies(size_t bytes);
 
 // required: what a call cannot do without; the weight copies make room for it.
 void *dalloc(size_t bytes, bool required = true) {
@@ -255,7 +255,7 @@ void *dalloc(size_t bytes, bool required = true) {
             (void)hipGetLastError();  // the failure is reported here, not by the next launch
             why = std::string("hipMalloc of ") + std::to_string(bytes >> 20) + " MiB failed: " + hipGetErrorString(e);
         }
-        if (!required || !release_copies()) throw Fail(why);
+        if (!required || !release_copies(bytes)) throw Fail(why);
     }
 }
 void dfree(void *p) {
@@ -3405,19 +3405,38 @@ void lay_out(const Codec &E) {
     for (int id : ids) prepare_x3(mat_at(id), g.stream);
 }
 
+template <class Fn>
+void each_copy(Fn fn) {
+    for (F5 *F : g.f5)
+        if (F) each_conv(*F, [&](F5Conv &c) { fn(c.wx); });
+    for (Cosy *E : g.cosy) {
+        if (!E) continue;
+        each_conv(*E, [&](F5Conv &c) { fn(c.wx); });
+        fn(E->tail_ws);
+        fn(E->tail_count);
+    }
+    for (GpuMat &m : g.mats) {
+        fn(m.w16);
+        fn(m.st);
+        fn(m.wx);
+    }
+}
 // After the work in flight, every copy and every graph that may read one; models go on with the weights as stored. The copies
 // are read by g.stream's work and this library's graphs only (the no-alloc call, whose launches a caller may capture, never
-// reads one), and no caller of dalloc holds one across the call. Not during a capture.
-bool release_copies() {
+// reads one), and no caller of dalloc holds one across the call. Not during a capture, and not for an allocation that would
+// find no room even so.
+bool release_copies(size_t bytes) {
+    uint64_t held = 0;
+    each_copy([&](auto *p) {
+        const auto it = g.allocs.find(p);
+        if (it != g.allocs.end()) held += it->second;
+    });
+    if (!held || (g.vram_limit && g.vram_used - held + bytes > g.vram_limit)) return false;
+    size_t avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) != hipSuccess || avail + held < bytes) return false;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (!g.ok || hipStreamIsCapturing(g.stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
+    if (hipStreamIsCapturing(g.stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
     if (hipStreamSynchronize(g.stream) != hipSuccess) return false;
-    bool any = false;
-    auto drop = [&](auto *&p) {
-        any = any || p;
-        dfree(p);
-        p = nullptr;
-    };
     for (Xfmr *X : g.xf)
         if (X) drop_graphs(*X);
     for (CodecSt *S : g.cstates) {
@@ -3425,26 +3444,19 @@ bool release_copies() {
         for (auto &kv : S->graphs) (void)hipGraphExecDestroy(kv.second);
         S->graphs.clear();
     }
-    for (F5 *F : g.f5) {
-        if (!F) continue;
-        F->split = false;
-        each_conv(*F, [&](F5Conv &c) { drop(c.wx); });
-    }
+    for (F5 *F : g.f5)
+        if (F) F->split = false;
     for (Cosy *E : g.cosy) {
         if (!E) continue;
         drop_step_graph(*E);
         E->split = false;
-        each_conv(*E, [&](F5Conv &c) { drop(c.wx); });
-        drop(E->tail_ws);
-        drop(E->tail_count);
     }
-    for (GpuMat &m : g.mats) {
-        drop(m.w16);
-        drop(m.st);
-        drop(m.wx);
-    }
+    each_copy([&](auto *&p) {
+        dfree(p);
+        p = nullptr;
+    });
     g.copies_off = true;
-    return any;
+    return true;
 }
 }  // namespace
 
